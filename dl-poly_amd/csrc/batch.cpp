@@ -135,7 +135,7 @@ static int ens_prepare(Ensemble &E, bool energies, const Shape &sh)
     // records the buffer's address (upper bounds: the z pass has at most
     // K1 K2 workgroups, the pair kernel at most natms * 16 / 512)
     for (Ctx *c : cs) {
-        const int ub = std::max({ceil_div((long)c->natms * 16, 512), step_blocks(c), excl_blocks(c),
+        const int ub = std::max({ceil_div((long)c->natms * 16, 512), excl_blocks(c),
                                  c->prm.electrostatics ? c->K[0] * c->K[1] : 1,
                                  c->prm.electrostatics ? ceil_div(c->natms, 16) : 1});
         if ((r = ensure_red_rows(c, ub))) return r;
@@ -151,7 +151,6 @@ static int ens_prepare(Ensemble &E, bool energies, const Shape &sh)
         Ctx *c = cs[k];
         for (int q = 0; q < kReduceSlots; q++) rows[k].rows[q] = 0;
         for (int q = R_ENGVDW; q <= R_S33; q++) rows[k].rows[q] = npair[k];
-        rows[k].rows[R_KIN] = step_blocks(c);
         const int nex = (c->excl_total > 0 && c->prm.electrostatics) ? excl_blocks(c) : 0;
         for (int q = R_ENGEX; q <= R_XS33; q++) rows[k].rows[q] = nex;
         if (c->prm.electrostatics) {
@@ -361,9 +360,8 @@ int ensemble_run(const std::vector<Ctx *> &cs, Ensemble *&E, int nsteps, bool en
         DLPX_HIP(c, hipMemsetAsync(c->flags + F_OVF_ANY, 0, sizeof(int32_t), c0->stream));
         DLPX_HIP(c, hipMemsetAsync(c->flags + F_NREB, 0, sizeof(int32_t) * 2, c0->stream));
         DLPX_HIP(c, hipMemsetAsync(c->flags + F_DMAX, 0, sizeof(int32_t) * 3, c0->stream));
-        // the totals that the gather and the step kernel accumulate atomically
+        // the totals that the gather accumulates atomically
         DLPX_HIP(c, hipMemsetAsync(c->acc, 0, sizeof(double) * 4 * kAccSlots, c0->stream));
-        DLPX_HIP(c, hipMemsetAsync(c->red_out + R_KIN, 0, sizeof(double), c0->stream));
     }
     for (Ctx *c : cs)
         if (c != c0) DLPX_HIP(c, hipStreamSynchronize(c->stream));  // the snapshots

@@ -26,6 +26,8 @@ constexpr int kPPStride = 16;
 // workgroup b adds into slot b % kAccSlots, so no address takes more than a
 // few dozen atomics
 constexpr int kAccSlots = 64;
+// most workgroups of the step kernel per system (nve.hip)
+constexpr int kStepBlocks = 512;
 
 // Workgroups of a launch are dispatched round-robin over the 8 XCDs of an
 // MI355X (workgroup b on XCD b % 8), each with its own L2.  Kernels whose
@@ -266,6 +268,7 @@ struct Ctx {
     int red_rows[kReduceSlots]{};    // rows written per column by the last evaluation
     double *red_out = nullptr;       // kReduceSlots totals (device)
     double *acc = nullptr;           // kAccSlots x 4 atomic totals of the gather (batched runs), zero between steps
+    double *step_part = nullptr;     // kStepBlocks x 2 workgroup partials of the step kernel
     double *h_red = nullptr;         // pinned mirror of red_out
     double *energies_dev = nullptr;  // per-step energies (resident runs)
     int energies_cap = 0;
@@ -477,7 +480,6 @@ int vv2_blocks(const Ctx *c);
 int excl_blocks(const Ctx *c);
 // one kernel per step of a batched run: stage 2 of the step, its reductions
 // and per-step record, stage 1 of the next step (nve.hip)
-int step_blocks(const Ctx *c);
 int step_prepare(const std::vector<Ctx *> &cs, const std::vector<RedRowsHost> &rows, bool energies,
                  BatchLaunch &bl);
 int step_launch(Ctx *c, hipStream_t s, const BatchLaunch &bl, bool stage2, bool stage1);

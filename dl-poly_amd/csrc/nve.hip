@@ -1,5 +1,6 @@
 // Velocity-Verlet NVE integration on the device (nve.F90:127-215) and the
 // host-order <-> cell-order transfers of per-atom data.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -262,15 +263,23 @@ int nve_second(Ctx *c, double dt, bool /*kinetic*/)
 // One launch per step of a resident batched run (every system of the batch):
 // S2, stage 2 of the step just evaluated: the reciprocal finish (frc +=
 // 2 scale (frc_recip - mean), the mean from the gather's atomic totals in
-// acc), frozen atoms, the second half-kick and m v^2; the step's partial
-// sums reduced into red_out (workgroup b takes columns b, b + nb, ...; the
-// kinetic energy is added atomically, the reciprocal energy and net force
-// come from the gather's slots), and the step's record when records are
-// kept; and
+// acc), frozen atoms, the second half-kick and m v^2; when records are kept,
+// the step's partial sums reduced into its record (one wavefront per column);
+// and
 // S1, stage 1 of the next step: half-kick, drift, and the displacement test,
 // whose largest value the last workgroup to finish turns into the rebuild
-// decision (as k_vv1).  Workgroups exchange data only through device-scope
-// atomics; the last one also clears the atomic totals for the next step.
+// decision (as k_vv1).  With both stages the total force is not stored: the
+// next pair kernel overwrites it, and a run's last step has no stage 1.
+//
+// Bound by HBM at many atoms (224 B each), by latency at few.  Atomics on one
+// word complete about every 25 ns whatever the load, so a workgroup issues
+// exactly one (the count of finished workgroups): its kinetic-energy and
+// displacement partials go to its own slot of part[], and a launch has at
+// most kStepBlocks workgroups per system, each striding over the atoms with
+// the next atom's loads in flight.  Against three atomics from each of
+// ceil(n / 256) workgroups, the column sums ahead of the atoms and the force
+// stored every step: 1,728,000 ions 596 -> 150 us (2.6 TB/s), 64,000 ions
+// 14.2 -> 12.4 us, 4,000 atoms 8.5 -> 6.0 us.
 struct StepArgs {
     double4 *pos, *vel, *frc;
     const double4 *frc_recip;  // null: no reciprocal part
@@ -279,7 +288,8 @@ struct StepArgs {
     int n;
     double dt, two_scale, inv_n, half_pad;
     Box b;
-    double *red, *red_out;
+    const double *red;
+    double *part;              // kStepBlocks x {m v^2, largest displacement squared}
     double *acc;               // the gather's kAccSlots x 4 totals (null: no reciprocal part)
     int rows[kReduceSlots];    // partial rows per column of the step
     double *energies;          // per-step records (kReduceSlots each) or null
@@ -287,73 +297,95 @@ struct StepArgs {
     int32_t *flags;
 };
 __device__ __forceinline__ bool atomic_column(int col) { return col == R_KIN || (col >= R_ERECIP && col <= R_FNETZ); }
-// 256 threads: one atom per thread in workgroups small enough to spread a
-// 64k-atom system over every CU (the partial-sum columns go to the first
-// workgroups, one column each)
+// 256 threads: workgroups small enough to spread a 64k-atom system over
+// every CU
 constexpr int kStepThreads = 256;
+// workgroups beside the atoms' that sum the record's columns, one column per
+// wavefront (23 columns of partial rows)
+constexpr int kStepColumnBlocks = 6;
 template <bool S2, bool S1>
 __device__ __forceinline__ void step_body(const StepArgs &a, int bid, int nb)
 {
-    __shared__ double lsum[kStepThreads];
-    __shared__ double wmax[kStepThreads / 64];
-    __shared__ double lred[kStepThreads / 64];
-    __shared__ double recip[4];  // reciprocal energy and net force (unscaled)
+    constexpr int NW = kStepThreads / 64;
+    __shared__ double wke[NW], wr2[NW];
     __shared__ bool last;
-    const int t = threadIdx.x;
-    if (S2) {
-        // the gather's slot totals, summed in a fixed order by the first wavefront
-        double v[4] = {0.0, 0.0, 0.0, 0.0};
-        if (a.acc && t < kAccSlots)
-            for (int k = 0; k < 4; k++) v[k] = a.acc[4 * t + k];
-        if (t < 64)
-            for (int k = 0; k < 4; k++) v[k] = wave_sum(v[k]);
-        if (t == 0)
-            for (int k = 0; k < 4; k++) recip[k] = v[k];
-        __syncthreads();
+    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    static_assert(kAccSlots == 64, "a wavefront reads one accumulator slot per lane");
+    // this thread's first atom is loaded before anything waits; each later one
+    // while its predecessor is computed
+    struct Atom {
+        double4 v, f, r, p, q;
+    } cur, nxt;
+    auto load = [&](int i, Atom &m) {
+        m.v = a.vel[i];
+        m.f = a.frc[i];
+        if (S2 && a.frc_recip) m.r = a.frc_recip[i];
+        if (S1) {
+            m.p = a.pos[i];
+            m.q = a.xref[i];
+        }
+    };
+    const int ncb = S2 && a.energies ? kStepColumnBlocks : 0;  // the last workgroups take the columns
+    const int stride = (nb - ncb) * kStepThreads;
+    int i = bid < nb - ncb ? bid * kStepThreads + t : a.n;
+    if (i < a.n) load(i, cur);
+    // reciprocal energy and net force (unscaled): the gather's slot totals,
+    // summed in a fixed order by every wavefront
+    double recip[4] = {0.0, 0.0, 0.0, 0.0};
+    if (S2 && a.acc) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) recip[k] = a.acc[4 * lane + k];
+#pragma unroll
+        for (int k = 0; k < 4; k++) recip[k] = wave_sum(recip[k]);
     }
     // the step's record index (the last workgroup advances it after every
     // workgroup has read it)
     const int rec = (S2 && a.energies) ? a.flags[F_STEP] : a.ecap;
     double *record = rec < a.ecap ? a.energies + (size_t)rec * kReduceSlots : nullptr;
-    if (S2) {
-        // the columns the step's kernels filled with partial rows
-        for (int col = bid; col < kReduceSlots; col += nb) {
+    if (S2 && record && bid >= nb - ncb) {
+        // the columns the step's kernels filled with partial rows, in a fixed
+        // order, eight rows of a lane in flight
+        for (int col = (bid - (nb - ncb)) * NW + wid; col < kReduceSlots; col += kStepColumnBlocks * NW) {
             if (atomic_column(col)) continue;
-            const double v = column_sum<kStepThreads>(a.red, a.rows[col], kReduceSlots, col, lsum);
-            if (t == 0) {
-                a.red_out[col] = v;
-                if (record) record[col] = v;
-            }
+            const int rows = a.rows[col];
+            constexpr int U = 8;
+            double s[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) s[u] = 0.0;
+            for (int r = lane; r < rows; r += 64 * U)
+#pragma unroll
+                for (int u = 0; u < U; u++)
+                    if (r + 64 * u < rows) s[u] += a.red[(size_t)(r + 64 * u) * kReduceSlots + col];
+            const double v = wave_sum(((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7])));
+            if (lane == 0) record[col] = v;
         }
     }
-    const int i = bid * blockDim.x + t;
     double ke = 0.0, r2 = 0.0;
-    if (i < a.n) {
-        double4 v = a.vel[i];
-        double4 f = a.frc[i];
+    const double mx = recip[1] * a.inv_n, my = recip[2] * a.inv_n, mz = recip[3] * a.inv_n;
+    for (; i < a.n; i += stride) {
+        if (i + stride < a.n) load(i + stride, nxt);
+        double4 v = cur.v, f = cur.f;
         if (S2) {
             if (a.frc_recip) {
-                const double mx = recip[1] * a.inv_n, my = recip[2] * a.inv_n, mz = recip[3] * a.inv_n;
-                const double4 r = a.frc_recip[i];
-                f.x += (r.x - mx) * a.two_scale;
-                f.y += (r.y - my) * a.two_scale;
-                f.z += (r.z - mz) * a.two_scale;
+                f.x += (cur.r.x - mx) * a.two_scale;
+                f.y += (cur.r.y - my) * a.two_scale;
+                f.z += (cur.r.z - mz) * a.two_scale;
             }
             if (a.frz && a.frz[a.gid[i]] != 0) {
                 f.x = f.y = f.z = 0.0;
                 v.x = v.y = v.z = 0.0;
             }
-            a.frc[i] = f;
+            if (!S1) a.frc[i] = f;
             if (v.w > 1.0e-6) {
                 const double tmp = (0.5 * a.dt) / v.w;
                 v.x += tmp * f.x;
                 v.y += tmp * f.y;
                 v.z += tmp * f.z;
-                ke = v.w * (v.x * v.x + v.y * v.y + v.z * v.z);
+                ke += v.w * (v.x * v.x + v.y * v.y + v.z * v.z);
             }
         }
         if (S1) {
-            double4 p = a.pos[i];
+            double4 p = cur.p;
             if (v.w > 1.0e-6) {
                 const double tmp = (0.5 * a.dt) / v.w;
                 v.x += tmp * f.x;
@@ -364,58 +396,62 @@ __device__ __forceinline__ void step_body(const StepArgs &a, int bid, int nb)
                 p.z += a.dt * v.z;
                 a.pos[i] = p;
             }
-            const double4 q = a.xref[i];
-            const double dx = min_image_1(p.x, q.x, a.b.L[0], a.b.invL[0]);
-            const double dy = min_image_1(p.y, q.y, a.b.L[1], a.b.invL[1]);
-            const double dz = min_image_1(p.z, q.z, a.b.L[2], a.b.invL[2]);
-            r2 = dx * dx + dy * dy + dz * dz;
+            const double dx = min_image_1(p.x, cur.q.x, a.b.L[0], a.b.invL[0]);
+            const double dy = min_image_1(p.y, cur.q.y, a.b.L[1], a.b.invL[1]);
+            const double dz = min_image_1(p.z, cur.q.z, a.b.L[2], a.b.invL[2]);
+            r2 = fmax(r2, dx * dx + dy * dy + dz * dz);
         }
         a.vel[i] = v;
+        cur = nxt;
     }
-    if (S2) {
-        double acc[1] = {ke};
-        const double tot = block_sum<1>(acc, lred, a.red + (size_t)bid * kReduceSlots + R_KIN);
-        if (t == 0) atomicAdd(&a.red_out[R_KIN], tot);
-    }
-    if (S1) {
+    auto wave_max = [](double x) {
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o, 64));
-        if ((t & 63) == 0) wmax[t >> 6] = r2;
+        for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
+        return x;
+    };
+    if (S2) ke = wave_sum(ke);
+    if (S1) r2 = wave_max(r2);
+    if (lane == 0) {
+        wke[wid] = ke;
+        wr2[wid] = r2;
     }
     __syncthreads();
     if (t == 0) {
-        if (S1) {
-            double m = 0.0;
-            for (int w = 0; w < (int)(blockDim.x >> 6); w++) m = fmax(m, wmax[w]);
-            atomicMax((unsigned long long *)(a.flags + F_DMAX), (unsigned long long)__double_as_longlong(m));
+        double k = 0.0, m = 0.0;
+        for (int w = 0; w < NW; w++) {
+            k += wke[w];
+            m = fmax(m, wr2[w]);
         }
+        __hip_atomic_store(&a.part[2 * bid], k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&a.part[2 * bid + 1], m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         wait_memory();
         last = atomicAdd((unsigned int *)(a.flags + F_DONE), 1u) == (unsigned)nb - 1;
     }
     __syncthreads();
     if (!last) return;
-    if (S2) {
-        // the gather's slots cleared for the next step (every workgroup has
-        // read them)
-        if (a.acc && t < 4 * kAccSlots)
-            __hip_atomic_store(&a.acc[t], 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // the last workgroup: every other one has read acc and F_STEP and its
+    // partials are in part[]
+    if (S2 && a.acc && t < 4 * kAccSlots)  // the gather's slots cleared for the next step
+        __hip_atomic_store(&a.acc[t], 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (wid != 0) return;
+    ke = r2 = 0.0;
+    for (int b = lane; b < nb; b += 64) {
+        if (S2 && record) ke += load_coherent(&a.part[2 * b]);
+        if (S1) r2 = fmax(r2, load_coherent(&a.part[2 * b + 1]));
     }
-    if (t != 0) return;
-    if (S2) {
-        // the atomic totals into red_out and the record; the kinetic one is
-        // cleared for the next step
-        const double kin = load_coherent(&a.red_out[R_KIN]);
-        __hip_atomic_store(&a.red_out[R_KIN], 0.0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        for (int k = 0; k < 4; k++) a.red_out[R_ERECIP + k] = recip[k];
+    if (S2 && record) ke = wave_sum(ke);
+    if (S1) r2 = wave_max(r2);
+    if (lane != 0) return;
+    if (S2 && a.energies) {
         if (record) {
-            record[R_KIN] = kin;
+            record[R_KIN] = ke;
+#pragma unroll
             for (int k = 0; k < 4; k++) record[R_ERECIP + k] = recip[k];
         }
-        if (a.energies) a.flags[F_STEP] = rec + 1;
+        a.flags[F_STEP] = rec + 1;
     }
     if (S1) {
-        const unsigned long long bits = load_coherent((unsigned long long *)(a.flags + F_DMAX));
-        const int upd = (a.half_pad <= 0.0 || sqrt(__longlong_as_double((long long)bits)) >= a.half_pad) ? 1 : 0;
+        const int upd = (a.half_pad <= 0.0 || sqrt(r2) >= a.half_pad) ? 1 : 0;
         a.flags[F_UPD] = upd;
         if (upd) {
             a.flags[F_OVF] = 0;
@@ -423,8 +459,6 @@ __device__ __forceinline__ void step_body(const StepArgs &a, int bid, int nb)
             a.flags[F_PAIRS] = 0;
             a.flags[F_NREB] += 1;
         }
-        __hip_atomic_store((unsigned long long *)(a.flags + F_DMAX), 0ull, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
     }
     __hip_atomic_store((unsigned int *)(a.flags + F_DONE), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -438,7 +472,11 @@ __global__ void __launch_bounds__(kStepThreads) k_step_batch(const StepArgs *__r
     step_body<S2, S1>(av[s], lb - boff[s], boff[s + 1] - boff[s]);
 }
 
-int step_blocks(const Ctx *c) { return ceil_div(c->natms, kStepThreads); }
+static int step_blocks(const Ctx *c, bool energies)
+{
+    const int cols = energies ? kStepColumnBlocks : 0;
+    return std::min(ceil_div(c->natms, kStepThreads), kStepBlocks - cols) + cols;
+}
 
 int step_prepare(const std::vector<Ctx *> &cs, const std::vector<RedRowsHost> &rows, bool energies,
                  BatchLaunch &bl)
@@ -465,14 +503,14 @@ int step_prepare(const std::vector<Ctx *> &cs, const std::vector<RedRowsHost> &r
             a.b.invL[d] = c->invL[d];
         }
         a.red = c->red;
-        a.red_out = c->red_out;
+        a.part = c->step_part;
         a.acc = c->prm.electrostatics ? c->acc : nullptr;
         for (int q = 0; q < kReduceSlots; q++) a.rows[q] = rows[k].rows[q];
         a.energies = energies ? c->energies_dev : nullptr;
         a.ecap = c->energies_cap;
         a.flags = c->flags;
         av.push_back(a);
-        nb.push_back(step_blocks(c));
+        nb.push_back(step_blocks(c, energies));
     }
     return batch_upload(cs[0], bl, av.data(), sizeof(StepArgs), nb, false);
 }
