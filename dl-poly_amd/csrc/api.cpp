@@ -391,7 +391,8 @@ std::vector<uint64_t> step_graph_key(const Ctx *c, double tstep)
             (uint64_t)c->d_keytab, (uint64_t)c->d_vdw_direct, (uint64_t)c->cap_lane, (uint64_t)c->ncell,  (uint64_t)c->natms,
             (uint64_t)c->nc[0],    (uint64_t)c->nc[1],   (uint64_t)c->nc[2],   (uint64_t)c->gid,
             (uint64_t)c->slot,     (uint64_t)c->excl_off, (uint64_t)c->excl_ids, (uint64_t)c->excl_total,
-            (uint64_t)c->frz,      (uint64_t)c->nfrozen, t, (uint64_t)c->theta,
+            (uint64_t)c->frz,      (uint64_t)c->nfrozen, t, (uint64_t)c->theta, (uint64_t)c->key_start,
+            (uint64_t)c->list_coded, (uint64_t)c->tile_list, (uint64_t)c->tile_cap, (uint64_t)c->tile_lists, bits(c->list_L[0]), bits(c->list_L[1]), bits(c->list_L[2]),
             // the cell: pair, spreading and influence arguments carry it
             bits(c->cell[0]), bits(c->cell[4]), bits(c->cell[8])};
 }
@@ -536,6 +537,8 @@ int dlpx_create(const dlpx_params *p, dlpx_ctx **out)
     // DLPX_REL_PAIRS=0: the mixed pair kernel forms separations from FP64 positions
     // DLPX_FFT_PLANES=0: separate x and y line kernels where the plane kernels would run
     if (const char *e = std::getenv("DLPX_FFT_PLANES")) c->fft_planes = std::atoi(e) != 0;
+    // DLPX_SPREAD_TILES: charges spread by mesh tiles never (0) or wherever the mesh allows (1), not by the rule
+    if (const char *e = std::getenv("DLPX_SPREAD_TILES")) c->spread_tiles = std::atoi(e) != 0 ? 1 : 0;
     if (const char *e = std::getenv("DLPX_REL_PAIRS")) c->rel_pairs = std::atoi(e) != 0;
     if (const char *e = std::getenv("DLPX_COMB_THREADS")) c->comb_threads = std::atoi(e) == 512 ? 512 : 1024;
     if (const char *e = std::getenv("DLPX_GRAPH_STEPS")) c->graph_steps = std::max(1, std::min(64, std::atoi(e)));
@@ -588,7 +591,7 @@ int dlpx_destroy(dlpx_ctx *ctx)
                    c->gid, c->gid_alt, c->slot, c->stage, c->stage_i, c->cell_of, c->perm, c->cell_count,
                    c->cell_start, c->cell_fill, c->key_start, c->nbr, c->cnt, c->flags, c->d_vdw, c->d_erfc, c->d_keytab,
                    c->d_vdw_direct, c->d_comb, c->d_comb_row, c->sub_of, c->prel, c->excl_off, c->excl_ids, c->frz, c->pp, c->Q2,
-                   c->Q, c->Phi, c->H, c->theta, c->tw, c->bsp_n2, c->red, c->red_out, c->acc, c->step_part, c->energies_dev,
+                   c->Q, c->spl_z, c->spl_wq, c->spl_base, c->tile_list, c->Phi, c->H, c->theta, c->tw, c->bsp_n2, c->red, c->red_out, c->acc, c->step_part, c->energies_dev,
                    c->snap_d, c->snap_i};
     for (void *p : dev)
         if (p) (void)hipFree(p);

@@ -77,7 +77,7 @@ struct Ensemble {
     ~Ensemble() { release(); }
     void release()
     {
-        for (BatchLaunch *b : {&step, &excl, &spme.spread, &spme.gather}) batch_free(*b);
+        for (BatchLaunch *b : {&step, &excl, &spme.splines, &spme.spread, &spme.tiles, &spme.gather}) batch_free(*b);
         for (auto &g : spme.fft.groups) batch_free(g.bl);
         spme.fft.groups.clear();
         for (auto &g : pair.groups) batch_free(g.bl);

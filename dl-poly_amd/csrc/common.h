@@ -78,6 +78,30 @@ __device__ __forceinline__ bool batch_pos(const int32_t *__restrict__ boff, int 
     return true;
 }
 
+// Binning of the atoms at a list build: nc link cells per axis, sub = 1 by
+// link cell, 2 by subcell (half the link-cell edge).
+struct CellGrid {
+    int nc[3];
+    double L[3], invL[3];
+    int sub;
+};
+
+// Binning key of a subcell (sx, sy, sz) of edge L/(2 nc): link-cell-major,
+// then the 2 x 2 x 2 subcells of that link cell, so a link cell's atoms are
+// one contiguous run of the sorted order.
+__host__ __device__ __forceinline__ int subcell_key(const CellGrid &g, int sx, int sy, int sz)
+{
+    const int blk = ((sz >> 1) * g.nc[1] + (sy >> 1)) * g.nc[0] + (sx >> 1);
+    return blk * 8 + ((sz & 1) * 4 + (sy & 1) * 2 + (sx & 1));
+}
+
+// The bin of a coordinate folded into [-L/2, L/2), nc bins to the axis.
+__host__ __device__ __forceinline__ int cell_coord(double x, double L, double invL, int nc)
+{
+    int k = (int)((x * invL + 0.5) * (double)nc);
+    return k < 0 ? 0 : (k >= nc ? nc - 1 : k);
+}
+
 // Words of Ctx::flags (int32, device).
 enum Flag : int {
     F_OVF = 0,      // largest per-lane count of an overflowing list build (0: none)
@@ -90,6 +114,8 @@ enum Flag : int {
     F_NREB = 8,     // rebuilds decided on the device since the run began
     F_STEP = 9,     // per-step energy records written since the run began
     F_ERR = 10,     // sticky: a list-build kernel met an index outside the atoms (internal error)
+    F_STRAY = 11,   // the last position upload (its number) with an atom further than half the padding
+                    // from its bin of the last list build
     F_WDONE = 12,   // workgroups of the list binning finished (zero between launches)
     F_WORDS = 16
 };
@@ -151,6 +177,7 @@ struct Ctx {
     bool fft_lines = true;           // compile-time-length line kernels for the FFT lengths that have them
     bool rel_pairs = true;           // mixed combined-table pairs from subcell-relative FP32 positions
     int comb_threads = 1024;         // workgroup size of the combined-table pair kernel (512 or 1024)
+    int spread_tiles = -1;           // charge spreading by mesh tiles: 0 never, 1 where the mesh allows, -1 where faster
     bool fft_planes = true;          // x and y passes fused per z-plane where the mesh allows
     int graph_steps = 8;             // resident steps per replayed graph (1..64)
     int overlap = -1;                // resident steps' branch layout 0..2 (batch.cpp, ens_enqueue); -1 by batch size
@@ -217,6 +244,9 @@ struct Ctx {
 
     // Verlet list: lane-interleaved chunks; element (c, i, g) at (c*cap + i)*G + g
     int cap_lane = 0;
+    double list_L[3]{};              // cell edges at the last host-driven list build
+    int32_t upload_no = 0;           // position uploads onto an existing list (F_STRAY)
+    int32_t stray_no = 0;            // the upload the positions came from; 0: they are the list's own
     bool list_coded = false;         // entries carry subcell offsets (the subcell build)
     int32_t *sub_of = nullptr;       // per sorted atom: its subcell at the build, sx | sy << 10 | sz << 20
     float4 *prel = nullptr;          // per sorted atom: position relative to that subcell (FP32), type bits
@@ -248,8 +278,15 @@ struct Ctx {
     int K[3]{0, 0, 0};
     int K1h = 0, K1hp = 0;           // K1/2+1 and the padded row stride of H
     size_t nreal = 0, nhalf = 0;
-    void *Q = nullptr;               // real charge grid K3 x K2 x K1; all zero between evaluations (the
-                                     // forward x pass clears each line it has read)
+    void *Q = nullptr;               // real charge grid K3 x K2 x K1; unless it is spread by tiles, all zero
+                                     // between evaluations (the forward x pass clears each line it has read)
+    void *spl_z = nullptr, *spl_wq = nullptr;  // the atoms' splines of one evaluation (spme.hip, k_splines)
+    ushort4 *spl_base = nullptr;
+    int32_t *tile_list = nullptr;    // atoms of each mesh tile, tile_cap each, then their numbers (spme.hip)
+    size_t tile_words = 0;
+    int tile_cap = 0;                // 0: the charges are spread by link cells
+    int list_evals = 0;              // reciprocal sums since the last host-driven list build
+    bool tile_lists = false;         // the tiles' lists are those of the present Verlet list
     void *Phi = nullptr;             // real potential grid (the convolution's output)
     void *H = nullptr;               // complex half grid K3 x K2 x K1hp (x < K1h used)
     void *tw = nullptr;              // twiddles per axis: 3 x max(K) complex
@@ -258,6 +295,7 @@ struct Ctx {
     double theta_key[13]{};          // K1..K3, rcell, alpha it was computed for
     bool theta_valid = false;
     void *Q2 = nullptr;              // per-particle stress grid (a copy of the charge grid, then convolved)
+    bool grid_used = false;          // Q holds a grid spread by tiles (not cleared)
     double self_energy = 0.0;
     double sumchg = 0.0;
     bool self_done = false;
@@ -336,7 +374,7 @@ struct FftBatch {
     std::vector<int> conv_rows;    // z-pass workgroups (reduction rows) per system
 };
 struct SpmeBatch {
-    BatchLaunch spread, gather;
+    BatchLaunch splines, spread, tiles, gather;  // a system spreads by link cells or by mesh tiles
     FftBatch fft;
     int S = 0;                     // spline order (0: no system has electrostatics)
     std::vector<int> gather_rows;  // gather workgroups per system
@@ -429,6 +467,8 @@ int excl_forces(Ctx *c);                     // adds the exclusion correction in
 int excl_blocks(const Ctx *c);
 int spme_forces(Ctx *c);                     // adds into c->frc and reduction slots
 int spme_setup(Ctx *c);
+bool spread_by_tiles(const Ctx *c);          // the context's charges are spread by mesh tiles
+int tile_room(Ctx *c);                       // after a list build: that choice, and the tiles' room
 int ensure_red_rows(Ctx *c, int rows);
 int reduce_partials(Ctx *c);                 // red -> red_out (device)
 int pair_blocks(const Ctx *c);

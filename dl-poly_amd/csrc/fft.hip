@@ -738,7 +738,7 @@ constexpr int kPlaneKey = 1 << 20;                 // group keys of the plane ke
 constexpr int kGroupPlaneFwd = 5, kGroupPlaneInv = 6;  // FftGroup::kind of the plane kernels
 
 // Batched convolution Q -> Phi (influence function mode 0, the forward pass
-// clearing Q) over the systems with electrostatics: each pass is one launch
+// clearing a Q that is spread by link cells) over the systems with electrostatics: each pass is one launch
 // per group of systems, a group for each line length that has compiled line
 // kernels and one for the rest (generic kernels, with one lines-per-workgroup
 // value per pass: the smallest any of its systems needs, so every system's
@@ -823,7 +823,7 @@ static int fft_prepare_t(const std::vector<Ctx *> &cs, const std::vector<InflPar
                     [&](Ctx *c, size_t, int, int &nb, size_t &lds) {
                         nb = c->K[2];
                         lds = plane_lds<T>(n);
-                        return kind == 0 ? plane_args<T>(c, c->Q, true) : plane_args<T>(c, c->Phi, false);
+                        return kind == 0 ? plane_args<T>(c, c->Q, !spread_by_tiles(c)) : plane_args<T>(c, c->Phi, false);
                     },
                     kind == 0 ? kGroupPlaneFwd : kGroupPlaneInv, n);
             } else if (kind == 0)
@@ -831,7 +831,7 @@ static int fft_prepare_t(const std::vector<Ctx *> &cs, const std::vector<InflPar
                                              [&](Ctx *c, size_t, int l, int &nb, size_t &lds) {
                                                  nb = x_blocks(c, l);
                                                  lds = key > 0 ? lines_lds<T>(2, key) : fft_lds<T>(l, c->K[0], 0);
-                                                 return r2c_args<T>(c, c->Q, true);
+                                                 return r2c_args<T>(c, c->Q, !spread_by_tiles(c));
                                              });
             else if (kind == 4)
                 r = add_group<T, C2RArgs<T>>(cs, fb, kind, key, lpb, keys,

@@ -18,28 +18,6 @@
 
 namespace dlpx {
 
-struct CellGrid {
-    int nc[3];
-    double L[3], invL[3];
-    int sub;  // 1: bin by link cell; 2: by subcell (half the link-cell edge)
-};
-
-// Binning key of a subcell (sx, sy, sz) of edge L/(2 nc): link-cell-major,
-// then the 2 x 2 x 2 subcells of that link cell, so a link cell's atoms are
-// one contiguous run of the sorted order.
-__host__ __device__ __forceinline__ int subcell_key(const CellGrid &g, int sx, int sy, int sz)
-{
-    const int blk = ((sz >> 1) * g.nc[1] + (sy >> 1)) * g.nc[0] + (sx >> 1);
-    return blk * 8 + ((sz & 1) * 4 + (sy & 1) * 2 + (sx & 1));
-}
-
-__device__ __forceinline__ int cell_coord(double x, double L, double invL, int nc)
-{
-    // x is already folded into [-L/2, L/2)
-    int k = (int)((x * invL + 0.5) * (double)nc);
-    return k < 0 ? 0 : (k >= nc ? nc - 1 : k);
-}
-
 // Runs of equal keys among consecutive active lanes of a wavefront: the
 // lane that starts this lane's run and the run's length (all lanes of the
 // run get the same answer).  Lanes past the end of the data must have exited.
@@ -1111,7 +1089,9 @@ int build_list(Ctx *c)
         return fail(c, DLPX_ERR_LIST_OVERFLOW, "neighbour list overflow after regrowth");
     }
     c->have_list = true;
-    return 0;
+    for (int d = 0; d < 3; d++) c->list_L[d] = c->L[d];
+    c->stray_no = 0;
+    return tile_room(c);
 }
 
 // Batched list builds of an ensemble, each gated by its context's device

@@ -157,10 +157,34 @@ int freeze_atoms(Ctx *c)
     return 0;
 }
 
+// The test of an upload onto an existing list: whether each atom is still
+// within half the padding of its bin (of the last list build, in fractions of
+// the cell edge), where the tiled spreading looks for it.
+struct StrayArgs {
+    const double4 *xref;
+    double L0[3], invL0[3];   // the cell of the list build
+    double invL[3], reach[3]; // the present cell; half the padding as a fraction of its edge
+    int bins[3];
+    int32_t *flag;
+    int32_t no;
+};
+__device__ __forceinline__ bool strayed(const StrayArgs &a, const double (&x)[3], const double (&x0)[3])
+{
+    bool out = false;
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const double lo = (double)cell_coord(x0[d], a.L0[d], a.invL0[d], a.bins[d]) / (double)a.bins[d];
+        double f = x[d] * a.invL[d] + 0.5 - (lo - a.reach[d]);  // from the reach's lower end
+        f -= floor(f);
+        out = out || f > 1.0 / (double)a.bins[d] + 2.0 * a.reach[d];
+    }
+    return out;
+}
+
 // host-order staging (8 doubles per atom: x y z q vx vy vz m) -> cell order
 __global__ void k_load(const double *__restrict__ st, const int32_t *__restrict__ st_t, int n, int cap,
                        const int32_t *__restrict__ slot, bool identity, bool with_vel, double4 *pos, int32_t *typ,
-                       int32_t *gid, double4 *vel)
+                       int32_t *gid, double4 *vel, StrayArgs sa)
 {
     const int h = blockIdx.x * blockDim.x + threadIdx.x;
     if (h >= n) return;
@@ -170,6 +194,11 @@ __global__ void k_load(const double *__restrict__ st, const int32_t *__restrict_
     typ[s] = st_t[h] - 1;
     if (identity) gid[s] = h;
     if (with_vel) vel[s] = make_double4(r[4], r[5], r[6], r[7]);
+    if (!identity) {
+        const double4 q = sa.xref[s];
+        const double x[3] = {r[0], r[1], r[2]}, x0[3] = {q.x, q.y, q.z};
+        if (strayed(sa, x, x0)) *sa.flag = sa.no;
+    }
 }
 
 // cell order -> host-order staging: x y z | vx vy vz | fx fy fz
@@ -528,8 +557,23 @@ int step_launch(Ctx *c, hipStream_t s, const BatchLaunch &bl, bool stage2, bool 
 
 int load_atoms(Ctx *c, const double *st_dev, const int32_t *st_t_dev, bool identity, bool with_vel)
 {
+    StrayArgs sa{};
+    if (!identity) {
+        sa.xref = c->xref;
+        for (int d = 0; d < 3; d++) {
+            sa.L0[d] = c->list_L[d];
+            sa.invL0[d] = 1.0 / c->list_L[d];
+            sa.invL[d] = c->invL[d];
+            sa.reach[d] = 0.5 * c->prm.padding * c->invL[d] * (1.0 + 1.0e-9) + 1.0e-12;
+            sa.bins[d] = (c->list_coded ? 2 : 1) * c->nc[d];
+        }
+        sa.flag = c->flags + F_STRAY;
+        c->upload_no = c->upload_no == INT32_MAX ? 1 : c->upload_no + 1;
+        sa.no = c->upload_no;
+    }
+    c->stray_no = sa.no;
     hipLaunchKernelGGL(k_load, dim3(ceil_div(c->natms, 256)), dim3(256), 0, c->stream, st_dev, st_t_dev, c->natms,
-                       c->cap, c->slot, identity, with_vel, c->pos, c->typ, c->gid, c->vel);
+                       c->cap, c->slot, identity, with_vel, c->pos, c->typ, c->gid, c->vel, sa);
     DLPX_HIP(c, hipGetLastError());
     return 0;
 }

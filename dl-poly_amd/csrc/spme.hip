@@ -5,6 +5,9 @@
 //               LDS and each wavefront adds one atom's S^3 charge weights into
 //               an LDS window of the grid (lanes over the (x, y) plane), which
 //               is then added to the global grid.
+//  k_splines, k_spread_tiles  the splines of every atom, then one workgroup per
+//               mesh tile that sums the atoms of its list with FP64 matrix
+//               instructions and stores each grid point once.
 //  (fft.hip)    Q <- FFT-(theta . FFT+(Q)); theta(m) on the half spectrum
 //               with the spherical cutoff 0.525 min_d K_d w*_d, and the
 //               reciprocal stress.
@@ -14,6 +17,7 @@
 //  k_finish     subtracts the mean reciprocal force (ewald_general.F90:857-864),
 //               scales by 2*scale and adds into the total force.
 // FP64 or FP32 (mixed) arithmetic; sums across lanes and atoms in FP64.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -37,8 +41,8 @@ struct SpmeParams {
 // values M[t] and first derivatives D[t] at the S grid points
 // floor(u) - S + 1 + t, t = 0..S-1, evaluated with the reference's recursion
 // (S even in 4..16; the reference forces an even order, control.F90:1651-1675).
-template <typename R, bool DERIV, int S, bool DERIV2 = false>
-__device__ __forceinline__ void bspline(R w, R *M, R *D, R *D2 = nullptr)
+template <typename R, int S, bool DERIV2 = false>
+__device__ __forceinline__ void bspline_low(R w, R *z, R *D2 = nullptr)
 {
     R zd[S + 2];
 #pragma unroll
@@ -71,21 +75,28 @@ __device__ __forceinline__ void bspline(R w, R *M, R *D, R *D2 = nullptr)
         if (DERIV2) D2[S - 1] = zd[S];
         zd[S] = zd[S] * w * km1_rr;
     }
-    // l = 1 stage: first derivatives from order S-1, then raise to order S
-    {
-        const R k_r = (R)S;
-        const R km1_rr = (R)1 / (R)(S - 1);
 #pragma unroll
-        for (int j = 1; j <= S - 1; j++) {
-            if (DERIV) D[j - 1] = zd[j] - zd[j + 1];
-            const R pt = w + (R)(S - j);
-            zd[j] = (pt * zd[j] + (k_r - pt) * zd[j + 1]) * km1_rr;
-        }
-        if (DERIV) D[S - 1] = zd[S];
-        zd[S] = zd[S] * w * km1_rr;
+    for (int j = 1; j <= S; j++) z[j - 1] = zd[j];
+}
+// l = 1 stage: first derivatives from the order S-1 values z, then order S
+template <typename R, int S, bool DERIV>
+__device__ __forceinline__ void bspline_top(const R *z, R w, R *M, R *D)
+{
+    const R k_r = (R)S;
+    const R km1_rr = (R)1 / (R)(S - 1);
+#pragma unroll
+    for (int k = 0; k < S; k++) {
+        if (DERIV) D[k] = k < S - 1 ? z[k] - z[k + 1] : z[k];
+        const R pt = w + (R)(S - 1 - k);
+        M[k] = k < S - 1 ? (pt * z[k] + (k_r - pt) * z[k + 1]) * km1_rr : z[k] * w * km1_rr;
     }
-#pragma unroll
-    for (int j = 1; j <= S; j++) M[j - 1] = zd[j];
+}
+template <typename R, bool DERIV, int S, bool DERIV2 = false>
+__device__ __forceinline__ void bspline(R w, R *M, R *D, R *D2 = nullptr)
+{
+    R z[S];
+    bspline_low<R, S, DERIV2>(w, z, D2);
+    bspline_top<R, S, DERIV>(z, w, M, D);
 }
 
 // Fractional grid coordinate of one axis, folded into [0, K) so an atom that
@@ -376,6 +387,439 @@ __global__ void __launch_bounds__(spread_threads<R>()) k_spread_cells_batch(cons
     if (!batch_pos(boff, nsys, bp)) return;
     const SpreadArgs<R> &a = av[bp.s];
     spread_body<R, S>(a, bp.b);
+}
+
+// The spline data of every atom, once per evaluation, for the spreading by
+// tiles (where an atom is met in about four tiles) and the gather: per axis
+// the order S-1 values z[0..S-1] that the last step of the recursion
+// (bspline) turns into the values and first derivatives of order S,
+//   M[t] = (pt z[t] + (S - pt) z[t+1]) / (S - 1), pt = w + S - 1 - t,
+//   D[t] = z[t] - z[t+1]   (z[S] = 0),
+// in [atom][axis][S]; {w_x, w_y, w_z, charge}; and the folded grid points
+// {floor(u_x), floor(u_y), floor(u_z), whether the atom has a charge}.
+template <typename R> struct R4T;
+template <> struct R4T<double> { using type = double4; };
+template <> struct R4T<float> { using type = float4; };
+template <typename R>
+struct SplineArgs {
+    const double4 *pos;
+    int n;
+    SpmeParams sp;
+    R *z, *wq;
+    ushort4 *base;
+};
+template <typename R, int S>
+__device__ __forceinline__ void splines_body(const SplineArgs<R> &a, int bid)
+{
+    const int k = bid * 256 + threadIdx.x, i = k / 3, d = k - 3 * i;
+    if (i >= a.n) return;
+    const double4 p = a.pos[i];
+    int idx;
+    double w;
+    grid_coord(a.sp, d, p.x, p.y, p.z, idx, w);
+    R z[S];
+    bspline_low<R, S>((R)w, z);
+    R *out = a.z + (size_t)k * S;
+#pragma unroll
+    for (int m = 0; m < S; m++) out[m] = z[m];
+    a.wq[4 * (size_t)i + d] = (R)w;
+    unsigned short *b = (unsigned short *)(a.base + i);
+    b[d] = (unsigned short)idx;
+    if (d == 0) {
+        a.wq[4 * (size_t)i + 3] = (R)p.w;
+        b[3] = fabs(p.w) > kZeroPlus ? 1 : 0;
+    }
+}
+template <typename R, int S>
+__global__ void __launch_bounds__(256) k_splines(SplineArgs<R> a) { splines_body<R, S>(a, blockIdx.x); }
+template <typename R, int S>
+__global__ void __launch_bounds__(256) k_splines_batch(const SplineArgs<R> *__restrict__ av,
+                                                       const int32_t *__restrict__ boff, int nsys)
+{
+    const int lb = blockIdx.x;
+    if (lb >= boff[nsys]) return;
+    const int s = batch_find(boff, nsys, lb);
+    splines_body<R, S>(av[s], lb - boff[s]);
+}
+// Charge spreading by mesh tiles: one workgroup per tile of kTileX x kTileY x
+// kTileZ grid points sums every atom that reaches into it and stores each
+// point once, so the grid needs no atomics and no clearing.  Over the atoms,
+// a y plane of the tile is a product of matrices,
+//   Q[z][x] = sum_a (q_a Mz_a[z]) (Mx_a[x] My_a[y]),
+// 16 x 16 outputs with the atoms as the contracted index: one FP64 matrix
+// instruction adds four atoms to a plane (FP64 in both precision modes, as
+// the LDS window of k_spread_cells is).  Each wavefront holds kTilePlanes.
+//
+// The atoms come from the tile's own list, made when the Verlet list is: every
+// atom of the bins in reach that comes within half the Verlet padding of the
+// tile's reach (its points and S - 1 below them); no atom moves further
+// without a rebuild.  A host that evaluates such positions all the same is
+// noticed at the upload (F_STRAY), and then every atom is tested.  The splines
+// of a chunk of kTileChunk atoms are laid out in LDS over the tile's points
+// with zeros outside, while the next chunk's are being loaded; each chunk of
+// the list is in y order, so that a wavefront only meets the groups of four
+// that reach its planes.
+//
+// Bound by instruction issue: an FP64 matrix instruction takes the FP64
+// vector unit's time (64 cycles for 1024 multiply-adds, the rate of the vector
+// unit), about a tenth of them useful (an atom's 8 x 8 points of a 16 x 16
+// plane, 2.1 tile columns an atom at S = 8), 8 us at 64,000 ions; laying out
+// a chunk costs about as much.  With the splines' own kernel, against
+// k_spread_cells (LDS atomics, one atom per wavefront at a time):
+// 64,000 ions, 128^3, S = 8 mixed 29 against 50 us, FP64 35 against 75;
+// 1,728,000 ions mixed 532 against 894; 10,296 ions, S = 6 FP64 14 against
+// 31; 1,000 ions, 32^3 mixed 14 against 38.  One wavefront per 16 atoms with
+// all eight planes, no barriers and a last exchange of planes: 38 against 29
+// (190 registers); 16 planes to a tile: 40 against 34; a wavefront's bounds of
+// 5 per SIMD keep the list making's registers off the rest (1,728,000 ions
+// 593 -> 546).
+constexpr int kTileX = 16, kTileY = 8, kTileZ = 16;
+constexpr int kTileThreads = 256, kTileChunk = 64;
+constexpr int kTilePlanes = kTileY / (kTileThreads / 64);
+constexpr int kTileScan = 2;     // candidates a thread tests per round of a list's making
+constexpr int kTileBins = 1024;  // most bins within a tile's reach
+template <typename R>
+struct TileArgs {
+    const R *z, *wq;        // the atoms' splines and grid points (k_splines)
+    const ushort4 *base;
+    int n;
+    const int32_t *start;   // first atom of each bin
+    CellGrid g;             // sub: 1 bins are link cells, 2 subcells
+    int bins[3], tiles[3];
+    int32_t *list, *count;  // cap atoms per tile; their number, -1 none
+    int cap;
+    const double4 *xref;    // the positions of the list build, in a cell of
+    double invL0[3];        // these reciprocal edges
+    double drift_k[3];      // grid points an atom moves from there at most
+    int slack[3];           // and floor(u) changes by
+    const int32_t *upd;     // nonzero: the Verlet list is new (may be null)
+    int fresh;              // so it is
+    const int32_t *flags;
+    int32_t no;             // upload whose strays matter (F_STRAY), 0: none
+    int all;                // test every atom
+    SpmeParams sp;
+    R *Q;
+};
+// Barrier for data exchanged through LDS: global loads stay in flight.
+__device__ __forceinline__ void lds_barrier()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+__device__ __forceinline__ int lanes_before(unsigned long long mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
+}
+template <typename R, int S>
+__device__ __forceinline__ void spread_tile_body(const TileArgs<R> &a, int b)
+{
+    typedef double double4v __attribute__((ext_vector_type(4)));
+    constexpr int T[3] = {kTileX, kTileY, kTileZ}, NW = kTileThreads / 64, PW = kTilePlanes;
+    // a chunk's splines over the tile's points, an atom per row: z, x, y (the
+    // odd stride puts a column's rows on distinct banks)
+    constexpr int OX = 16, OY = 32, RS = OY + kTileY + 1;
+    static_assert(kTileX == 16 && kTileZ == 16, "planes of 16 x 16");
+    __shared__ double rows[kTileChunk * RS];
+    __shared__ int sOy[kTileChunk];
+    __shared__ int s_start[kTileBins], s_off[kTileBins];  // the making of a list
+    __shared__ int wcnt[kTileScan][NW];
+    const SpmeParams &sp = a.sp;
+    const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int tc[3] = {b % a.tiles[0], (b / a.tiles[0]) % a.tiles[1], b / (a.tiles[0] * a.tiles[1])};
+    int t0[3], reach[3];  // first point; largest floor(u) - t0 of an atom that reaches the tile
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        t0[d] = tc[d] * T[d];
+        reach[d] = min(T[d], sp.K[d] - t0[d]) + S - 2;
+    }
+    int32_t *const list = a.list + (size_t)b * a.cap;
+    double4v acc[PW];
+#pragma unroll
+    for (int p = 0; p < PW; p++) acc[p] = (double4v){0.0, 0.0, 0.0, 0.0};
+
+    // wavefronts 0-2 hold one axis each of a chunk's atoms, an atom per lane
+    const int d = wid < 3 ? wid : 0;
+    const int td = d == 0 ? t0[0] : d == 1 ? t0[1] : t0[2], rd = d == 0 ? reach[0] : d == 1 ? reach[1] : reach[2];
+    const int kd = d == 0 ? sp.K[0] : d == 1 ? sp.K[1] : sp.K[2], sd = d == 0 ? a.slack[0] : d == 1 ? a.slack[1] : a.slack[2];
+    // first point of an atom's spline relative to the tile's, the image in reach
+    auto offset = [](int idx, int t, int r, int K, int slack) {
+        int rel = idx - t;
+        if (rel < -slack) rel += K;
+        else if (rel > r + slack) rel -= K;
+        return rel - (S - 1);
+    };
+    R z[S], w = (R)0, q = (R)0;
+    int id = 0;
+    auto fetch = [&](int j) {  // the splines of atom j
+        if (wid < 3) {
+            const R *zp = a.z + ((size_t)j * 3 + d) * S;
+#pragma unroll
+            for (int k = 0; k < S; k++) z[k] = zp[k];
+            w = a.wq[4 * (size_t)j + d];
+            q = a.wq[4 * (size_t)j + 3];
+            id = ((const unsigned short *)(a.base + j))[d];
+        }
+    };
+    // the splines of the m fetched atoms over the tile's points
+    double *const row = rows + lane * RS + (d == 0 ? OX : d == 1 ? OY : 0);
+    auto lay = [&](int m) {
+        if (wid < 3) {
+            const bool on = lane < m;
+            const int od = offset(id, td, rd, kd, sd);
+            const unsigned len = d == 1 ? kTileY : 16;
+#pragma unroll
+            for (int k = 0; k < 16; k++)
+                if (d != 1 || k < kTileY) row[k] = 0.0;
+            if (d == 1) sOy[lane] = on ? od : 1 << 20;
+            R M[S];
+            bspline_top<R, S, false>(z, w, M, nullptr);
+            const R f = d == 2 ? q : (R)1;
+            // points outside the tile go to the row's padding: a select, not a branch
+            const unsigned lim = on ? len : 0u;
+            double *const pad = rows + lane * RS + RS - 1;
+#pragma unroll
+            for (int k = 0; k < S; k++) {
+                double *const out = (unsigned)(od + k) < lim ? row + od + k : pad;
+                *out = (double)(f * M[k]);
+            }
+        }
+    };
+    // the laid-out atoms into this wavefront's planes: the groups of four from
+    // the first to the last that reach one of them (a chunk is in y order), the
+    // next group's values read while the matrix unit adds the present one's
+    const double *const pzx = rows + (lane >> 4) * RS + (lane & 15), *const py = rows + (lane >> 4) * RS + OY + PW * wid;
+    struct Group {
+        double z, x, y[PW];
+    };
+    auto add = [&]() {
+        const int oy = sOy[lane], y0 = PW * wid;
+        const unsigned long long any = __ballot(oy <= y0 + PW - 1 && oy + S - 1 >= y0);
+        if (any == 0) return;
+        const int first = __builtin_ctzll(any) >> 2, last = (63 - __builtin_clzll(any)) >> 2;
+        auto read = [&](int g, Group &v) {
+            const int h = 4 * min(g, kTileChunk / 4 - 1) * RS;
+            v.z = pzx[h];
+            v.x = pzx[h + OX];
+#pragma unroll
+            for (int p = 0; p < PW; p++) v.y[p] = py[h + p];
+            __builtin_amdgcn_sched_barrier(0);  // not sunk to their use
+        };
+        auto mul = [&](const Group &v) {
+            double dy[PW];
+#pragma unroll
+            for (int p = 0; p < PW; p++) dy[p] = v.x * v.y[p];
+#pragma unroll
+            for (int p = 0; p < PW; p++) acc[p] = __builtin_amdgcn_mfma_f64_16x16x4f64(v.z, dy[p], acc[p], 0, 0, 0);
+        };
+        Group va, vb;
+        read(first, va);
+        for (int g = first; g <= last; g += 2) {
+            read(g + 1, vb);
+            mul(va);
+            if (g + 1 > last) break;
+            read(g + 2, va);
+            mul(vb);
+        }
+    };
+    // the n atoms of the list into the tile
+    auto sum = [&](int n) {
+        int jn = lane < n ? list[lane] : 0;
+        if (n > 0) fetch(jn);
+        if (n > kTileChunk) jn = list[min(kTileChunk + lane, n - 1)];
+        for (int h = 0; h < n; h += kTileChunk) {
+            lay(min(kTileChunk, n - h));
+            if (h + kTileChunk < n) {
+                fetch(jn);
+                jn = list[min(h + 2 * kTileChunk + lane, n - 1)];
+            }
+            lds_barrier();
+            add();
+            lds_barrier();
+        }
+    };
+
+    // each chunk of the list put in y order, as its atoms are placed now, so
+    // that the four atoms of a matrix instruction reach about the same planes
+    auto order = [&](int n) {
+        for (int h = wid * kTileChunk; h < n; h += NW * kTileChunk) {
+            const bool on = h + lane < n;
+            const int j = on ? list[h + lane] : 0;
+            const int oy = offset(a.base[j].y, t0[1], reach[1], sp.K[1], a.slack[1]);
+            // the atom's place, from the lanes with a smaller key and the
+            // earlier ones with the same (lanes past n last)
+            const int key = on ? min(max(oy + S, 0), 62) : 63;
+            unsigned long long less = 0, same = ~0ull;
+#pragma unroll
+            for (int bit = 5; bit >= 0; bit--) {
+                const bool one = key >> bit & 1;
+                const unsigned long long m1 = __ballot(one);
+                less |= one ? same & ~m1 : 0ull;
+                same &= one ? m1 : ~m1;
+            }
+            if (on) list[h + __popcll(less) + lanes_before(same)] = j;
+        }
+        __syncthreads();
+    };
+
+    const bool all = a.all != 0 || (a.no != 0 && a.flags[F_STRAY] == a.no);
+    const bool fresh = a.fresh != 0 || (a.upd && *a.upd != 0);
+    const int have = fresh || all ? -1 : a.count[b];
+    if (have >= 0) {
+        sum(have);
+    } else {
+        // the list made anew, from the bins within reach
+        int ncand = a.n, nq = 0;  // candidates; entries of s_off
+        if (!all) {
+            int nb[3], b0[3];
+#pragma unroll
+            for (int k = 0; k < 3; k++) {
+                const double per = (double)a.bins[k] / (double)sp.K[k];
+                const int lo = (int)floor((t0[k] - a.drift_k[k]) * per);
+                const int hi = (int)floor((t0[k] + reach[k] + 1 + a.drift_k[k]) * per);
+                nb[k] = min(hi - lo + 1, a.bins[k]);
+                b0[k] = lo;
+            }
+            // bin q of the reach, y fastest, so that a chunk holds every y (a
+            // thread takes bins U t .. U t + U-1, U as small as holds them)
+            constexpr int UM = kTileBins / kTileThreads;
+            const int nreg = nb[0] * nb[1] * nb[2], U = (nreg + kTileThreads - 1) / kTileThreads;
+            const float iby = 1.0f / (float)nb[1], ibx = 1.0f / (float)nb[0];
+            int cnt[UM], tot = 0;
+#pragma unroll
+            for (int u = 0; u < UM; u++) {
+                cnt[u] = 0;
+                const int qb = U * t + u;
+                if (u < U && qb < nreg) {
+                    int o[3];
+                    o[2] = fdiv_floor(fdiv_floor(qb, nb[1], iby, o[1]), nb[0], ibx, o[0]);
+#pragma unroll
+                    for (int k = 0; k < 3; k++) {
+                        o[k] += b0[k];
+                        if (o[k] < 0) o[k] += a.bins[k];
+                        if (o[k] >= a.bins[k]) o[k] -= a.bins[k];
+                    }
+                    const int key = a.g.sub == 2 ? subcell_key(a.g, o[0], o[1], o[2])
+                                                 : (o[2] * a.g.nc[1] + o[1]) * a.g.nc[0] + o[0];
+                    const int st = a.start[key];
+                    cnt[u] = a.start[key + 1] - st;
+                    s_start[qb] = st;
+                }
+                tot += cnt[u];
+            }
+            int incl = tot;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += y;
+            }
+            if (lane == 63) wcnt[0][wid] = incl;
+            __syncthreads();
+            int run = incl - tot;
+            for (int v = 0; v < wid; v++) run += wcnt[0][v];
+            ncand = 0;
+            for (int v = 0; v < NW; v++) ncand += wcnt[0][v];
+#pragma unroll
+            for (int u = 0; u < UM; u++)
+                if (u < U) {
+                    s_off[U * t + u] = run;
+                    run += cnt[u];
+                }
+            nq = U * kTileThreads;
+            __syncthreads();
+        }
+        int fill = 0;
+        bool whole = !all;  // the list so far holds every atom found
+        for (int c0 = 0; c0 < ncand; c0 += kTileScan * kTileThreads) {
+            int j[kTileScan];
+            double at[kTileScan][3];  // where the atom was at the list build, or is if it is looked for anywhere
+#pragma unroll
+            for (int u = 0; u < kTileScan; u++) {
+                j[u] = min(c0 + u * kTileThreads + t, ncand - 1);
+                if (!all) {
+                    int lo = 0;  // the last bin with off[lo] <= j
+#pragma unroll
+                    for (int s = kTileBins / 2; s > 0; s >>= 1)
+                        if (lo + s < nq && s_off[lo + s] <= j[u]) lo += s;
+                    j[u] = s_start[lo] + (j[u] - s_off[lo]);
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < kTileScan; u++) {
+                if (all) {
+                    const ushort4 pb = a.base[j[u]];
+                    const R *w = a.wq + 4 * (size_t)j[u];
+                    at[u][0] = pb.x + (double)w[0];
+                    at[u][1] = pb.y + (double)w[1];
+                    at[u][2] = pb.z + (double)w[2];
+                } else {
+                    const double4 p = a.xref[j[u]];
+                    at[u][0] = p.x;
+                    at[u][1] = p.y;
+                    at[u][2] = p.z;
+                }
+            }
+            unsigned long long mask[kTileScan];
+#pragma unroll
+            for (int u = 0; u < kTileScan; u++) {
+                bool in = c0 + u * kTileThreads + t < ncand;
+#pragma unroll
+                for (int x = 0; x < 3; x++) {
+                    double rel = (all ? at[u][x] : sp.kr[x] * (at[u][x] * a.invL0[x] + 0.5)) - t0[x];
+                    if (rel < -a.drift_k[x]) rel += sp.K[x];
+                    else if (rel >= sp.K[x] - a.drift_k[x]) rel -= sp.K[x];  // just below the tile's first point
+                    in = in && !(rel >= reach[x] + 1 + a.drift_k[x]);
+                }
+                mask[u] = __ballot(in);
+                if (lane == 0) wcnt[u][wid] = __popcll(mask[u]);
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < kTileScan; u++)
+#pragma unroll
+                for (int v = 0; v < NW; v++) {
+                    if (v == wid && (mask[u] >> lane & 1)) list[fill + lanes_before(mask[u])] = j[u];
+                    fill += wcnt[u][v];
+                }
+            __syncthreads();
+            if (fill + kTileScan * kTileThreads > a.cap && c0 + kTileScan * kTileThreads < ncand) {
+                // no room for another round: what is there goes into the tile now
+                order(fill);
+                sum(fill);
+                fill = 0;
+                whole = false;
+            }
+        }
+        if (t == 0) a.count[b] = whole ? fill : -1;
+        order(fill);
+        sum(fill);
+    }
+    // lane l of plane y holds x = l % 16 and z = 4 r + l / 16, r = 0..3
+    const int gx = t0[0] + (lane & 15);
+#pragma unroll
+    for (int p = 0; p < PW; p++) {
+        const int gy = t0[1] + PW * wid + p;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const int gz = t0[2] + 4 * r + (lane >> 4);
+            if (gx < sp.K[0] && gy < sp.K[1] && gz < sp.K[2])
+                a.Q[((size_t)gz * sp.K[1] + gy) * sp.K[0] + gx] = (R)acc[p][r];
+        }
+    }
+}
+template <typename R, int S>
+__global__ void __launch_bounds__(kTileThreads, 5) k_spread_tiles(TileArgs<R> a)
+{
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    if (b < a.tiles[0] * a.tiles[1] * a.tiles[2]) spread_tile_body<R, S>(a, b);
+}
+template <typename R, int S>
+__global__ void __launch_bounds__(kTileThreads, 5) k_spread_tiles_batch(const TileArgs<R> *__restrict__ av,
+                                                                     const int32_t *__restrict__ boff, int nsys)
+{
+    BatchPos bp;
+    if (!batch_pos(boff, nsys, bp)) return;
+    spread_tile_body<R, S>(av[bp.s], bp.b);
 }
 
 // Lanes per atom in the gather: the next power of two >= S, lane tx < S
@@ -729,6 +1173,9 @@ int spme_setup(Ctx *c)
     DLPX_HIP(c, hipMalloc(&c->theta, 2 * rs * c->nhalf));
     DLPX_HIP(c, dev_zero(c->stream, c->theta, 2 * rs * c->nhalf));  // the row padding stays zero
     c->theta_valid = false;
+    DLPX_HIP(c, hipMalloc(&c->spl_z, rs * 3 * S * (size_t)c->cap));
+    DLPX_HIP(c, hipMalloc(&c->spl_wq, rs * 4 * (size_t)c->cap));
+    DLPX_HIP(c, hipMalloc((void **)&c->spl_base, sizeof(ushort4) * (size_t)c->cap));
     const int ksum = c->K[0] + c->K[1] + c->K[2];
     std::vector<double> n2(ksum);
     bspline_norm2(c->K[0], S, n2.data());
@@ -780,6 +1227,111 @@ static SpreadArgs<R> spread_args(const Ctx *c)
 {
     return SpreadArgs<R>{c->pos, c->cell_start, c->ncell, spme_params(c), (R *)c->Q};
 }
+// Grid points an atom moves along axis d at most between list builds.
+static double tile_drift(const Ctx *c, int d)
+{
+    return 0.5 * c->prm.padding * c->K[d] / c->list_L[d] * (1.0 + 1.0e-6) + 1.0e-4;
+}
+static int tile_slack(const Ctx *c, int d) { return (int)std::ceil(tile_drift(c, d)) + 1; }
+static int tile_blocks(const Ctx *c)
+{
+    return ceil_div(c->K[0], kTileX) * ceil_div(c->K[1], kTileY) * ceil_div(c->K[2], kTileZ);
+}
+// Mesh tiles need a mesh that holds a tile and an atom's reach without
+// meeting itself (an atom then has one image in reach of a tile), and bins
+// not much finer than a tile (kTileBins of them in reach).
+static bool tiles_fit(const Ctx *c)
+{
+    if (!c->prm.electrostatics || c->spread_tiles == 0) return false;
+    const int T[3] = {kTileX, kTileY, kTileZ}, S = c->prm.nsplines;
+    long bins = 1;
+    for (int d = 0; d < 3; d++) {
+        if (c->K[d] < T[d] + S - 1 + 2 * tile_slack(c, d)) return false;
+        const int nb = (c->list_coded ? 2 : 1) * c->nc[d];
+        bins *= std::min<long>(nb, (long)((T[d] + S - 1 + 2.0 * tile_drift(c, d)) * nb / c->K[d]) + 2);
+    }
+    return bins <= kTileBins;
+}
+// A host that asks for one evaluation of a Verlet list has no use for the
+// tiles' lists, whose making costs more than they save in one: its first
+// evaluation spreads by link cells, the next by tiles (4,000 atoms of three
+// species on 36^3: 14 us by cells, 32 by tiles with the making of the lists).
+bool spread_by_tiles(const Ctx *c) { return c->tile_cap > 0 && (c->resident || c->tile_lists || c->list_evals > 0); }
+// After a list build: whether the charges are spread by tiles, and room for
+// the tiles' lists (1.3 times the mean, and one round of their making).
+// Where the mesh allows, the faster of the two by their measured times: a
+// tile's workgroup takes 1.35 us for each chunk of its atoms, one by link
+// cells 0.27 us for each atom of its cell, the busiest CU sets the time, and
+// they start from 3.5 us (the splines' kernel) and 5.  Many tiles or none on
+// a CU, tiles win by their lower rate; few atoms in many link cells and many
+// in few tiles (a coarse mesh) are the other case: 4,000 atoms on 36^3, 216
+// cells and 45 tiles, 14 us by cells and 21 by tiles.
+int tile_room(Ctx *c)
+{
+    c->tile_cap = 0;
+    c->tile_lists = false;
+    c->list_evals = 0;
+    if (!tiles_fit(c)) return 0;
+    const int T[3] = {kTileX, kTileY, kTileZ};
+    double mean = c->natms;
+    for (int d = 0; d < 3; d++)
+        mean *= std::min(1.0, (T[d] + c->prm.nsplines - 1 + 2.0 * tile_drift(c, d)) / c->K[d]);
+    const double chunks = mean / kTileChunk, cells = std::max(1, c->ncell);
+    if (c->spread_tiles < 0 &&
+        1.35 * chunks * std::max(1.0, tile_blocks(c) / 256.0) + 3.5 >
+        0.27 * c->natms / std::min(cells, 256.0) + 5.0)
+        return 0;
+    const int cap = kTileScan * kTileThreads + (int)(1.3 * mean / 64.0 + 1.0) * 64;
+    const size_t words = (size_t)tile_blocks(c) * (cap + 1);
+    if (words > c->tile_words) {
+        if (c->tile_list) (void)hipFree(c->tile_list);
+        c->tile_list = nullptr;
+        c->tile_words = 0;
+        DLPX_HIP(c, hipMalloc((void **)&c->tile_list, sizeof(int32_t) * words));
+        c->tile_words = words;
+    }
+    c->tile_cap = cap;
+    return 0;
+}
+template <typename R>
+static SplineArgs<R> spline_args(const Ctx *c)
+{
+    return SplineArgs<R>{c->pos, c->natms, spme_params(c), (R *)c->spl_z, (R *)c->spl_wq, c->spl_base};
+}
+static int spline_blocks(const Ctx *c) { return ceil_div(3L * c->natms, 256); }
+template <typename R>
+static TileArgs<R> tile_args(const Ctx *c, int32_t no, const int32_t *upd)
+{
+    const int T[3] = {kTileX, kTileY, kTileZ};
+    TileArgs<R> a{};
+    a.z = (const R *)c->spl_z;
+    a.wq = (const R *)c->spl_wq;
+    a.base = c->spl_base;
+    a.n = c->natms;
+    a.g.sub = c->list_coded ? 2 : 1;
+    a.start = c->list_coded ? c->key_start : c->cell_start;
+    a.list = c->tile_list;
+    a.cap = c->tile_cap;
+    a.count = c->tile_list + (size_t)tile_blocks(c) * c->tile_cap;
+    a.xref = c->xref;
+    a.upd = upd;
+    a.fresh = c->tile_lists ? 0 : 1;
+    a.flags = c->flags;
+    a.no = no;
+    for (int d = 0; d < 3; d++) {
+        a.g.nc[d] = c->nc[d];
+        a.bins[d] = a.g.sub * c->nc[d];
+        a.tiles[d] = ceil_div(c->K[d], T[d]);
+        a.invL0[d] = 1.0 / c->list_L[d];
+        a.drift_k[d] = tile_drift(c, d);
+        a.slack[d] = tile_slack(c, d);
+        // the lists of another cell than the present one, positions not compared with them
+        if (no == 0 && c->list_L[d] != c->L[d]) a.all = 1;
+    }
+    a.sp = spme_params(c);
+    a.Q = (R *)c->Q;
+    return a;
+}
 template <typename R>
 static GatherArgs<R> gather_args(const Ctx *c)
 {
@@ -799,6 +1351,23 @@ static GatherArgs<R> gather_args(const Ctx *c)
     }
 
 template <typename R>
+__global__ void __launch_bounds__(256) k_zero(R *p, size_t n)
+{
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) p[i] = (R)0;
+}
+// The charge grid zero for a spreading by link cells, after one by tiles.
+template <typename R>
+static int grid_zero(Ctx *c, hipStream_t s)
+{
+    if (!c->grid_used) return 0;
+    hipLaunchKernelGGL((k_zero<R>), dim3(std::min<size_t>((c->nreal + 255) / 256, 2048)), dim3(256), 0, s, (R *)c->Q,
+                       c->nreal);
+    DLPX_HIP(c, hipGetLastError());
+    c->grid_used = false;
+    return 0;
+}
+
+template <typename R>
 static int spme_run(Ctx *c)
 {
     const int n = c->natms;
@@ -806,14 +1375,31 @@ static int spme_run(Ctx *c)
     const SpmeParams sp = spme_params(c);
     const int nb = gather_blocks(c);  // evaluate() has sized the partial-sum rows
     int r;
-    // ewald_general.F90:517-576 charge spreading into the charge grid, which
-    // is zero here: set at allocation, and cleared by the forward x pass of
-    // each convolution after reading it
-    const SpreadArgs<R> spa = spread_args<R>(c);
+    // ewald_general.F90:517-576 charge spreading into the charge grid
+    const bool tiles = spread_by_tiles(c);
+    c->list_evals++;
+    if (tiles) {
+        const SplineArgs<R> sa = spline_args<R>(c);
+#define DLPX_SPLINES(SS) hipLaunchKernelGGL((k_splines<R, SS>), dim3(spline_blocks(c)), dim3(256), 0, s, sa)
+        DLPX_S_SWITCH(sp.S, DLPX_SPLINES)
+#undef DLPX_SPLINES
+        const TileArgs<R> ta = tile_args<R>(c, c->stray_no, nullptr);
+#define DLPX_TILES(SS) \
+    hipLaunchKernelGGL((k_spread_tiles<R, SS>), dim3(xcd_grid(tile_blocks(c))), dim3(kTileThreads), 0, s, ta)
+        DLPX_S_SWITCH(sp.S, DLPX_TILES)
+#undef DLPX_TILES
+        c->grid_used = true;
+        c->tile_lists = true;
+    } else {
+        // onto a grid that is zero here: set at allocation, and cleared by
+        // the forward x pass of each convolution after reading it
+        if ((r = grid_zero<R>(c, s))) return r;
+        const SpreadArgs<R> spa = spread_args<R>(c);
 #define DLPX_SPREAD(SS) \
     hipLaunchKernelGGL((k_spread_cells<R, SS>), dim3(xcd_grid(c->ncell)), dim3(spread_threads<R>()), 0, s, spa)
-    DLPX_S_SWITCH(sp.S, DLPX_SPREAD)
+        DLPX_S_SWITCH(sp.S, DLPX_SPREAD)
 #undef DLPX_SPREAD
+    }
     if (c->timing) DLPX_HIP(c, hipEventRecord(c->ev[2], s));
     InflParams ip = infl_params(c);
     if (c->pp_now) {
@@ -821,7 +1407,7 @@ static int spme_run(Ctx *c)
         const size_t bytes = (c->prm.precision == DLPX_MIXED ? sizeof(float) : sizeof(double)) * c->nreal;
         DLPX_HIP(c, hipMemcpyAsync(c->Q2, c->Q, bytes, hipMemcpyDeviceToDevice, s));
     }
-    if ((r = fft_convolve(c, ip, c->Q, c->Phi, true))) return r;
+    if ((r = fft_convolve(c, ip, c->Q, c->Phi, !tiles))) return r;
     if (c->timing) DLPX_HIP(c, hipEventRecord(c->ev[3], s));
     const GatherArgs<R> ga = gather_args<R>(c);
 #define DLPX_GATHER(SS) hipLaunchKernelGGL((k_gather<R, SS>), dim3(nb), dim3(256), 0, s, ga)
@@ -856,10 +1442,12 @@ template <typename R>
 static int spme_prepare_t(const std::vector<Ctx *> &cs, SpmeBatch &sb)
 {
     std::vector<SpreadArgs<R>> spa;
+    std::vector<SplineArgs<R>> sa;
+    std::vector<TileArgs<R>> ta;
     std::vector<GatherArgs<R>> ga;
     std::vector<InflParams> ips;
-    std::vector<int> nbs, nbg;
-    int S = 0;
+    std::vector<int> nbp, nbs, nbt, nbg;
+    int r, S = 0;
     for (Ctx *c : cs) {
         const bool on = c->prm.electrostatics != 0;
         if (on) {
@@ -867,16 +1455,27 @@ static int spme_prepare_t(const std::vector<Ctx *> &cs, SpmeBatch &sb)
                 return fail(c, DLPX_ERR_UNSUPPORTED, "systems of one batch must share the spline order");
             S = c->prm.nsplines;
         }
-        spa.push_back(on ? spread_args<R>(c) : SpreadArgs<R>{});
+        const bool tiles = on && spread_by_tiles(c);
+        if (tiles) c->grid_used = true;
+        else if (on) {
+            if ((r = grid_zero<R>(c, c->stream))) return r;
+            DLPX_HIP(c, hipStreamSynchronize(c->stream));
+        }
+        sa.push_back(tiles ? spline_args<R>(c) : SplineArgs<R>{});
+        nbp.push_back(tiles ? spline_blocks(c) : 0);
+        spa.push_back(on && !tiles ? spread_args<R>(c) : SpreadArgs<R>{});
+        ta.push_back(tiles ? tile_args<R>(c, 0, c->flags + F_UPD) : TileArgs<R>{});
         ga.push_back(on ? gather_args<R>(c) : GatherArgs<R>{});
         ga.back().acc = on ? c->acc : nullptr;
         ips.push_back(on ? infl_params(c) : InflParams{});
-        nbs.push_back(on ? c->ncell : 0);
+        nbs.push_back(on && !tiles ? c->ncell : 0);
+        nbt.push_back(tiles ? tile_blocks(c) : 0);
         nbg.push_back(on ? gather_blocks_exact(c) : 0);
     }
     sb.S = S;
-    int r;
     if ((r = batch_upload(cs[0], sb.spread, spa.data(), sizeof(SpreadArgs<R>), nbs, true)) ||
+        (r = batch_upload(cs[0], sb.splines, sa.data(), sizeof(SplineArgs<R>), nbp, false)) ||
+        (r = batch_upload(cs[0], sb.tiles, ta.data(), sizeof(TileArgs<R>), nbt, true)) ||
         (r = batch_upload(cs[0], sb.gather, ga.data(), sizeof(GatherArgs<R>), nbg, true)))
         return r;
     sb.gather_rows = nbg;
@@ -893,11 +1492,27 @@ template <typename R>
 static int spme_launch_t(Ctx *c, hipStream_t s, const SpmeBatch &sb, hipEvent_t *marks)
 {
     if (sb.S == 0) return 0;
-    const BatchLaunch &bs = sb.spread, &bg = sb.gather;
+    const BatchLaunch &bp = sb.splines, &bs = sb.spread, &bt = sb.tiles, &bg = sb.gather;
+#define DLPX_SPLINESB(SS)                                                                                        \
+    hipLaunchKernelGGL((k_splines_batch<R, SS>), dim3(bp.total), dim3(256), 0, s, (const SplineArgs<R> *)bp.args, \
+                       bp.boff, bp.nsys)
+    if (bp.total > 0) {
+        DLPX_S_SWITCH(sb.S, DLPX_SPLINESB)
+    }
+#undef DLPX_SPLINESB
+#define DLPX_TILESB(SS)                                                                                          \
+    hipLaunchKernelGGL((k_spread_tiles_batch<R, SS>), dim3(bt.total), dim3(kTileThreads), 0, s,                  \
+                       (const TileArgs<R> *)bt.args, bt.boff, bt.nsys)
+    if (bt.total > 0) {
+        DLPX_S_SWITCH(sb.S, DLPX_TILESB)
+    }
+#undef DLPX_TILESB
 #define DLPX_SPREADB(SS)                                                                                         \
     hipLaunchKernelGGL((k_spread_cells_batch<R, SS>), dim3(bs.total), dim3(spread_threads<R>()), 0, s,          \
                        (const SpreadArgs<R> *)bs.args, bs.boff, bs.nsys)
-    DLPX_S_SWITCH(sb.S, DLPX_SPREADB)
+    if (bs.total > 0) {
+        DLPX_S_SWITCH(sb.S, DLPX_SPREADB)
+    }
 #undef DLPX_SPREADB
     if (marks && marks[0]) DLPX_HIP(c, hipEventRecord(marks[0], s));
     int r;

@@ -924,3 +924,68 @@ def test_fortran_host_through_iso_c_binding(tmp_path, precision):
     tol_md = 1e-10 if precision == 0 else 1e-5
     assert np.abs(dx).max() <= tol_md * L.max()
     assert rms_rel(md_v, v) <= tol_md and rms_rel(md_f, f) <= 10 * tol_md
+
+
+# mesh, spline order: meshes of whole and partial tiles (16 x 8 x 16 points),
+# the smallest that hold a tile and its reach, two link cells per axis (bins
+# are link cells) and more (subcells), every spline order
+@pytest.mark.parametrize("ncells,kvec,order", [((5, 5, 5), (32, 32, 32), 8), ((5, 6, 7), (27, 30, 24), 4),
+                                               ((7, 8, 9), (45, 50, 54), 6), ((7, 7, 7), (36, 40, 48), 10),
+                                               ((8, 7, 6), (48, 36, 40), 12), ((6, 6, 6), (40, 36, 45), 14),
+                                               ((7, 7, 8), (50, 48, 40), 16)])
+def test_tile_and_cell_spreading_agree(ncells, kvec, order, monkeypatch):
+    """The spreading by mesh tiles, which a list's second evaluation takes, and
+    by link cells (DLPX_SPREAD_TILES=0): on the list's own positions, on
+    moved ones, on ones moved further than the tiles' lists allow for (every
+    atom by up to 3 A without a rebuild) and in a cell scaled by half a
+    percent since the build; and in resident steps across rebuilds.  Both add
+    the same products in FP64: 1e-12 apart at most in FP64; in the mixed mode
+    the grid is rounded to FP32 once against once per link cell, and each
+    spline weight once, 1e-6."""
+    s = systems.nacl(ncells=ncells, kvec=kvec, nsplines=order, seed=11)
+    rng = np.random.default_rng(12)
+    near = s.pos + rng.uniform(-0.14, 0.14, s.pos.shape)
+    far = s.pos + rng.uniform(-3.0, 3.0, s.pos.shape)
+    for precision, tol in ((lib.FP64, 1e-12), (lib.MIXED, 1e-6)):
+        res = {}
+        for tiles in ("1", "0"):
+            monkeypatch.setenv("DLPX_SPREAD_TILES", tiles)
+            ctx = lib.Context(s, precision=precision)
+            ctx.link_cell_pairs(s.pos)
+            got = [ctx.two_body_forces(p) for p in (s.pos, s.pos, near, far, near)]
+            ctx.cell = ctx.cell * 1.005
+            got += [ctx.two_body_forces(p) for p in (near * 1.005, far)]
+            ctx.cell = ctx.cell / 1.005
+            ctx.link_cell_pairs(near)
+            got += [ctx.two_body_forces(near), ctx.two_body_forces(s.pos)]
+            ctx.md_load(s.pos, s.vel)
+            ctx.md_run(12, s.timestep)
+            got.append(dict(frc=ctx.md_store()[2], engcpe=ctx.md_last_output()["engcpe"]))
+            ctx.close()
+            res[tiles] = got
+        for k, (a, b) in enumerate(zip(res["1"], res["0"])):
+            # 12 steps let the differences of the first grow tenfold at most
+            t = tol * (10.0 if k == len(res["0"]) - 1 else 1.0)
+            print("case", ncells, order, precision, k, rms_rel(a["frc"], b["frc"]), flush=True)
+            assert rms_rel(a["frc"], b["frc"]) <= t, (precision, k)
+            assert abs(a["engcpe"] - b["engcpe"]) <= t * abs(b["engcpe"]), (precision, k)
+
+
+def test_tile_lists_longer_than_their_room(monkeypatch):
+    """A droplet: all the ions of one corner of the box, so that a tile's list
+    outgrows its room (sized by the mean density) and the tile adds it in
+    several rounds.  Against the spreading by link cells, FP64 to rounding."""
+    s = systems.nacl(ncells=10, kvec=(64, 64, 64), seed=13)
+    s.pos = s.pos * 0.35 - 0.3 * s.cell[0]
+    s.cutoff = s.vdw_cutoff = 6.0
+    got = {}
+    for tiles in ("1", "0"):
+        monkeypatch.setenv("DLPX_SPREAD_TILES", tiles)
+        ctx = lib.Context(s, precision=lib.FP64)
+        ctx.link_cell_pairs(s.pos)
+        got[tiles] = [ctx.two_body_forces(s.pos) for _ in range(3)]
+        ctx.close()
+    for a, b in zip(got["1"], got["0"]):
+        # the close ions' real-space forces dominate; the reciprocal energy shows the spreading
+        assert rms_rel(a["frc"], b["frc"]) <= 1e-12
+        assert abs(a["buffer"][9] - b["buffer"][9]) <= 1e-12 * abs(b["buffer"][9])
