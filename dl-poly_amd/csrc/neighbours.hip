@@ -9,6 +9,7 @@
 // split over G lanes per atom: lane g keeps every G-th candidate it accepts,
 // element (i, c, g) lives at nbr[(i*cap_lane + c)*G + g] (list_slot), so one
 // atom's entries, and one workgroup's atoms, are contiguous.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -272,10 +273,12 @@ __device__ __forceinline__ void sort_permute_body(const SortArgs &a, int c)
     for (int k = threadIdx.x; k < n; k += blockDim.x) permute_one(a, s + k, sorted[k]);
 }
 
-// One workgroup per link cell.  The atoms of the (up to) 27 stencil cells
-// are staged once in LDS as float4 {x + sx, y + sy, z + sz, j}, with the
-// cell's periodic image shift s L already added, and then every atom of the
-// cell (G lanes each, lane g taking candidates k = g, g + G, ...) tests them.
+// The link-cell build: parts workgroups per link cell.  The atoms of the (up
+// to) 27 stencil cells are staged once in LDS as float4 {x + sx, y + sy,
+// z + sz, j}, with the cell's periodic image shift s L already added, and then
+// the cell's atoms are tested against them, one per wavefront at a time: the
+// 64 lanes test 64 candidates, and the accepted ones are packed with a ballot
+// into the atom's next entries (entry e at list_slot(i, e / G, e % G)).
 //
 // Positions are folded into [-L/2, L/2) at the rebuild, so a stencil cell's
 // image shift is -L, 0 or +L per axis.  The separation is x_i - (x_j + s L)
@@ -285,11 +288,15 @@ __device__ __forceinline__ void sort_permute_body(const SortArgs &a, int c)
 // precision without fused multiply-add from the FP64 positions, with the
 // arithmetic of the host, so the accepted set is reproducible bit for bit.
 // With fewer than 3 cells on an axis the stencil shift need not be the
-// minimum image, and every candidate is decided exactly by minimum image.
+// minimum image, which is then taken of the single-precision separation (it
+// is ambiguous only at half the cell, beyond the cutoff).  1,000 ions in 8
+// cells: 15 us, against 136 with one workgroup per cell and four lanes to an
+// atom, whose every candidate was decided in FP64 from memory.
 //
 // Stencils with more than kListStage candidates are processed in rounds.
 constexpr int kListThreads = 512;
 constexpr int kListStage = 3072;  // 48 KB of float4
+constexpr int kListAtomChunk = 256;  // atoms of a link cell whose counts persist across staging rounds
 // The workgroup's partial counters into the build's flags (one global
 // atomic each: a single address hit by every atom would serialise tens of
 // thousands of atomics); an overflow also sets the sticky F_OVF_ANY that a
@@ -313,24 +320,28 @@ struct BuildArgs {
     int32_t *nbr, *cnt, *flags;
     const int32_t *upd;
     int32_t *sub_of;  // subcell build: each atom's subcell (see Ctx::sub_of)
+    int parts;        // workgroups per link cell, each taking some of its atoms
 };
 template <int G>
-__device__ __forceinline__ void build_list_body(const BuildArgs &a, int c)
+__device__ __forceinline__ void build_list_body(const BuildArgs &a, int b)
 {
     static_assert(G == kLanesPerAtom, "list_slot assumes kLanesPerAtom lanes per atom");
-    __shared__ float4 cand[kListStage];
+    __shared__ float4 cand[kListStage + 64];
     __shared__ int s_start[27], s_off[28];
     __shared__ double s_sh[27][3];
+    __shared__ int s_acnt[kListAtomChunk];
     __shared__ int s_ovf, s_big, s_tot;  // workgroup partials of flags[0], [1], [3]
     const double4 *__restrict__ pos = a.pos;
     const CellGrid &g = a.g;
     const int32_t *__restrict__ start = a.start;
     const double rc2 = a.rc2;
-    const int cap_lane = a.cap_lane;
+    const int cap_lane = a.cap_lane, cap_tot = cap_lane * G;
     int32_t *__restrict__ nbr = a.nbr;
     int32_t *__restrict__ cnt = a.cnt;
+    const int c = b / a.parts, part = b - c * a.parts;
     if (c >= g.nc[0] * g.nc[1] * g.nc[2]) return;
-    const int t = threadIdx.x;
+    const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6);
+    constexpr int NW = kListThreads / 64;
     if (t == 0) {
         s_ovf = 0;
         s_big = 0;
@@ -348,7 +359,7 @@ __device__ __forceinline__ void build_list_body(const BuildArgs &a, int c)
             const int lo = g.nc[d] >= 3 ? -1 : 0, hi = g.nc[d] >= 2 ? 1 : 0;
             valid = valid && o[d] >= lo && o[d] <= hi;
             jj[d] = (cc[d] + o[d] + g.nc[d]) % g.nc[d];
-            s_sh[t][d] = (double)((cc[d] + o[d]) - jj[d]) / g.nc[d] * g.L[d];
+            s_sh[t][d] = small ? 0.0 : (double)((cc[d] + o[d]) - jj[d]) / g.nc[d] * g.L[d];
         }
         const int jc = (jj[2] * g.nc[1] + jj[1]) * g.nc[0] + jj[0];
         s_start[t] = start[jc];
@@ -361,19 +372,17 @@ __device__ __forceinline__ void build_list_body(const BuildArgs &a, int c)
     }
     __syncthreads();
     const int ncand = s_off[27];
-    const int hs = start[c], he = start[c + 1];
+    const int hs = start[c], nat = start[c + 1] - hs;
     const float rc2_lo = (float)(rc2 * (1.0 - 2.0e-5)), rc2_hi = (float)(rc2 * (1.0 + 2.0e-5));
-    for (int h0 = hs; h0 < he; h0 += kListThreads / G) {
-        const int i = h0 + t / G, lane = t % G;
-        const bool active = i < he;
-        const double4 pi = active ? pos[i] : make_double4(0.0, 0.0, 0.0, 0.0);
-        const float pfx = (float)pi.x, pfy = (float)pi.y, pfz = (float)pi.z;
-        int count = 0;
+    const float Lf[3] = {(float)g.L[0], (float)g.L[1], (float)g.L[2]};
+    const float iLf[3] = {(float)g.invL[0], (float)g.invL[1], (float)g.invL[2]};
+    for (int a0 = 0; a0 < nat; a0 += kListAtomChunk) {
+        const int a1 = min(nat, a0 + kListAtomChunk);
         for (int r0 = 0; r0 < ncand; r0 += kListStage) {
             const int m = min(kListStage, ncand - r0);
-            // stage candidates r0 .. r0+m-1 (skipped when a single round is
-            // already in LDS from the previous pass of atoms)
-            if (!(r0 == 0 && m == ncand && h0 > hs)) {
+            const bool last = r0 + m == ncand;
+            // stage candidates r0 .. r0+m-1 (kept when one round holds them all)
+            if (!(r0 == 0 && last && a0 > 0)) {
                 __syncthreads();
                 constexpr int U = 6;
                 for (int k0 = t; k0 < m; k0 += U * kListThreads) {
@@ -403,66 +412,54 @@ __device__ __forceinline__ void build_list_body(const BuildArgs &a, int c)
                 }
                 __syncthreads();
             }
-            if (!active) continue;
-            if (small) {
-                // 1-2 cells per axis: every candidate decided by exact minimum image
-                for (int k = lane; k < m; k += G) {
-                    const int j = __float_as_int(cand[k].w);
-                    if (j == i) continue;
-                    const double4 pj = pos[j];
-                    const double dx = min_image_1(pi.x, pj.x, g.L[0], g.invL[0]);
-                    const double dy = min_image_1(pi.y, pj.y, g.L[1], g.invL[1]);
-                    const double dz = min_image_1(pi.z, pj.z, g.L[2], g.invL[2]);
-                    const double rsq = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-                    if (rsq <= rc2) {
-                        if (count < cap_lane) nbr[list_slot(i, count, lane, cap_lane)] = j;
-                        count++;
+            for (int q = a0 + part * NW + wid; q < a1; q += NW * a.parts) {
+                const int i = hs + q;
+                const double4 pi = pos[i];
+                const float pfx = (float)pi.x, pfy = (float)pi.y, pfz = (float)pi.z;
+                int32_t *const row_out = nbr + list_slot(i, 0, 0, cap_lane);
+                int count = __builtin_amdgcn_readfirstlane(r0 == 0 ? 0 : s_acnt[q - a0]);
+                for (int k0 = 0; k0 < m; k0 += 64) {
+                    const float4 e = cand[k0 + lane];
+                    const int j = __float_as_int(e.w);
+                    float ex = pfx - e.x, ey = pfy - e.y, ez = pfz - e.z;
+                    if (small) {
+                        ex -= Lf[0] * rintf(ex * iLf[0]);
+                        ey -= Lf[1] * rintf(ey * iLf[1]);
+                        ez -= Lf[2] * rintf(ez * iLf[2]);
                     }
-                }
-                continue;
-            }
-            // the accept test is predicated rather than branched (divergent
-            // branches here cost more scalar than vector instructions), and
-            // the rare band of pairs within 2e-5 of the cutoff is settled in
-            // FP64 behind a wavefront-uniform test
-#pragma unroll 2
-            for (int k = lane; k < m; k += G) {
-                const float4 e = cand[k];
-                const int j = __float_as_int(e.w);
-                const float ex = pfx - e.x, ey = pfy - e.y, ez = pfz - e.z;
-                const float r2f = ex * ex + ey * ey + ez * ez;
-                bool in = r2f < rc2_lo && j != i;
-                const bool near = r2f >= rc2_lo && r2f <= rc2_hi && j != i;
-                if (__any(near)) {
-                    if (near) {
-                        // x_i - (x_j + s L) with the stencil's s, which for a pair this
-                        // close (well under L/2) is the minimum image
-                        const double4 pj = pos[j];
-                        const double dx = min_image_1(pi.x, pj.x, g.L[0], g.invL[0]);
-                        const double dy = min_image_1(pi.y, pj.y, g.L[1], g.invL[1]);
-                        const double dz = min_image_1(pi.z, pj.z, g.L[2], g.invL[2]);
-                        const double rsq = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)),
-                                                     __dmul_rn(dz, dz));
-                        in = rsq <= rc2;
+                    const float r2f = ex * ex + ey * ey + ez * ez;
+                    bool in = lane < m - k0 && j != i && r2f <= rc2_hi;
+                    const bool near = in && r2f >= rc2_lo;
+                    if (__any(near)) {
+                        if (near) {
+                            // x_i - (x_j + s L) at the minimum image
+                            const double4 pj = pos[j];
+                            const double dx = min_image_1(pi.x, pj.x, g.L[0], g.invL[0]);
+                            const double dy = min_image_1(pi.y, pj.y, g.L[1], g.invL[1]);
+                            const double dz = min_image_1(pi.z, pj.z, g.L[2], g.invL[2]);
+                            const double rsq = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)),
+                                                         __dmul_rn(dz, dz));
+                            in = rsq <= rc2;
+                        }
                     }
+                    const unsigned long long acc = __ballot(in);
+                    const int slot = __builtin_amdgcn_mbcnt_hi(
+                        (unsigned)(acc >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)acc, (unsigned)count));
+                    if (in) row_out[min(slot, cap_tot - 1)] = j;
+                    count += __popcll(acc);
                 }
-                if (in) {
-                    if (count < cap_lane) nbr[list_slot(i, count, lane, cap_lane)] = j;
-                    count++;
+                if (!last) {
+                    if (lane == 0) s_acnt[q - a0] = count;
+                    continue;
+                }
+                // per-lane counts of the G-way interleave: lane g holds entries g, g+G, ...
+                if (lane < G) cnt[(size_t)i * G + lane] = (count - lane + G - 1) / G;
+                if (lane == 0) {
+                    if (count > cap_tot) atomicMax(&s_ovf, (count + G - 1) / G);
+                    atomicMax(&s_big, count);
+                    atomicAdd(&s_tot, count);
                 }
             }
-        }
-        if (active) {
-            cnt[(size_t)i * G + lane] = count;
-            if (count > cap_lane) atomicMax(&s_ovf, count);
-        }
-        // per-atom total (lanes of one atom are adjacent in the wavefront)
-        int tot = count;
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1) tot += __shfl_xor(tot, o, 64);
-        if (active && lane == 0) {
-            atomicMax(&s_big, tot);
-            atomicAdd(&s_tot, tot);
         }
     }
     __syncthreads();
@@ -470,7 +467,7 @@ __device__ __forceinline__ void build_list_body(const BuildArgs &a, int c)
 }
 
 // List build over subcells of half the link-cell edge (used when every axis
-// has at least 3 link cells).  One workgroup per link cell (2 x 2 x 2
+// has at least 3 link cells).  parts workgroups per link cell (2 x 2 x 2
 // subcells); the 6 x 6 x 6 subcells around it are staged in LDS as float4
 // {x + sx, y + sy, z + sz, j}, grouped by subcell in x-fastest order, so that
 // for an atom the 5 subcells of each of its 25 (y, z) rows are one
@@ -496,16 +493,15 @@ __device__ __forceinline__ void build_list_body(const BuildArgs &a, int c)
 // 187 us before, 174 with the registers bounded alone, 148 now; leaving out
 // the stores changed nothing.
 constexpr int kSubSide = 6, kSubStencil = kSubSide * kSubSide * kSubSide;
-constexpr int kSubAtomChunk = 256;  // atoms of a link cell whose counts persist across staging rounds
 template <int G>
-__device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int b)
+__device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int lb)
 {
     static_assert(G == kLanesPerAtom, "list_slot assumes kLanesPerAtom lanes per atom");
     __shared__ float4 cand[kListStage + 64];
     __shared__ int s_start[kSubStencil], s_off[kSubStencil + 1];  // s_off: sizes, then their exclusive scan
     __shared__ double s_sh[3][kSubSide];
     __shared__ int s_lo[9];
-    __shared__ int s_acnt[kSubAtomChunk];
+    __shared__ int s_acnt[kListAtomChunk];
     __shared__ int s_ovf, s_big, s_tot;
     const double4 *__restrict__ pos = a.pos;
     const CellGrid &g = a.g;
@@ -515,6 +511,7 @@ __device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int b)
     int32_t *__restrict__ nbr = a.nbr;
     int32_t *__restrict__ cnt = a.cnt;
     int32_t *__restrict__ sub_of = a.sub_of;
+    const int b = lb / a.parts, part = lb - b * a.parts;
     if (b >= g.nc[0] * g.nc[1] * g.nc[2]) return;
     const int t = threadIdx.x, lane = t & 63, wid = __builtin_amdgcn_readfirstlane(t >> 6);
     constexpr int NW = kListThreads / 64;
@@ -573,8 +570,8 @@ __device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int b)
     const int hs = s_lo[0], nat = s_lo[8] - hs;
     const int cap_tot = cap_lane * G;
     const float rc2_lo = (float)(rc2 * (1.0 - 2.0e-5)), rc2_hi = (float)(rc2 * (1.0 + 2.0e-5));
-    for (int a0 = 0; a0 < nat; a0 += kSubAtomChunk) {
-        const int a1 = min(nat, a0 + kSubAtomChunk);
+    for (int a0 = 0; a0 < nat; a0 += kListAtomChunk) {
+        const int a1 = min(nat, a0 + kListAtomChunk);
         for (int r0 = 0; r0 < ncand; r0 += kListStage) {
             const int m = min(kListStage, ncand - r0);
             const bool last = r0 + m == ncand;
@@ -618,12 +615,13 @@ __device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int b)
                 __syncthreads();
             }
             // the next atom's position is loaded while this atom is processed
-            int a = a0 + wid;
-            double4 pnext = a < a1 ? pos[hs + a] : make_double4(0.0, 0.0, 0.0, 0.0);
-            for (; a < a1; a += NW) {
-                const int i = hs + a;
+            const int step = NW * a.parts;
+            int q = a0 + part * NW + wid;
+            double4 pnext = q < a1 ? pos[hs + q] : make_double4(0.0, 0.0, 0.0, 0.0);
+            for (; q < a1; q += step) {
+                const int i = hs + q;
                 const double4 pi = pnext;
-                if (a + NW < a1) pnext = pos[i + NW];
+                if (q + step < a1) pnext = pos[i + step];
                 // the atom's subcell among the link cell's 8 (s_lo is non-decreasing)
                 int l = 0;
 #pragma unroll
@@ -640,7 +638,7 @@ __device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int b)
                     rlo = min(max(s_off[qrow], r0), r0 + m) - r0;
                     rhi = min(s_off[qrow + 5], r0 + m) - r0;
                 }
-                int count = __builtin_amdgcn_readfirstlane(r0 == 0 ? 0 : s_acnt[a - a0]);
+                int count = __builtin_amdgcn_readfirstlane(r0 == 0 ? 0 : s_acnt[q - a0]);
                 int32_t *const row_out = nbr + list_slot(i, 0, 0, cap_lane);
                 // one chunk of up to 64 candidates; accepted ones are packed into the
                 // next list entries (an overflowing list is rebuilt, so entries past
@@ -721,7 +719,7 @@ __device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int b)
                     }
                 }
                 if (!last) {
-                    if (lane == 0) s_acnt[a - a0] = count;
+                    if (lane == 0) s_acnt[q - a0] = count;
                     continue;
                 }
                 // per-lane counts of the G-way interleave: lane g holds entries g, g+G, ...
@@ -786,43 +784,65 @@ __global__ void k_max_disp(const double4 *pos, const double4 *xref, int n, CellG
 // Frozen-frozen and excluded pairs leave the list, as link_cell_pairs moves
 // them past list(0,i) so that the two-body loop never sees them
 // (neighbours.F90:1198-1250: a pair of two frozen atoms, lfrzn /= 0, and
-// every j found in list_excl(:,i)).  Thread t = i*G + g compacts lane g of
-// sorted atom i in place, keeping the order of what stays; F_PAIRS (the
-// entry count) loses what was dropped.  excl_off / frz may be null.
+// every j found in list_excl(:,i)).  One wavefront per atom compacts its
+// entries in place, 64 at a time, keeping the order of what stays; F_PAIRS
+// (the entry count) loses what was dropped.  excl_off / frz may be null.  The
+// excluded atoms' places in the list order are compared with the entries, so
+// an entry costs one coalesced load: 2,592 atoms of triatomic molecules 10 us,
+// against 72 with a thread per list lane that looked up every entry's host
+// index.
 struct ExclListArgs {
     int n, cap_lane;
     int32_t *nbr, *cnt;
-    const int32_t *gid, *excl_off, *excl_ids, *frz;
+    const int32_t *gid, *slot, *excl_off, *excl_ids, *frz;
     int32_t *flags;
     const int32_t *upd;
 };
+// atoms (wavefronts) per workgroup, which subtracts what it dropped once: the
+// atomics on F_PAIRS complete one after another
+constexpr int kExclAtoms = 16, kExclThreads = 64 * kExclAtoms;
 __device__ __forceinline__ void list_exclude_body(const ExclListArgs &a, int bid)
 {
     constexpr int G = kLanesPerAtom;
-    const int t = bid * blockDim.x + threadIdx.x;
-    const int i = t / G, g = t % G;
-    int dropped = 0;
-    if (i < a.n) {
-        const int h = a.gid[i];
-        const int e0 = a.excl_off ? a.excl_off[h] : 0, e1 = a.excl_off ? a.excl_off[h + 1] : 0;
-        const bool fi = a.frz && a.frz[h] != 0;
-        if (e1 > e0 || fi) {
-            const int m = min(a.cnt[t], a.cap_lane);
-            int w = 0;
-            for (int k = 0; k < m; k++) {
-                const int32_t en = a.nbr[list_slot(i, k, g, a.cap_lane)];
-                const int hj = a.gid[list_j(en)];
-                bool ex = fi && a.frz[hj] != 0;
-                for (int e = e0; e < e1; e++) ex = ex || a.excl_ids[e] == hj;
-                if (!ex) a.nbr[list_slot(i, w++, g, a.cap_lane)] = en;
+    __shared__ int s_drop;
+    if (threadIdx.x == 0) s_drop = 0;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, i = bid * kExclAtoms + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int h = i < a.n ? a.gid[i] : 0;
+    const int e0 = a.excl_off && i < a.n ? a.excl_off[h] : 0, e1 = a.excl_off && i < a.n ? a.excl_off[h + 1] : 0;
+    const bool fi = a.frz && i < a.n && a.frz[h] != 0;
+    // entry e of the atom is list lane e % G's entry e / G
+    int m = 0;
+    if (e1 > e0 || fi)
+        for (int g = 0; g < G; g++) {
+            const int c = a.cnt[(size_t)i * G + g];
+            if (c > a.cap_lane) {  // an overflowed list is rebuilt anyway
+                m = 0;
+                break;
             }
-            dropped = m - w;
-            if (a.cnt[t] <= a.cap_lane) a.cnt[t] = w;  // an overflowed lane is rebuilt anyway
+            m += c;
         }
+    int32_t *const row = a.nbr + list_slot(i, 0, 0, a.cap_lane);
+    int w = 0;
+    for (int k0 = 0; k0 < m; k0 += 64) {
+        const bool on = k0 + lane < m;
+        const int32_t en = on ? row[k0 + lane] : 0;
+        const int j = on ? list_j(en) : i;
+        bool keep = on;
+        for (int e = e0; e < e1; e++) keep = keep && j != a.slot[a.excl_ids[e]];
+        if (fi) keep = keep && a.frz[a.gid[j]] == 0;
+        // the chunk is read before its kept entries go to or below its place
+        const unsigned long long acc = __ballot(keep);
+        if (keep)
+            row[w + __builtin_amdgcn_mbcnt_hi((unsigned)(acc >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)acc, 0u))] = en;
+        w += __popcll(acc);
     }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) dropped += __shfl_xor(dropped, o, 64);
-    if ((threadIdx.x & 63) == 0 && dropped) atomicSub(&a.flags[F_PAIRS], dropped);
+    if (w < m) {
+        if (lane < G) a.cnt[(size_t)i * G + lane] = (w - lane + G - 1) / G;
+        if (lane == 0) atomicAdd(&s_drop, m - w);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0 && s_drop) atomicSub(&a.flags[F_PAIRS], s_drop);
 }
 
 // Single-system kernels (arguments by value) and batched ones (argument
@@ -884,7 +904,7 @@ DLPX_LIST_KERNELS(k_wrap_scan, WrapArgs, (kWrapThreads), wrap_scan_body(a, block
                   wrap_scan_body(a, bp.b, bp.nb), false)
 DLPX_LIST_KERNELS(k_scatter_copy, ScatterArgs, (256), scatter_copy_body(a, blockIdx.x), scatter_copy_body(a, bp.b), false)
 DLPX_LIST_KERNELS(k_sort_permute, SortArgs, (256), sort_permute_body(a, blockIdx.x), sort_permute_body(a, bp.b), false)
-DLPX_LIST_KERNELS(k_list_exclude, ExclListArgs, (256), list_exclude_body(a, blockIdx.x), list_exclude_body(a, bp.b),
+DLPX_LIST_KERNELS(k_list_exclude, ExclListArgs, (kExclThreads), list_exclude_body(a, blockIdx.x), list_exclude_body(a, bp.b),
                   false)
 DLPX_LIST_KERNELS(k_build_list, BuildArgs, (kListThreads),
                   build_list_body<kLanesPerAtom>(a, xcd_block(blockIdx.x, gridDim.x)),
@@ -979,10 +999,10 @@ struct ListChain {
     BuildArgs build;
     ExclListArgs excl;
     bool sub, excl_on;
-    int n, ncell, nkey;
+    int n, ncell, nkey, nbuild;
 };
 
-static int list_chain(Ctx *c, const int32_t *upd, ListChain &lc)
+static int list_chain(Ctx *c, const int32_t *upd, ListChain &lc, int nsys = 1)
 {
     const int n = c->natms;
     if (c->excl_total > 0 && c->excl_natms != n)
@@ -1034,11 +1054,18 @@ static int list_chain(Ctx *c, const int32_t *upd, ListChain &lc)
     lc.sort = SortArgs{c->perm,    kstart, nkey,   n,      upd,     c->flags,
                        c->pos_alt, c->pos, c->typ_alt, c->typ, c->gid_alt, c->gid,
                        res ? c->vel_alt : nullptr, res ? c->vel : nullptr, c->slot, c->xref};
+    // several workgroups per link cell, each staging the cell's surroundings for
+    // some of its atoms, where the cells are too few to fill the GPU (with the
+    // other systems of a batch), down to an atom per wavefront; at 512 of them
+    // every CU has two.  One and several: 2,592 atoms in 27 cells 66 and 24 us,
+    // 10,296 in 120 cells 87 and 40, 4,000 in 216 cells 25 and 20.
+    const int parts = std::max(1, std::min(512 / (ncell * nsys), ceil_div(n, 8 * ncell)));
     lc.build = BuildArgs{c->pos, g, sub ? c->key_start : c->cell_start, rc_ext * rc_ext, c->cap_lane,
-                         c->nbr, c->cnt, c->flags, upd, c->sub_of};
+                         c->nbr, c->cnt, c->flags, upd, c->sub_of, parts};
+    lc.nbuild = ncell * parts;
     c->list_coded = sub;
     lc.excl_on = c->excl_total > 0 || c->nfrozen > 1;
-    lc.excl = ExclListArgs{n,      c->cap_lane, c->nbr, c->cnt, c->gid,
+    lc.excl = ExclListArgs{n,      c->cap_lane, c->nbr, c->cnt, c->gid, c->slot,
                            c->excl_total > 0 ? c->excl_off : nullptr, c->excl_ids,
                            c->nfrozen > 1 ? c->frz : nullptr, c->flags, upd};
     return 0;
@@ -1056,11 +1083,11 @@ static void launch_sort(const ListChain &lc, hipStream_t s)
 static void launch_build(const ListChain &lc, hipStream_t s)
 {
     if (lc.sub)
-        hipLaunchKernelGGL(k_build_list_sub, dim3(xcd_grid(lc.ncell)), dim3(kListThreads), 0, s, lc.build);
+        hipLaunchKernelGGL(k_build_list_sub, dim3(xcd_grid(lc.nbuild)), dim3(kListThreads), 0, s, lc.build);
     else
-        hipLaunchKernelGGL(k_build_list, dim3(xcd_grid(lc.ncell)), dim3(kListThreads), 0, s, lc.build);
+        hipLaunchKernelGGL(k_build_list, dim3(xcd_grid(lc.nbuild)), dim3(kListThreads), 0, s, lc.build);
     if (lc.excl_on)
-        hipLaunchKernelGGL(k_list_exclude, dim3(ceil_div((long)lc.n * kLanesPerAtom, 256)), dim3(256), 0, s, lc.excl);
+        hipLaunchKernelGGL(k_list_exclude, dim3(ceil_div(lc.n, kExclAtoms)), dim3(kExclThreads), 0, s, lc.excl);
 }
 
 // Bin, sort, permute and build the list from c->pos (current order); the
@@ -1138,7 +1165,7 @@ int list_prepare(const std::vector<Ctx *> &cs, ListBatch &lb)
     int r;
     for (Ctx *c : cs) {
         ListChain lc;
-        if ((r = list_chain(c, c->flags + F_UPD, lc))) return r;
+        if ((r = list_chain(c, c->flags + F_UPD, lc, (int)std::min<size_t>(cs.size(), 512)))) return r;
         if (c->cap_lane == 0 || !c->nbr) return fail(c, DLPX_ERR_STATE, "no list to rebuild on the device");
         wrap.push_back(lc.wrap);
         scat.push_back(lc.scat);
@@ -1147,9 +1174,9 @@ int list_prepare(const std::vector<Ctx *> &cs, ListBatch &lb)
         nb_wrap.push_back(ceil_div(lc.n, kWrapThreads));
         nb_atoms.push_back(ceil_div(lc.n, 256));
         nb_keys.push_back(lc.nkey);
-        nb_sub.push_back(lc.sub ? lc.ncell : 0);
-        nb_link.push_back(lc.sub ? 0 : lc.ncell);
-        nb_excl.push_back(lc.excl_on ? ceil_div((long)lc.n * kLanesPerAtom, 256) : 0);
+        nb_sub.push_back(lc.sub ? lc.nbuild : 0);
+        nb_link.push_back(lc.sub ? 0 : lc.nbuild);
+        nb_excl.push_back(lc.excl_on ? ceil_div(lc.n, kExclAtoms) : 0);
         bsub.push_back(lc.build);
         blink.push_back(lc.build);
     }
@@ -1213,7 +1240,7 @@ int list_launch(Ctx *c, hipStream_t s, const ListBatch &lb, int part)
         if (p1) {
             DLPX_LC(k_build_list_sub_cbatch, lb.bsub, BuildArgs, kListThreads, 3);
             DLPX_LC(k_build_list_cbatch, lb.blink, BuildArgs, kListThreads, 4);
-            DLPX_LC(k_list_exclude_cbatch, lb.excl, ExclListArgs, 256, 5);
+            DLPX_LC(k_list_exclude_cbatch, lb.excl, ExclListArgs, kExclThreads, 5);
         }
 #undef DLPX_LC
         DLPX_HIP(c, hipGetLastError());
@@ -1231,7 +1258,7 @@ int list_launch(Ctx *c, hipStream_t s, const ListBatch &lb, int part)
     if (p1) {
         DLPX_LB(k_build_list_sub_batch, lb.bsub, BuildArgs, kListThreads);
         DLPX_LB(k_build_list_batch, lb.blink, BuildArgs, kListThreads);
-        DLPX_LB(k_list_exclude_batch, lb.excl, ExclListArgs, 256);
+        DLPX_LB(k_list_exclude_batch, lb.excl, ExclListArgs, kExclThreads);
     }
 #undef DLPX_LB
     DLPX_HIP(c, hipGetLastError());
