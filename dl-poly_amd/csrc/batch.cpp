@@ -133,9 +133,10 @@ static int ens_prepare(Ensemble &E, bool energies, const Shape &sh)
     }
     // room for every stage's partial-sum rows before any argument struct
     // records the buffer's address (upper bounds: the z pass has at most
-    // K1 K2 workgroups, the pair kernel at most natms * 16 / 512)
+    // K1 K2 workgroups, the pair kernel at most natms * 16 / 512 or kWideGroups
+    // in a launch of few atoms)
     for (Ctx *c : cs) {
-        const int ub = std::max({ceil_div((long)c->natms * 16, 512), excl_blocks(c),
+        const int ub = std::max({ceil_div((long)c->natms * 16, 512), kWideGroups, excl_blocks(c),
                                  c->prm.electrostatics ? c->K[0] * c->K[1] : 1,
                                  c->prm.electrostatics ? ceil_div(c->natms, 16) : 1});
         if ((r = ensure_red_rows(c, ub))) return r;

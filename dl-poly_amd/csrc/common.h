@@ -507,6 +507,7 @@ void list_batch_free(ListBatch &lb);
 int pair_prepare(const std::vector<Ctx *> &cs, PairBatch &pb, int lanes, std::vector<int> &rows);
 int pair_launch(Ctx *c, hipStream_t s, const PairBatch &pb);
 int pair_blocks_exact(const Ctx *c);
+constexpr int kWideGroups = 512;  // most workgroups of a pair launch with 32 lanes to an atom
 int excl_prepare(const std::vector<Ctx *> &cs, BatchLaunch &bl);
 int excl_launch(Ctx *c, hipStream_t s, const BatchLaunch &bl);
 InflParams infl_params(const Ctx *c);

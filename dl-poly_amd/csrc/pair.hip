@@ -322,6 +322,30 @@ constexpr int kPairThreads = 512;
 // the combined-table kernel: 1024 threads, so the two workgroups its LDS rows
 // leave room for on a CU hold 8 wavefronts per SIMD
 constexpr int kCombThreads = 1024;
+constexpr int kWideLanes = 32, kWideMin = 256, kWideMax = 512;  // launches of few atoms, see wide_shape
+
+// A table from global memory into LDS by the whole workgroup, eight loads of
+// a thread in flight at a time.
+template <typename T>
+__device__ __forceinline__ void table_to_lds(T *__restrict__ dst, const T *__restrict__ src, const int n)
+{
+    constexpr int U = 8;
+    const int nt = blockDim.x;
+    int k = threadIdx.x;
+    for (; k + (U - 1) * nt < n; k += U * nt) {
+        T v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = src[k + u * nt];
+#pragma unroll
+        for (int u = 0; u < U; u++) dst[k + u * nt] = v[u];
+    }
+    T v[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) v[u] = src[min(k + u * nt, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (k + u * nt < n) dst[k + u * nt] = v[u];
+}
 
 // GP lanes serve one atom (a multiple of the list's kLanesPerAtom lanes):
 // pair lane p walks list lane p % kLanesPerAtom, entries c = p / kLanesPerAtom,
@@ -388,9 +412,9 @@ __device__ __forceinline__ void pair_body(const PairArgs<R> &a, int bid)
     if (DIRECT)
         for (int k = threadIdx.x; k < kDirectStride * pp.nkeys; k += blockDim.x) dv[k] = direct_g[k];
     else if (!GT)
-        for (int k = threadIdx.x; k < pp.nkeys * pp.mg1; k += blockDim.x) tvl[k] = vdw_g[k];
+        table_to_lds(tvl, vdw_g, pp.nkeys * pp.mg1);
     if (pp.electro)
-        for (int k = threadIdx.x; k < pp.ns1; k += blockDim.x) te[k] = erfc_g[k];
+        table_to_lds(te, erfc_g, pp.ns1);
     for (int k = threadIdx.x; k < pp.ntypes * pp.ntypes; k += blockDim.x) kt[k] = keytab_g[k];
     __syncthreads();
 
@@ -579,7 +603,7 @@ __device__ __forceinline__ void pair_comb_body(const PairArgs<float> &a, int bid
     float4 *tc = offt + (REL ? 256 : 0);
     int32_t *kt = (int32_t *)(tc + (size_t)pp.nkeys * pp.mg1);
     double *lred = (double *)(kt + ((pp.ntypes * pp.ntypes + 1) & ~1));
-    for (int k = threadIdx.x; k < pp.nkeys * pp.mg1; k += blockDim.x) tc[k] = a.comb_g[k];
+    table_to_lds(tc, a.comb_g, pp.nkeys * pp.mg1);
     for (int k = threadIdx.x; k < pp.ntypes * pp.ntypes; k += blockDim.x) kt[k] = a.comb_row_g[k];
     if (REL && threadIdx.x < 125) {
         const int k = threadIdx.x;
@@ -887,8 +911,66 @@ struct PairVariant {
     }
 };
 
+// Launches of few atoms.  Eight lanes to an atom give a small launch few
+// wavefronts and each lane a long serial walk (1,000 ions with the combined
+// tables: 8 workgroups of 1024 threads, one per 32 CUs), so up to
+// kWideGroups workgroups of 512 an atom takes 32 lanes: that many fit on the
+// 256 CUs at once, and each pays the fill of its LDS tables (77 KB in FP64)
+// only once.  Below half a workgroup per CU 256 threads spread them further.
+// Measured, 8 lanes / this: combined tables, 1,000 ions 29.9 / 10.1 us (512
+// threads 11.1), 2,592 molecules' atoms 31.4 / 12.8; FP64, 256 argon atoms
+// 11.1 / 7.9, a 4,000-atom mixture 14.5 / 11.6 (256 threads 18.9: two table
+// fills per CU); 4,000 argon atoms mixed 10.8 / 8.8.  At 10,296 ions FP64 (643
+// workgroups) the two are level, 38.0 / 37.2.
+static void wide_shape(long natms, int &lanes, int &nt)
+{
+    if (lanes != 8) return;  // asked for, or tried by the tuner
+    for (int t = kWideMin; t <= kWideMax; t *= 2)
+        if (ceil_div(natms * kWideLanes, t) <= (t == kWideMin ? kWideGroups / 2 : kWideGroups)) {
+            lanes = kWideLanes;
+            nt = t;
+            return;
+        }
+}
+
+// The kernel and launch shape of a context's pair forces in a launch of natms
+// atoms (all systems of a batch), with its dynamic LDS.
+static PairVariant pair_variant(const Ctx *c, int lanes, long natms, size_t &lds)
+{
+    const int nt = c->prm.ntypes;
+    const size_t r2 = c->prm.precision == DLPX_MIXED ? sizeof(float2) : sizeof(double2);
+    const size_t ktab = sizeof(int32_t) * ((nt * nt + 1) & ~1);
+    if (comb_ok(c)) {
+        const bool rel = c->list_coded && c->rel_pairs;
+        int threads = comb_threads(c);
+        if (threads == kCombThreads) wide_shape(natms, lanes, threads);
+        lds = (rel ? sizeof(float4) * 256 : 0) + sizeof(float4) * (size_t)(nt * (nt + 1) / 2) * (c->max_grid + 1) + ktab +
+              sizeof(double) * 10 * (kCombThreads / 64);
+        PairVariant v{lanes, false, false, false, false, true, rel};
+        v.nt = threads;
+        return v;
+    }
+    const bool direct = c->vdw_direct;
+    const size_t lds_rest = r2 * (c->prm.electrostatics ? c->nsamples + 1 : 0) + ktab +
+                            (direct ? r2 / 2 * kDirectStride * c->nrows : 0) + sizeof(double) * 10 * (kPairThreads / 64);
+    // the vdW tables go to LDS when they fit in its 160 KiB with the rest,
+    // else they are read from global memory
+    const size_t lds_tab = direct ? 0 : r2 * (size_t)c->nrows * (c->max_grid + 1);
+    const bool gtab = !direct && lds_tab + lds_rest > 160 * 1024;
+    lds = (gtab ? 0 : lds_tab) + lds_rest;
+    // per-particle output, direct mode and global tables run with 8 lanes per
+    // atom; per-particle output from LDS tables also in the few-atom shape
+    int threads = kPairThreads;
+    if (gtab || c->pp_now || direct) lanes = 8;
+    if (!gtab && !direct) wide_shape(natms, lanes, threads);
+    PairVariant v{lanes, c->vdw_force_shift, direct, c->pp_now, gtab};
+    v.nt = threads;
+    return v;
+}
+
+// natms: atoms of the whole launch (all systems of a batch).
 template <typename R>
-static int pair_setup(Ctx *c, PairArgs<R> &a, size_t &lds, PairVariant &v, int lanes)
+static int pair_setup(Ctx *c, PairArgs<R> &a, size_t &lds, PairVariant &v, int lanes, long natms)
 {
     using R2 = typename R2T<R>::type;
     PairParams &pp = a.pp;
@@ -931,53 +1013,67 @@ static int pair_setup(Ctx *c, PairArgs<R> &a, size_t &lds, PairVariant &v, int l
         a.hs[d] = (float)h;
         a.hs_lo[d] = (float)(h - (double)a.hs[d]);
     }
-    const bool direct = c->vdw_direct;
-    if (sizeof(R) == 4 && comb_ok(c)) {
-        const int nt = pp.ntypes;
-        const bool rel = c->list_coded && c->rel_pairs;
-        pp.nkeys = nt * (nt + 1) / 2;  // combined rows
-        lds = (rel ? sizeof(float4) * 256 : 0) + sizeof(float4) * (size_t)pp.nkeys * pp.mg1 +
-              sizeof(int32_t) * ((nt * nt + 1) & ~1) + sizeof(double) * 10 * (kCombThreads / 64);
-        v = PairVariant{lanes, false, false, false, false, true, rel};
-        v.nt = comb_threads(c);
-        return 0;
-    }
-    const size_t lds_rest = sizeof(R2) * (pp.electro ? pp.ns1 : 0) + sizeof(int32_t) * ((pp.ntypes * pp.ntypes + 1) & ~1) +
-                            (direct ? sizeof(R) * kDirectStride * pp.nkeys : 0) + sizeof(double) * 10 * (kPairThreads / 64);
-    // the vdW tables go to LDS when they fit in its 160 KiB with the rest,
-    // else they are read from global memory
-    const size_t lds_tab = direct ? 0 : sizeof(R2) * (size_t)pp.nkeys * pp.mg1;
-    const bool gtab = !direct && lds_tab + lds_rest > 160 * 1024;
-    lds = (gtab ? 0 : lds_tab) + lds_rest;
-    if (lds > 160 * 1024)
+    v = pair_variant(c, lanes, natms, lds);
+    if (v.comb) pp.nkeys = pp.ntypes * (pp.ntypes + 1) / 2;  // combined rows
+    else if (lds > 160 * 1024)
         return fail(c, DLPX_ERR_UNSUPPORTED, "the erfc and key tables exceed the 160 KiB LDS of a CU");
-    // per-particle output, direct mode and global tables run with 8 lanes per atom
-    v = PairVariant{(gtab || c->pp_now || direct) ? 8 : lanes, c->vdw_force_shift, direct, c->pp_now, gtab};
     return 0;
 }
 
-// Calls CALL(GP, FS, DIRECT, PP, GT) with the compile-time values of v.
+// Calls CALL(GP, NT, FS, DIRECT, PP, GT) with the compile-time values of v.
+#define DLPX_PAIR_SHAPES(v, CALL, FS, PP)                                                        \
+    do {                                                                                     \
+        if ((v).gp == kWideLanes) {                                                          \
+            if ((v).nt == kWideMin) CALL(kWideLanes, kWideMin, FS, false, PP, false);        \
+            else CALL(kWideLanes, kWideMax, FS, false, PP, false);                           \
+        } else if (PP) {                                                                     \
+            CALL(8, kPairThreads, FS, false, PP, false);                                     \
+        } else {                                                                             \
+            switch ((v).gp) {                                                                \
+                case 16: CALL(16, kPairThreads, FS, false, false, false); break;             \
+                case 8: CALL(8, kPairThreads, FS, false, false, false); break;               \
+                default: CALL(4, kPairThreads, FS, false, false, false); break;              \
+            }                                                                                \
+        }                                                                                    \
+    } while (0)
 #define DLPX_PAIR_VARIANTS(v, CALL)                                                          \
     do {                                                                                     \
         if ((v).gt) {                                                                        \
-            if ((v).pp) { if ((v).fs) CALL(8, true, false, true, true); else CALL(8, false, false, true, true); } \
-            else { if ((v).fs) CALL(8, true, false, false, true); else CALL(8, false, false, false, true); }      \
+            if ((v).pp) { if ((v).fs) CALL(8, kPairThreads, true, false, true, true); else CALL(8, kPairThreads, false, false, true, true); } \
+            else { if ((v).fs) CALL(8, kPairThreads, true, false, false, true); else CALL(8, kPairThreads, false, false, false, true); }      \
         } else if ((v).pp) {                                                                 \
-            if ((v).direct) { if ((v).fs) CALL(8, true, true, true, false); else CALL(8, false, true, true, false); } \
-            else { if ((v).fs) CALL(8, true, false, true, false); else CALL(8, false, false, true, false); }         \
+            if ((v).direct) { if ((v).fs) CALL(8, kPairThreads, true, true, true, false); else CALL(8, kPairThreads, false, true, true, false); } \
+            else { if ((v).fs) DLPX_PAIR_SHAPES(v, CALL, true, true); else DLPX_PAIR_SHAPES(v, CALL, false, true); } \
         } else if ((v).direct) {                                                             \
-            if ((v).fs) CALL(8, true, true, false, false); else CALL(8, false, true, false, false); \
+            if ((v).fs) CALL(8, kPairThreads, true, true, false, false); else CALL(8, kPairThreads, false, true, false, false); \
         } else if ((v).fs) {                                                                 \
-            switch ((v).gp) {                                                                \
-                case 16: CALL(16, true, false, false, false); break;                         \
-                case 8: CALL(8, true, false, false, false); break;                           \
-                default: CALL(4, true, false, false, false); break;                          \
-            }                                                                                \
+            DLPX_PAIR_SHAPES(v, CALL, true, false);                                                 \
         } else {                                                                             \
-            switch ((v).gp) {                                                                \
-                case 16: CALL(16, false, false, false, false); break;                        \
-                case 8: CALL(8, false, false, false, false); break;                          \
-                default: CALL(4, false, false, false, false); break;                         \
+            DLPX_PAIR_SHAPES(v, CALL, false, false);                                                \
+        }                                                                                    \
+    } while (0)
+// Calls CALL(GP, REL, NT) for the combined-table kernel's shapes.
+#define DLPX_COMB_VARIANTS(v, CALL)                                                          \
+    do {                                                                                     \
+        if ((v).gp == kWideLanes) {                                                          \
+            if ((v).nt == kWideMin) {                                                        \
+                if ((v).rel) CALL(kWideLanes, true, kWideMin);                               \
+                else CALL(kWideLanes, false, kWideMin);                                      \
+            } else {                                                                         \
+                if ((v).rel) CALL(kWideLanes, true, kWideMax);                               \
+                else CALL(kWideLanes, false, kWideMax);                                      \
+            }                                                                                \
+        } else if ((v).nt == 512) {                                                          \
+            if ((v).rel) CALL(8, true, 512);                                                 \
+            else CALL(8, false, 512);                                                        \
+        } else {                                                                             \
+            switch ((v).gp * 2 + ((v).rel ? 1 : 0)) {                                        \
+                case 33: CALL(16, true, kCombThreads); break;                                \
+                case 32: CALL(16, false, kCombThreads); break;                               \
+                case 17: CALL(8, true, kCombThreads); break;                                 \
+                case 16: CALL(8, false, kCombThreads); break;                                \
+                case 9: CALL(4, true, kCombThreads); break;                                  \
+                default: CALL(4, false, kCombThreads); break;                                \
             }                                                                                \
         }                                                                                    \
     } while (0)
@@ -989,7 +1085,7 @@ static int launch_pair(Ctx *c)
     size_t lds;
     PairVariant v;
     int r;
-    if ((r = pair_setup<R>(c, a, lds, v, c->pair_lanes))) return r;
+    if ((r = pair_setup<R>(c, a, lds, v, c->pair_lanes, c->natms))) return r;
     if constexpr (sizeof(R) == 4) {
         if (v.comb) {
             if (v.rel)
@@ -999,29 +1095,17 @@ static int launch_pair(Ctx *c)
         DLPX_LDS_MAX(c, (k_pair_comb<GP, NT, REL>));                                                          \
         hipLaunchKernelGGL((k_pair_comb<GP, NT, REL>), dim3(pair_blocks(c)), dim3(NT), lds, c->stream, a);    \
     } while (0)
-            if (v.nt == 512) {
-                if (v.rel) DLPX_PAIRC(8, true, 512);
-                else DLPX_PAIRC(8, false, 512);
-            } else {
-                switch (v.gp * 2 + (v.rel ? 1 : 0)) {
-                    case 33: DLPX_PAIRC(16, true, kCombThreads); break;
-                    case 32: DLPX_PAIRC(16, false, kCombThreads); break;
-                    case 17: DLPX_PAIRC(8, true, kCombThreads); break;
-                    case 16: DLPX_PAIRC(8, false, kCombThreads); break;
-                    case 9: DLPX_PAIRC(4, true, kCombThreads); break;
-                    default: DLPX_PAIRC(4, false, kCombThreads); break;
-                }
-            }
+            DLPX_COMB_VARIANTS(v, DLPX_PAIRC);
 #undef DLPX_PAIRC
             DLPX_HIP(c, hipGetLastError());
             return 0;
         }
     }
-#define DLPX_PAIR1(GP, FS, DIR, PPK, GTK)                                                                \
-    do {                                                                                                 \
-        DLPX_LDS_MAX(c, (k_pair<R, GP, kPairThreads, FS, DIR, PPK, GTK>));                                \
-        hipLaunchKernelGGL((k_pair<R, GP, kPairThreads, FS, DIR, PPK, GTK>), dim3(pair_blocks(c)),         \
-                           dim3(kPairThreads), lds, c->stream, a);                                       \
+#define DLPX_PAIR1(GP, NT, FS, DIR, PPK, GTK)                                                              \
+    do {                                                                                                   \
+        DLPX_LDS_MAX(c, (k_pair<R, GP, NT, FS, DIR, PPK, GTK>));                                           \
+        hipLaunchKernelGGL((k_pair<R, GP, NT, FS, DIR, PPK, GTK>), dim3(pair_blocks(c)), dim3(NT), lds,    \
+                           c->stream, a);                                                                  \
     } while (0)
     DLPX_PAIR_VARIANTS(v, DLPX_PAIR1);
 #undef DLPX_PAIR1
@@ -1045,11 +1129,13 @@ static int pair_prepare_t(const std::vector<Ctx *> &cs, PairBatch &pb, int lanes
     std::vector<std::vector<int>> nbs;
     std::vector<size_t> lds_max;
     int r;
+    long natms = 0;
+    for (Ctx *c : cs) natms += c->natms;
     for (Ctx *c : cs) {
         PairArgs<R> a;
         size_t lds;
         PairVariant v;
-        if ((r = pair_setup<R>(c, a, lds, v, lanes))) return r;
+        if ((r = pair_setup<R>(c, a, lds, v, lanes, natms))) return r;
         size_t g = 0;
         while (g < vs.size() && !(vs[g] == v)) g++;
         if (g == vs.size()) {
@@ -1085,7 +1171,7 @@ static int pair_prepare_t(const std::vector<Ctx *> &cs, PairBatch &pb, int lanes
         PairArgs<R> a;
         size_t lds;
         PairVariant v;
-        if ((r = pair_setup<R>(c, a, lds, v, lanes))) return r;
+        if ((r = pair_setup<R>(c, a, lds, v, lanes, natms))) return r;
         pa.push_back(prel_args(c));
         pnb.push_back(v.rel ? ceil_div(c->natms, 256) : 0);
     }
@@ -1117,28 +1203,16 @@ static int pair_launch_t(Ctx *c, hipStream_t s, const PairBatch &pb)
         hipLaunchKernelGGL((k_pair_comb_batch<GP, NT, REL>), dim3(gr.bl.total), dim3(NT), lds, s,                  \
                            (const PairArgs<float> *)gr.bl.args, gr.bl.boff, gr.bl.nsys);                          \
     } while (0)
-                if (v.nt == 512) {
-                    if (v.rel) DLPX_PAIRCB(8, true, 512);
-                    else DLPX_PAIRCB(8, false, 512);
-                } else {
-                    switch (v.gp * 2 + (v.rel ? 1 : 0)) {
-                        case 33: DLPX_PAIRCB(16, true, kCombThreads); break;
-                        case 32: DLPX_PAIRCB(16, false, kCombThreads); break;
-                        case 17: DLPX_PAIRCB(8, true, kCombThreads); break;
-                        case 16: DLPX_PAIRCB(8, false, kCombThreads); break;
-                        case 9: DLPX_PAIRCB(4, true, kCombThreads); break;
-                        default: DLPX_PAIRCB(4, false, kCombThreads); break;
-                    }
-                }
+                DLPX_COMB_VARIANTS(v, DLPX_PAIRCB);
 #undef DLPX_PAIRCB
                 continue;
             }
         }
-#define DLPX_PAIRB(GP, FS, DIR, PPK, GTK)                                                                   \
+#define DLPX_PAIRB(GP, NT, FS, DIR, PPK, GTK)                                                                   \
     do {                                                                                                    \
-        DLPX_LDS_MAX(c, (k_pair_batch<R, GP, kPairThreads, FS, DIR, PPK, GTK>));                             \
-        hipLaunchKernelGGL((k_pair_batch<R, GP, kPairThreads, FS, DIR, PPK, GTK>), dim3(gr.bl.total),         \
-                           dim3(kPairThreads), lds, s, (const PairArgs<R> *)gr.bl.args, gr.bl.boff,           \
+        DLPX_LDS_MAX(c, (k_pair_batch<R, GP, NT, FS, DIR, PPK, GTK>));                             \
+        hipLaunchKernelGGL((k_pair_batch<R, GP, NT, FS, DIR, PPK, GTK>), dim3(gr.bl.total),         \
+                           dim3(NT), lds, s, (const PairArgs<R> *)gr.bl.args, gr.bl.boff,           \
                            gr.bl.nsys);                                                                     \
     } while (0)
         DLPX_PAIR_VARIANTS(v, DLPX_PAIRB);
@@ -1156,7 +1230,9 @@ int pair_launch(Ctx *c, hipStream_t s, const PairBatch &pb)
 
 int pair_blocks_exact(const Ctx *c)
 {
-    return ceil_div((long)c->natms * c->pair_lanes, comb_ok(c) ? comb_threads(c) : kPairThreads);
+    size_t lds;
+    const PairVariant v = pair_variant(c, c->pair_lanes, c->natms, lds);
+    return ceil_div((long)c->natms * v.gp, v.nt);
 }
 int pair_blocks(const Ctx *c) { return xcd_grid(pair_blocks_exact(c)); }
 

@@ -989,3 +989,35 @@ def test_tile_lists_longer_than_their_room(monkeypatch):
         # the close ions' real-space forces dominate; the reciprocal energy shows the spreading
         assert rms_rel(a["frc"], b["frc"]) <= 1e-12
         assert abs(a["buffer"][9] - b["buffer"][9]) <= 1e-12 * abs(b["buffer"][9])
+
+
+# atom counts on both sides of the lines between the launch shapes (4,096 and
+# 8,192 atoms), a lone pair of atoms and an odd count
+@pytest.mark.parametrize("kind,size", [("argon", 2), ("argon", 777), ("argon", 4096), ("argon", 4097),
+                                       ("argon", 8192), ("argon", 8193), ("nacl", (5, 5, 5)), ("nacl", (8, 8, 8)),
+                                       ("nacl", (8, 8, 9)), ("nacl", (8, 8, 16)), ("nacl", (8, 8, 17))])
+def test_pair_launch_shapes_agree(kind, size, monkeypatch):
+    """The pair kernels' default launch shape and four lanes to an atom
+    (DLPX_PAIR_LANES=4): the same pairs with the same arithmetic, summed in
+    another order.  FP64 to 1e-12; mixed results of either shape to the mode's
+    bar (forces 1e-5 RMS, energies 1e-6) against FP64's."""
+    if kind == "argon":
+        s = systems.argon(ncells=13, jitter=0.2)
+        s.pos, s.vel, s.types = s.pos[:size].copy(), s.vel[:size].copy(), s.types[:size].copy()
+    else:
+        s = systems.nacl(ncells=size, kvec=(32, 32, 32), seed=14)
+    ref = None
+    for precision, tol, etol in ((lib.FP64, 1e-12, 1e-12), (lib.MIXED, 1e-5, 1e-6)):
+        for lanes in ("4", None):
+            if lanes:
+                monkeypatch.setenv("DLPX_PAIR_LANES", lanes)
+            else:
+                monkeypatch.delenv("DLPX_PAIR_LANES", raising=False)
+            ctx = lib.Context(s, precision=precision)
+            ctx.link_cell_pairs(s.pos)
+            r = ctx.two_body_forces(s.pos)
+            ctx.close()
+            ref = ref or r
+            print("case", kind, size, precision, lanes, rms_rel(r["frc"], ref["frc"]), flush=True)
+            assert rms_rel(r["frc"], ref["frc"]) <= tol
+            assert abs(r["engsrp"] - ref["engsrp"]) <= etol * abs(ref["engsrp"])
