@@ -12,12 +12,13 @@
 
 namespace dlpx {
 
-int load_atoms(Ctx *c, const double *st_dev, const int32_t *st_t_dev, bool identity, bool with_vel);
+int load_atoms(Ctx *c, bool identity, bool with_vel, bool disp);
+int load_blocks(const Ctx *c);
 struct Ensemble;
 uint64_t next_serial();
 void ensemble_free(void *e);
 int ensemble_run(const std::vector<Ctx *> &cs, Ensemble *&E, int nsteps, bool energies, std::vector<int> &rebuilds);
-int store_atoms(Ctx *c, double *st_dev, bool with_pos, bool with_vel);
+int store_atoms(Ctx *c, bool with_state, bool finish);
 int spme_finish(Ctx *c, double two_scale);
 
 int fail(Ctx *c, int code, const std::string &msg)
@@ -160,9 +161,10 @@ int upload_tables(Ctx *c)
     return c->noalloc_now ? 0 : upload_comb(c);
 }
 
-// host arrays (strided) -> pinned staging -> device staging -> cell order
+// host arrays (strided) -> pinned staging -> cell order.  With disp the
+// displacements since the list build go to h_disp.
 static int upload(Ctx *c, const dlpx_atoms *a, bool identity, const double *vx, const double *vy, const double *vz,
-                  const double *mass, int vstride = 0)
+                  const double *mass, int vstride = 0, bool disp = false)
 {
     if (!a || !a->x || !a->y || !a->z || !a->chge || !a->ltype) return fail(c, DLPX_ERR_BAD_ARG, "atom arrays");
     if (a->natms <= 0 || a->natms > c->cap) return fail(c, DLPX_ERR_BAD_ARG, "natms outside 1..natms_max");
@@ -170,12 +172,18 @@ static int upload(Ctx *c, const dlpx_atoms *a, bool identity, const double *vx, 
     const int n = a->natms, st = a->stride, vst = vstride > 0 ? vstride : a->stride;
     auto at = [st](const double *p, int i) { return *(const double *)((const char *)p + (size_t)st * i); };
     auto atv = [vst](const double *p, int i) { return *(const double *)((const char *)p + (size_t)vst * i); };
+    const int row = vx ? 8 : 4;
+    // charge per atom type, for the pair kernel's combined-table path
+    std::vector<double> tq(c->prm.ntypes, 0.0);
+    std::vector<char> seen(c->prm.ntypes, 0);
+    bool per_type = true;
     for (int i = 0; i < n; i++) {
-        double *r = c->h_st + (size_t)8 * i;
+        double *r = c->h_st + (size_t)row * i;
+        const double q = at(a->chge, i);
         r[0] = at(a->x, i);
         r[1] = at(a->y, i);
         r[2] = at(a->z, i);
-        r[3] = at(a->chge, i);
+        r[3] = q;
         if (vx) {
             r[4] = atv(vx, i);
             r[5] = atv(vy, i);
@@ -185,30 +193,20 @@ static int upload(Ctx *c, const dlpx_atoms *a, bool identity, const double *vx, 
         const int t = a->ltype[i];
         if (t < 1 || t > c->prm.ntypes) return fail(c, DLPX_ERR_BAD_ARG, "ltype outside 1..ntypes");
         c->h_t[i] = t;
+        if (!seen[t - 1]) {
+            if (per_type) {
+                seen[t - 1] = 1;
+                tq[t - 1] = q;
+            }
+        } else if (q != tq[t - 1]) {
+            per_type = false;
+        }
     }
     c->natms = n;
-    {
-        // charge per atom type, for the pair kernel's combined-table path
-        std::vector<double> tq(c->prm.ntypes, 0.0);
-        std::vector<char> seen(c->prm.ntypes, 0);
-        bool per_type = true;
-        for (int i = 0; i < n && per_type; i++) {
-            const int t = c->h_t[i] - 1;
-            const double q = c->h_st[(size_t)8 * i + 3];
-            if (!seen[t]) {
-                seen[t] = 1;
-                tq[t] = q;
-            } else if (q != tq[t]) {
-                per_type = false;
-            }
-        }
-        if (per_type != c->q_per_type || (per_type && tq != c->type_q)) c->comb_dirty = true;
-        c->q_per_type = per_type;
-        c->type_q = tq;
-    }
-    DLPX_HIP(c, hipMemcpyAsync(c->stage, c->h_st, sizeof(double) * 8 * n, hipMemcpyHostToDevice, c->stream));
-    DLPX_HIP(c, hipMemcpyAsync(c->stage_i, c->h_t, sizeof(int32_t) * n, hipMemcpyHostToDevice, c->stream));
-    return load_atoms(c, c->stage, c->stage_i, identity, vx != nullptr);
+    if (per_type != c->q_per_type || (per_type && tq != c->type_q)) c->comb_dirty = true;
+    c->q_per_type = per_type;
+    c->type_q = tq;
+    return load_atoms(c, identity, vx != nullptr, disp);
 }
 
 static void charges_summary(Ctx *c, const dlpx_atoms *a)
@@ -232,9 +230,10 @@ double recip_scale(const Ctx *c)
 }
 
 // pair + SPME forces into c->frc (cell order); partial sums reduced to
-// red_out.  With defer_finish the reciprocal forces are left in frc_recip for
-// the velocity stage to add (nve_second), saving a pass over the atoms.
-static int evaluate(Ctx *c, bool defer_finish = false)
+// red_out, and to the host's h_red with fetch.  With defer_finish the
+// reciprocal forces are left in frc_recip for the velocity stage (nve_second)
+// or the copy to the host (store_forces) to add, saving a pass over the atoms.
+static int evaluate(Ctx *c, bool defer_finish = false, bool fetch = false)
 {
     int r;
     if ((r = upload_tables(c))) return r;
@@ -274,7 +273,7 @@ static int evaluate(Ctx *c, bool defer_finish = false)
     for (int k = R_ENGVDW; k <= R_S33; k++) c->red_rows[k] = pair_blocks(c);
     if (c->excl_total > 0 && c->prm.electrostatics)
         for (int k = R_ENGEX; k <= R_XS33; k++) c->red_rows[k] = excl_blocks(c);
-    if ((r = reduce_partials(c))) return r;
+    if ((r = reduce_partials(c, fetch ? c->h_red_dev : nullptr))) return r;
     c->finish_in_vv2 = false;
     if (c->prm.electrostatics) {
         if (defer_finish)
@@ -364,11 +363,30 @@ static void assemble(Ctx *c, const double *red, dlpx_two_body_out *o)
     std::memcpy(o->stress, st, sizeof(st));
 }
 
+// Wait for an evaluation with fetch: h_red holds its sums.
 static int fetch_red(Ctx *c)
 {
-    DLPX_HIP(c, hipMemcpyAsync(c->h_red, c->red_out, sizeof(double) * kReduceSlots, hipMemcpyDeviceToHost, c->stream));
     DLPX_HIP(c, hipStreamSynchronize(c->stream));
     return collect_timing(c);
+}
+
+// The forces of an evaluation with defer_finish and fetch, added to the
+// host's arrays.
+static int store_forces(Ctx *c, const dlpx_atoms *a)
+{
+    int r;
+    const bool finish = c->finish_in_vv2;
+    c->finish_in_vv2 = false;
+    if ((r = store_atoms(c, false, finish))) return r;
+    if ((r = fetch_red(c))) return r;
+    const int st = a->stride;
+    for (int i = 0; i < c->natms; i++) {
+        const double *f = c->h_st + (size_t)3 * i;
+        *(double *)((char *)a->fx + (size_t)st * i) += f[0];
+        *(double *)((char *)a->fy + (size_t)st * i) += f[1];
+        *(double *)((char *)a->fz + (size_t)st * i) += f[2];
+    }
+    return 0;
 }
 
 // What a captured step graph bakes in (buffers, sizes, launch shapes, the
@@ -554,7 +572,7 @@ int dlpx_create(const dlpx_params *p, dlpx_ctx **out)
         (r = dalloc(c, &c->vel_alt, n)) || (r = dalloc(c, &c->frc, n)) || (r = dalloc(c, &c->frc_recip, n)) ||
         (r = dalloc(c, &c->xref, n)) || (r = dalloc(c, &c->typ, n)) || (r = dalloc(c, &c->typ_alt, n)) ||
         (r = dalloc(c, &c->gid, n)) || (r = dalloc(c, &c->gid_alt, n)) || (r = dalloc(c, &c->slot, n)) ||
-        (r = dalloc(c, &c->stage, 9 * n)) || (r = dalloc(c, &c->stage_i, n)) || (r = dalloc(c, &c->cell_of, n)) ||
+        (r = dalloc(c, &c->cell_of, n)) ||
         (r = dalloc(c, &c->perm, n)) || (r = dalloc(c, &c->cnt, n * kLanesPerAtom)) || (r = dalloc(c, &c->flags, F_WORDS)) ||
         (r = dalloc(c, &c->red_out, kReduceSlots)) || (r = dalloc(c, &c->acc, 4 * kAccSlots)) ||
         (r = dalloc(c, &c->step_part, 2 * kStepBlocks)) ||
@@ -565,13 +583,15 @@ int dlpx_create(const dlpx_params *p, dlpx_ctx **out)
     if (dev_zero(c->stream, c->flags, sizeof(int32_t) * F_WORDS) != hipSuccess) return bail(DLPX_ERR_HIP);
     c->serial = next_serial();
     // host words the GPU writes directly (the displacement maximum of each step)
-    if (hipHostMalloc((void **)&c->h_flags, 64, hipHostMallocMapped) != hipSuccess) return bail(DLPX_ERR_HIP);
-    if (hipHostGetDevicePointer((void **)&c->h_flags_dev, c->h_flags, 0) != hipSuccess) return bail(DLPX_ERR_HIP);
-    if (hipHostMalloc((void **)&c->h_red, sizeof(double) * kReduceSlots, hipHostMallocDefault) != hipSuccess)
-        return bail(DLPX_ERR_HIP);
-    if (hipHostMalloc((void **)&c->h_st, sizeof(double) * 9 * n, hipHostMallocDefault) != hipSuccess)
-        return bail(DLPX_ERR_HIP);
-    if (hipHostMalloc((void **)&c->h_t, sizeof(int32_t) * n, hipHostMallocDefault) != hipSuccess)
+    // the second half of h_flags: a copy of the device words
+    auto pinned = [](auto **host, auto **dev, size_t bytes) {
+        return hipHostMalloc((void **)host, bytes, hipHostMallocMapped) == hipSuccess &&
+               hipHostGetDevicePointer((void **)dev, *host, 0) == hipSuccess;
+    };
+    if (!pinned(&c->h_flags, &c->h_flags_dev, sizeof(int32_t) * 2 * F_WORDS) ||
+        !pinned(&c->h_red, &c->h_red_dev, sizeof(double) * kReduceSlots) ||
+        !pinned(&c->h_st, &c->h_st_dev, sizeof(double) * 9 * n) || !pinned(&c->h_t, &c->h_t_dev, sizeof(int32_t) * n) ||
+        !pinned(&c->h_disp, &c->h_disp_dev, sizeof(double) * (n / 64 + 1)))
         return bail(DLPX_ERR_HIP);
     if (p->electrostatics && (r = spme_setup(c))) return bail(r);
     if ((r = scratch_address(c))) return bail(r);
@@ -588,7 +608,7 @@ int dlpx_destroy(dlpx_ctx *ctx)
     if (c->ens) ensemble_free(c->ens);
     if (c->ens_multi) ensemble_free(c->ens_multi);
     void *dev[] = {c->pos, c->pos_alt, c->vel, c->vel_alt, c->frc, c->frc_recip, c->xref, c->typ, c->typ_alt,
-                   c->gid, c->gid_alt, c->slot, c->stage, c->stage_i, c->cell_of, c->perm, c->cell_count,
+                   c->gid, c->gid_alt, c->slot, c->cell_of, c->perm, c->cell_count,
                    c->cell_start, c->cell_fill, c->key_start, c->nbr, c->cnt, c->flags, c->d_vdw, c->d_erfc, c->d_keytab,
                    c->d_vdw_direct, c->d_comb, c->d_comb_row, c->sub_of, c->prel, c->excl_off, c->excl_ids, c->frz, c->pp, c->Q2,
                    c->Q, c->spl_z, c->spl_wq, c->spl_base, c->tile_list, c->Phi, c->H, c->theta, c->tw, c->bsp_n2, c->red, c->red_out, c->acc, c->step_part, c->energies_dev,
@@ -597,6 +617,7 @@ int dlpx_destroy(dlpx_ctx *ctx)
         if (p) (void)hipFree(p);
     if (c->h_st) (void)hipHostFree(c->h_st);
     if (c->h_t) (void)hipHostFree(c->h_t);
+    if (c->h_disp) (void)hipHostFree(c->h_disp);
     if (c->h_flags) (void)hipHostFree(c->h_flags);
     if (c->h_red) (void)hipHostFree(c->h_red);
     for (int k = 0; k < 8; k++)
@@ -938,10 +959,14 @@ int dlpx_vnl_check(dlpx_ctx *ctx, const dlpx_atoms *atoms, int32_t *update)
         return 0;
     }
     int r;
-    if ((r = upload(c, atoms, false, nullptr, nullptr, nullptr, nullptr))) return r;
-    int u = 0;
-    if ((r = vnl_check_dev(c, &u))) return r;
-    *update = u;
+    if ((r = upload(c, atoms, false, nullptr, nullptr, nullptr, nullptr, 0, true))) return r;
+    DLPX_HIP(c, hipStreamSynchronize(c->stream));
+    // the largest of the workgroups' maxima, as bit patterns
+    uint64_t b = 0;
+    for (int k = 0; k < load_blocks(c); k++) b = std::max(b, bits(c->h_disp[k]));
+    double r2;
+    memcpy(&r2, &b, sizeof(r2));
+    *update = std::sqrt(r2) >= kHalfMinus * c->prm.padding ? 1 : 0;
     return 0;
 }
 
@@ -971,21 +996,11 @@ int dlpx_two_body_forces(dlpx_ctx *ctx, const double cell[9], const dlpx_atoms *
         }
         c->pp_now = true;
     }
-    r = evaluate(c);
+    r = evaluate(c, !c->timing, true);
     c->pp_now = false;
     if (r) return r;
     c->pp_valid = c->per_particle;
-    if ((r = store_atoms(c, c->stage, false, false))) return r;
-    const int n = c->natms;
-    DLPX_HIP(c, hipMemcpyAsync(c->h_st, c->stage, sizeof(double) * 9 * n, hipMemcpyDeviceToHost, c->stream));
-    if ((r = fetch_red(c))) return r;
-    const int st = atoms->stride;
-    for (int i = 0; i < n; i++) {
-        const double *f = c->h_st + (size_t)9 * i + 6;
-        *(double *)((char *)atoms->fx + (size_t)st * i) += f[0];
-        *(double *)((char *)atoms->fy + (size_t)st * i) += f[1];
-        *(double *)((char *)atoms->fz + (size_t)st * i) += f[2];
-    }
+    if ((r = store_forces(c, atoms))) return r;
     assemble(c, c->h_red, out);
     return 0;
 }
@@ -1023,28 +1038,15 @@ int dlpx_two_body_forces_noalloc(dlpx_ctx *ctx, const double cell[9], const dlpx
     c->red_cap = kScratchRows;
     c->red_out = scr + (size_t)kScratchRows * kReduceSlots;
     c->noalloc_now = true;  // no table upload: stale combined rows fall back to the two-table pair path
-    r = evaluate(c);
+    r = evaluate(c, !c->timing, true);
     c->noalloc_now = false;
-    if (!r) r = store_atoms(c, c->stage, false, false);
-    if (!r) {
-        const hipError_t e = hipMemcpyAsync(c->h_st, c->stage, sizeof(double) * 9 * c->natms,
-                                            hipMemcpyDeviceToHost, c->stream);
-        r = e != hipSuccess ? fail(c, DLPX_ERR_HIP + (int)e, std::string("hipMemcpyAsync: ") + hipGetErrorString(e))
-                            : fetch_red(c);  // waits for the stream: the scratch is free again on return
-    }
+    if (!r) r = store_forces(c, atoms);  // waits for the stream: the scratch is free again on return
     c->red = red;
     c->red_cap = red_cap;
     c->red_out = red_out;
     if (r) {
         (void)hipStreamSynchronize(c->stream);
         return r;
-    }
-    const int st = atoms->stride;
-    for (int i = 0; i < c->natms; i++) {
-        const double *f = c->h_st + (size_t)9 * i + 6;
-        *(double *)((char *)atoms->fx + (size_t)st * i) += f[0];
-        *(double *)((char *)atoms->fy + (size_t)st * i) += f[1];
-        *(double *)((char *)atoms->fz + (size_t)st * i) += f[2];
     }
     assemble(c, c->h_red, out);
     return 0;
@@ -1063,7 +1065,7 @@ int dlpx_md_load(dlpx_ctx *ctx, const double cell[9], const dlpx_atoms *atoms, c
     charges_summary(c, atoms);
     if ((r = build_list(c))) return r;
     // forces at the starting configuration (md_vv computes them before step 1)
-    if ((r = evaluate(c))) return r;
+    if ((r = evaluate(c, false, true))) return r;
     if ((r = freeze_atoms(c))) return r;
     if ((r = fetch_red(c))) return r;
     // the starting configuration's output, until a run with energies replaces it
@@ -1205,9 +1207,8 @@ int dlpx_md_store(dlpx_ctx *ctx, double *x, double *y, double *z, double *vx, do
     if (!c || stride < 0 || vstride < 0) return DLPX_ERR_BAD_ARG;
     if (!c->resident) return fail(c, DLPX_ERR_STATE, "call dlpx_md_load first");
     int r;
-    if ((r = store_atoms(c, c->stage, true, true))) return r;
+    if ((r = store_atoms(c, true, false))) return r;
     const int n = c->natms;
-    DLPX_HIP(c, hipMemcpyAsync(c->h_st, c->stage, sizeof(double) * 9 * n, hipMemcpyDeviceToHost, c->stream));
     DLPX_HIP(c, hipStreamSynchronize(c->stream));
     double *dst[9] = {x, y, z, vx, vy, vz, fx, fy, fz};
     for (int k = 0; k < 9; k++) {

@@ -227,10 +227,12 @@ struct Ctx {
     int32_t *typ = nullptr, *typ_alt = nullptr;      // 0-based type
     int32_t *gid = nullptr, *gid_alt = nullptr;      // sorted -> host index
     int32_t *slot = nullptr;                         // host index -> sorted
-    double *stage = nullptr;                         // host-order staging, 9 doubles per atom
-    int32_t *stage_i = nullptr;                      // host-order int staging
-    double *h_st = nullptr;                          // pinned host staging, 9 doubles per atom
-    int32_t *h_t = nullptr;                          // pinned host staging, 1 int per atom
+    // pinned host staging in host order, which the kernels read and write
+    // directly (_dev: its device address): atoms in and out (9 doubles per atom),
+    // types, the displacement of each workgroup's atoms
+    double *h_st = nullptr, *h_st_dev = nullptr;
+    int32_t *h_t = nullptr, *h_t_dev = nullptr;
+    double *h_disp = nullptr, *h_disp_dev = nullptr;
     int32_t *cell_of = nullptr, *perm = nullptr;
 
     // link cells
@@ -307,7 +309,8 @@ struct Ctx {
     double *red_out = nullptr;       // kReduceSlots totals (device)
     double *acc = nullptr;           // kAccSlots x 4 atomic totals of the gather (batched runs), zero between steps
     double *step_part = nullptr;     // kStepBlocks x 2 workgroup partials of the step kernel
-    double *h_red = nullptr;         // pinned mirror of red_out
+    double *h_red = nullptr;         // pinned mirror of red_out, written by the reduction
+    double *h_red_dev = nullptr;     // its device address
     double *energies_dev = nullptr;  // per-step energies (resident runs)
     int energies_cap = 0;
     dlpx_two_body_out last_out{};    // the last step of the last resident run with energies
@@ -460,7 +463,6 @@ void vdw_lrc(int ntypes, const double *num_type, const int *kinds, const double 
 int upload_tables(Ctx *c);
 int upload_comb(Ctx *c);                     // the combined rows when the conditions hold (pair.hip)
 int build_list(Ctx *c);                      // from c->pos (current order), sorts & permutes
-int vnl_check_dev(Ctx *c, int *update);
 int count_pairs_dev(Ctx *c, double r, int64_t *npairs);
 int pair_forces(Ctx *c);                     // writes c->frc and reduction slots
 int excl_forces(Ctx *c);                     // adds the exclusion correction into c->frc
@@ -470,7 +472,7 @@ int spme_setup(Ctx *c);
 bool spread_by_tiles(const Ctx *c);          // the context's charges are spread by mesh tiles
 int tile_room(Ctx *c);                       // after a list build: that choice, and the tiles' room
 int ensure_red_rows(Ctx *c, int rows);
-int reduce_partials(Ctx *c);                 // red -> red_out (device)
+int reduce_partials(Ctx *c, double *rec = nullptr);  // red -> red_out (device), and rec
 int pair_blocks(const Ctx *c);
 int gather_blocks(const Ctx *c);
 int nve_first(Ctx *c, double dt);            // also the vnl_check displacement (flags[4..6])

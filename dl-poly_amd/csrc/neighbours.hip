@@ -117,6 +117,7 @@ struct WrapArgs {
     int32_t *cell_start;     // subcells: link-cell starts; else null (start is them)
     unsigned int *done;      // workgroups finished (zero between builds)
     const int32_t *upd;
+    int32_t *clear;          // the four list words, zeroed for a host-decided build; else null
 };
 __device__ __forceinline__ void wrap_scan_body(const WrapArgs &a, int bid, int nb)
 {
@@ -153,6 +154,7 @@ __device__ __forceinline__ void wrap_scan_body(const WrapArgs &a, int bid, int n
     if (!last) return;
     scan_keys(a.count, a.start, a.fill, a.nkey, a.cell_start);
     if (threadIdx.x == 0) __hip_atomic_store(a.done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (a.clear && threadIdx.x < 4) a.clear[threadIdx.x] = 0;  // F_OVF .. F_PAIRS
 }
 
 struct ScatterArgs {
@@ -762,25 +764,6 @@ __global__ void __launch_bounds__(256) k_count_pairs(const double4 *__restrict__
     if ((threadIdx.x & 63) == 0 && k) atomicAdd(out, k);
 }
 
-// vnl_check (neighbours.F90:150-178): largest minimum-image displacement since
-// the list was built, as the bit pattern of a non-negative double.
-__global__ void k_max_disp(const double4 *pos, const double4 *xref, int n, CellGrid g,
-                           unsigned long long *out)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    double r2 = 0.0;
-    if (i < n) {
-        const double4 p = pos[i], q = xref[i];
-        const double dx = min_image_1(p.x, q.x, g.L[0], g.invL[0]);
-        const double dy = min_image_1(p.y, q.y, g.L[1], g.invL[1]);
-        const double dz = min_image_1(p.z, q.z, g.L[2], g.invL[2]);
-        r2 = dx * dx + dy * dy + dz * dz;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, (unsigned long long)__double_as_longlong(r2));
-}
-
 // Frozen-frozen and excluded pairs leave the list, as link_cell_pairs moves
 // them past list(0,i) so that the two-body loop never sees them
 // (neighbours.F90:1198-1250: a pair of two frozen atoms, lfrzn /= 0, and
@@ -1047,7 +1030,8 @@ static int list_chain(Ctx *c, const int32_t *upd, ListChain &lc, int nsys = 1)
     lc.sub = sub;
     const bool res = c->resident;
     lc.wrap = WrapArgs{c->pos,    n,     g, c->cell_of, c->cell_count, kstart, c->cell_fill, nkey,
-                       sub ? c->cell_start : nullptr, (unsigned int *)(c->flags + F_WDONE), upd};
+                       sub ? c->cell_start : nullptr, (unsigned int *)(c->flags + F_WDONE), upd,
+                       upd ? nullptr : c->flags};
     lc.scat = ScatterArgs{c->cell_of, c->cell_fill, c->perm,    n,          upd,
                           c->flags,   c->pos,       c->pos_alt, c->typ,     c->typ_alt,
                           c->gid,     c->gid_alt,   res ? c->vel : nullptr, res ? c->vel_alt : nullptr};
@@ -1113,14 +1097,15 @@ int build_list(Ctx *c)
         }
         lc.build.cap_lane = lc.excl.cap_lane = c->cap_lane;
         lc.build.nbr = lc.excl.nbr = c->nbr;
-        DLPX_HIP(c, hipMemsetAsync(c->flags, 0, sizeof(int32_t) * 4, s));
+        if (attempt > 0) DLPX_HIP(c, hipMemsetAsync(c->flags, 0, sizeof(int32_t) * 4, s));
         if (c->timing) DLPX_HIP(c, hipEventRecord(c->ev[6], s));
         launch_build(lc, s);
         if (c->timing) DLPX_HIP(c, hipEventRecord(c->ev[7], s));
-        DLPX_HIP(c, hipMemcpyAsync(c->h_flags, c->flags, sizeof(int32_t) * 4, hipMemcpyDeviceToHost, s));
-        DLPX_HIP(c, hipMemcpyAsync(c->h_flags + 10, c->flags + F_ERR, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        int32_t *const all = c->h_flags + F_WORDS;  // every word in one copy
+        DLPX_HIP(c, hipMemcpyAsync(all, c->flags, sizeof(int32_t) * F_WORDS, hipMemcpyDeviceToHost, s));
         DLPX_HIP(c, hipStreamSynchronize(s));
-        if (c->h_flags[10] != 0) {
+        std::memcpy(c->h_flags, all, sizeof(int32_t) * 4);
+        if (all[F_ERR] != 0) {
             c->have_list = false;
             return fail(c, DLPX_ERR_STATE, "internal error: the list build met an atom index out of range");
         }
@@ -1273,24 +1258,6 @@ void list_batch_free(ListBatch &lb)
     lb.plan = lb.plan_nb = nullptr;
     lb.plan_gates = nullptr;
     lb.gate = nullptr;
-}
-
-int vnl_check_dev(Ctx *c, int *update)
-{
-    const int n = c->natms;
-    hipStream_t s = c->stream;
-    unsigned long long *d = (unsigned long long *)(c->flags + 4);
-    DLPX_HIP(c, hipMemsetAsync(d, 0, sizeof(unsigned long long), s));
-    hipLaunchKernelGGL(k_max_disp, dim3(ceil_div(n, 256)), dim3(256), 0, s, c->pos, c->xref, n, make_grid(c), d);
-    DLPX_HIP(c, hipMemcpyAsync(c->h_flags + 4, d, sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
-    DLPX_HIP(c, hipStreamSynchronize(s));
-    unsigned long long bits;
-    memcpy(&bits, c->h_flags + 4, sizeof(bits));
-    double r2;
-    memcpy(&r2, &bits, sizeof(r2));
-    const double tol = sqrt(r2);
-    *update = (tol >= kHalfMinus * c->prm.padding) ? 1 : 0;
-    return 0;
 }
 
 int count_pairs_dev(Ctx *c, double r, int64_t *npairs)

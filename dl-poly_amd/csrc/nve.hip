@@ -181,44 +181,111 @@ __device__ __forceinline__ bool strayed(const StrayArgs &a, const double (&x)[3]
     return out;
 }
 
-// host-order staging (8 doubles per atom: x y z q vx vy vz m) -> cell order
-__global__ void k_load(const double *__restrict__ st, const int32_t *__restrict__ st_t, int n, int cap,
-                       const int32_t *__restrict__ slot, bool identity, bool with_vel, double4 *pos, int32_t *typ,
-                       int32_t *gid, double4 *vel, StrayArgs sa)
+// Host order -> cell order, from pinned host memory (4 doubles per atom, x y z
+// q, or 8 with vx vy vz m; and its type from 1).  disp, when not null, gets
+// the largest minimum-image displacement squared since the list build of each
+// workgroup's atoms, as the bit pattern of a non-negative double (vnl_check,
+// neighbours.F90:150-178).
+//
+// Bound by the host link (36 B an atom without velocities), and in a small
+// system by the number of operations: the kernel reads the host's rows and
+// writes the displacements to the host itself, one launch where copies to
+// staging, a load, a clear, a displacement kernel and a copy back were six.
+// LOAD_FIGURES
+struct LoadArgs {
+    const double *st;
+    const int32_t *st_t;
+    int n, row;
+    const int32_t *slot;  // null: the order as given
+    double4 *pos, *vel;
+    int32_t *typ, *gid;
+    unsigned long long *disp;
+    Box b;
+    StrayArgs stray;
+};
+constexpr int kLoadThreads = 256;
+__global__ void __launch_bounds__(kLoadThreads) k_load(LoadArgs a)
 {
-    const int h = blockIdx.x * blockDim.x + threadIdx.x;
-    if (h >= n) return;
-    const int s = identity ? h : slot[h];
-    const double *r = st + (size_t)8 * h;
-    pos[s] = make_double4(r[0], r[1], r[2], r[3]);
-    typ[s] = st_t[h] - 1;
-    if (identity) gid[s] = h;
-    if (with_vel) vel[s] = make_double4(r[4], r[5], r[6], r[7]);
-    if (!identity) {
-        const double4 q = sa.xref[s];
-        const double x[3] = {r[0], r[1], r[2]}, x0[3] = {q.x, q.y, q.z};
-        if (strayed(sa, x, x0)) *sa.flag = sa.no;
+    __shared__ double wmax[kLoadThreads / 64];
+    const int h = blockIdx.x * kLoadThreads + threadIdx.x;
+    double r2 = 0.0;
+    if (h < a.n) {
+        const int s = a.slot ? a.slot[h] : h;
+        const double4 *r = (const double4 *)(a.st + (size_t)a.row * h);
+        const double4 p = r[0];
+        a.typ[s] = a.st_t[h] - 1;
+        a.pos[s] = p;
+        if (!a.slot) a.gid[s] = h;
+        if (a.row == 8) a.vel[s] = r[1];
+        if (a.slot) {
+            const double4 q = a.stray.xref[s];
+            const double x[3] = {p.x, p.y, p.z}, x0[3] = {q.x, q.y, q.z};
+            if (strayed(a.stray, x, x0)) *a.stray.flag = a.stray.no;
+            const double dx = min_image_1(p.x, q.x, a.b.L[0], a.b.invL[0]);
+            const double dy = min_image_1(p.y, q.y, a.b.L[1], a.b.invL[1]);
+            const double dz = min_image_1(p.z, q.z, a.b.L[2], a.b.invL[2]);
+            r2 = dx * dx + dy * dy + dz * dz;
+        }
+    }
+    if (!a.disp) return;  // uniform
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) r2 = fmax(r2, __shfl_xor(r2, o, 64));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = r2;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long m = 0;
+        for (int w = 0; w < kLoadThreads / 64; w++)
+            m = max(m, (unsigned long long)__double_as_longlong(wmax[w]));
+        a.disp[blockIdx.x] = m;
     }
 }
 
-// cell order -> host-order staging: x y z | vx vy vz | fx fy fz
-__global__ void k_store(double *__restrict__ st, int n, const int32_t *__restrict__ gid, const double4 *pos,
-                        const double4 *vel, const double4 *frc)
+// Cell order -> host order, into pinned host memory: W = 3, the forces; W =
+// 9, x y z | vx vy vz | fx fy fz.  frc_recip, when not null, is added first
+// (total force += 2 scale (F_recip - mean F_recip), ewald_general.F90:857-864,
+// ewald_spole.F90:430), here and in frc.  Bound by the host link (8 W bytes an
+// atom): threads take the atoms in host order, gathering from the card's own
+// memory, and a workgroup's rows go out through LDS as whole lines.
+// STORE_FIGURES
+struct StoreArgs {
+    double *out;
+    int n;
+    const int32_t *slot;
+    const double4 *pos, *vel;
+    double4 *frc;
+    const double4 *frc_recip;
+    const double *red_out;
+    double two_scale, inv_n;
+};
+constexpr int kStoreThreads = 256;
+template <int W>
+__global__ void __launch_bounds__(kStoreThreads) k_store(StoreArgs a)
 {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int h = gid[s];
-    double *r = st + (size_t)9 * h;
-    if (pos) {
-        const double4 p = pos[s];
-        r[0] = p.x; r[1] = p.y; r[2] = p.z;
+    __shared__ double row[kStoreThreads * W];
+    const int t = threadIdx.x, h = blockIdx.x * kStoreThreads + t;
+    if (h < a.n) {
+        const int s = a.slot[h];
+        double4 f = a.frc[s];
+        if (a.frc_recip) {
+            const double4 r = a.frc_recip[s];
+            f.x += (r.x - a.red_out[R_FNETX] * a.inv_n) * a.two_scale;
+            f.y += (r.y - a.red_out[R_FNETY] * a.inv_n) * a.two_scale;
+            f.z += (r.z - a.red_out[R_FNETZ] * a.inv_n) * a.two_scale;
+            a.frc[s] = f;
+        }
+        double *o = row + W * t;
+        if (W == 9) {
+            const double4 p = a.pos[s], v = a.vel[s];
+            o[0] = p.x; o[1] = p.y; o[2] = p.z;
+            o[3] = v.x; o[4] = v.y; o[5] = v.z;
+        }
+        o[W - 3] = f.x; o[W - 2] = f.y; o[W - 1] = f.z;
     }
-    if (vel) {
-        const double4 v = vel[s];
-        r[3] = v.x; r[4] = v.y; r[5] = v.z;
-    }
-    const double4 f = frc[s];
-    r[6] = f.x; r[7] = f.y; r[8] = f.z;
+    __syncthreads();
+    const size_t base = (size_t)blockIdx.x * kStoreThreads * W, end = (size_t)a.n * W;
+#pragma unroll
+    for (int k = 0; k < W; k++)
+        if (base + k * kStoreThreads + t < end) a.out[base + k * kStoreThreads + t] = row[k * kStoreThreads + t];
 }
 
 static Vv1Args vv1_args(Ctx *c, double dt)
@@ -555,10 +622,13 @@ int step_launch(Ctx *c, hipStream_t s, const BatchLaunch &bl, bool stage2, bool 
     return 0;
 }
 
-int load_atoms(Ctx *c, const double *st_dev, const int32_t *st_t_dev, bool identity, bool with_vel)
+int load_blocks(const Ctx *c) { return ceil_div(c->natms, kLoadThreads); }
+
+int load_atoms(Ctx *c, bool identity, bool with_vel, bool disp)
 {
-    StrayArgs sa{};
+    LoadArgs a{};
     if (!identity) {
+        StrayArgs &sa = a.stray;
         sa.xref = c->xref;
         for (int d = 0; d < 3; d++) {
             sa.L0[d] = c->list_L[d];
@@ -571,17 +641,42 @@ int load_atoms(Ctx *c, const double *st_dev, const int32_t *st_t_dev, bool ident
         c->upload_no = c->upload_no == INT32_MAX ? 1 : c->upload_no + 1;
         sa.no = c->upload_no;
     }
-    c->stray_no = sa.no;
-    hipLaunchKernelGGL(k_load, dim3(ceil_div(c->natms, 256)), dim3(256), 0, c->stream, st_dev, st_t_dev, c->natms,
-                       c->cap, c->slot, identity, with_vel, c->pos, c->typ, c->gid, c->vel, sa);
+    c->stray_no = a.stray.no;
+    a.st = c->h_st_dev;
+    a.st_t = c->h_t_dev;
+    a.n = c->natms;
+    a.row = with_vel ? 8 : 4;
+    a.slot = identity ? nullptr : c->slot;
+    a.pos = c->pos;
+    a.vel = c->vel;
+    a.typ = c->typ;
+    a.gid = c->gid;
+    a.disp = disp ? (unsigned long long *)c->h_disp_dev : nullptr;
+    for (int d = 0; d < 3; d++) {
+        a.b.L[d] = c->L[d];
+        a.b.invL[d] = c->invL[d];
+    }
+    hipLaunchKernelGGL(k_load, dim3(load_blocks(c)), dim3(kLoadThreads), 0, c->stream, a);
     DLPX_HIP(c, hipGetLastError());
     return 0;
 }
 
-int store_atoms(Ctx *c, double *st_dev, bool with_pos, bool with_vel)
+int store_atoms(Ctx *c, bool with_state, bool finish)
 {
-    hipLaunchKernelGGL(k_store, dim3(ceil_div(c->natms, 256)), dim3(256), 0, c->stream, st_dev, c->natms, c->gid,
-                       with_pos ? c->pos : nullptr, with_vel ? c->vel : nullptr, c->frc);
+    StoreArgs a{};
+    a.out = c->h_st_dev;
+    a.n = c->natms;
+    a.slot = c->slot;
+    a.pos = c->pos;
+    a.vel = c->vel;
+    a.frc = c->frc;
+    a.frc_recip = finish ? c->frc_recip : nullptr;
+    a.red_out = c->red_out;
+    a.two_scale = finish ? 2.0 * recip_scale(c) : 0.0;
+    a.inv_n = 1.0 / (double)c->natms;
+    const dim3 grid(ceil_div(c->natms, kStoreThreads));
+    if (with_state) hipLaunchKernelGGL(k_store<9>, grid, dim3(kStoreThreads), 0, c->stream, a);
+    else hipLaunchKernelGGL(k_store<3>, grid, dim3(kStoreThreads), 0, c->stream, a);
     DLPX_HIP(c, hipGetLastError());
     return 0;
 }

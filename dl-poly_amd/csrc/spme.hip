@@ -1108,9 +1108,9 @@ __device__ __forceinline__ void reduce_body(const double *__restrict__ red, cons
         if (rec) rec[col] = v;
     }
 }
-__global__ void __launch_bounds__(256) k_reduce(const double *__restrict__ red, RedRows rr, double *out)
+__global__ void __launch_bounds__(256) k_reduce(const double *__restrict__ red, RedRows rr, double *out, double *rec)
 {
-    reduce_body(red, rr.rows, out, blockIdx.x, nullptr);
+    reduce_body(red, rr.rows, out, blockIdx.x, rec);
 }
 
 int ensure_red_rows(Ctx *c, int rows)
@@ -1123,11 +1123,11 @@ int ensure_red_rows(Ctx *c, int rows)
     return 0;
 }
 
-int reduce_partials(Ctx *c)
+int reduce_partials(Ctx *c, double *rec)
 {
     RedRows rr;
     for (int k = 0; k < kReduceSlots; k++) rr.rows[k] = c->red_rows[k];
-    hipLaunchKernelGGL(k_reduce, dim3(kReduceSlots), dim3(256), 0, c->stream, c->red, rr, c->red_out);
+    hipLaunchKernelGGL(k_reduce, dim3(kReduceSlots), dim3(256), 0, c->stream, c->red, rr, c->red_out, rec);
     DLPX_HIP(c, hipGetLastError());
     return 0;
 }
