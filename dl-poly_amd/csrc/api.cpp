@@ -19,6 +19,7 @@ uint64_t next_serial();
 void ensemble_free(void *e);
 int ensemble_run(const std::vector<Ctx *> &cs, Ensemble *&E, int nsteps, bool energies, std::vector<int> &rebuilds);
 int store_atoms(Ctx *c, bool with_state, bool finish);
+int store_per_particle(Ctx *c, double scale);
 int spme_finish(Ctx *c, double two_scale);
 
 int fail(Ctx *c, int code, const std::string &msg)
@@ -851,13 +852,6 @@ int dlpx_add_per_particle(dlpx_ctx *ctx, double *energy, double *stress)
     if (!c->pp_valid)
         return fail(c, DLPX_ERR_STATE, "no per-particle data: dlpx_set_per_particle(ctx, 1), then dlpx_two_body_forces");
     const int n = c->natms;
-    std::vector<double> pp((size_t)n * kPPStride);
-    std::vector<double4> fr(c->prm.electrostatics ? n : 0);
-    std::vector<int32_t> gid(n);
-    DLPX_HIP(c, hipMemcpy(pp.data(), c->pp, sizeof(double) * pp.size(), hipMemcpyDeviceToHost));
-    DLPX_HIP(c, hipMemcpy(gid.data(), c->gid, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-    if (c->prm.electrostatics)
-        DLPX_HIP(c, hipMemcpy(fr.data(), c->frc_recip, sizeof(double4) * n, hipMemcpyDeviceToHost));
     // ewald_spole.F90:429-431,464-466 (reciprocal energy and stress scaled,
     // the self energy shared evenly) and two_body.F90:783 (the vdW long-range
     // correction shared evenly); the exclusion correction and the net-charge
@@ -866,14 +860,15 @@ int dlpx_add_per_particle(dlpx_ctx *ctx, double *energy, double *stress)
                                                      (0.5 * (1.0 / c->volm)) * (kR4pie0 / c->prm.epsilon)
                                                : 0.0;
     const double share = (c->prm.electrostatics ? c->self_energy : 0.0) / n + c->elrc / n;
+    int r;
+    if ((r = store_per_particle(c, scale))) return r;
+    DLPX_HIP(c, hipStreamSynchronize(c->stream));
     const int sym[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};  // 3x3 element -> (xx, xy, xz, yy, yz, zz)
-    for (int i = 0; i < n; i++) {
-        const double *p = pp.data() + (size_t)i * kPPStride;
-        const int h = gid[i];
-        if (energy) energy[h] += p[0] + (c->prm.electrostatics ? fr[i].w * scale : 0.0) + share;
+    for (int h = 0; h < n; h++) {
+        const double *p = c->h_st + (size_t)7 * h;
+        if (energy) energy[h] += p[0] + share;
         if (stress)
-            for (int k = 0; k < 9; k++)
-                stress[(size_t)9 * h + k] += p[1 + sym[k]] + (c->prm.electrostatics ? p[8 + sym[k]] * scale : 0.0);
+            for (int k = 0; k < 9; k++) stress[(size_t)9 * h + k] += p[1 + sym[k]];
     }
     return 0;
 }

@@ -959,10 +959,10 @@ static PairVariant pair_variant(const Ctx *c, int lanes, long natms, size_t &lds
     const bool gtab = !direct && lds_tab + lds_rest > 160 * 1024;
     lds = (gtab ? 0 : lds_tab) + lds_rest;
     // per-particle output, direct mode and global tables run with 8 lanes per
-    // atom; per-particle output from LDS tables also in the few-atom shape
+    // atom; all but the global tables also in the few-atom shape
     int threads = kPairThreads;
     if (gtab || c->pp_now || direct) lanes = 8;
-    if (!gtab && !direct) wide_shape(natms, lanes, threads);
+    if (!gtab) wide_shape(natms, lanes, threads);
     PairVariant v{lanes, c->vdw_force_shift, direct, c->pp_now, gtab};
     v.nt = threads;
     return v;
@@ -1021,13 +1021,13 @@ static int pair_setup(Ctx *c, PairArgs<R> &a, size_t &lds, PairVariant &v, int l
 }
 
 // Calls CALL(GP, NT, FS, DIRECT, PP, GT) with the compile-time values of v.
-#define DLPX_PAIR_SHAPES(v, CALL, FS, PP)                                                        \
+#define DLPX_PAIR_SHAPES(v, CALL, FS, DIRECT, PP)                                            \
     do {                                                                                     \
         if ((v).gp == kWideLanes) {                                                          \
-            if ((v).nt == kWideMin) CALL(kWideLanes, kWideMin, FS, false, PP, false);        \
-            else CALL(kWideLanes, kWideMax, FS, false, PP, false);                           \
-        } else if (PP) {                                                                     \
-            CALL(8, kPairThreads, FS, false, PP, false);                                     \
+            if ((v).nt == kWideMin) CALL(kWideLanes, kWideMin, FS, DIRECT, PP, false);       \
+            else CALL(kWideLanes, kWideMax, FS, DIRECT, PP, false);                          \
+        } else if (PP || DIRECT) {                                                           \
+            CALL(8, kPairThreads, FS, DIRECT, PP, false);                                    \
         } else {                                                                             \
             switch ((v).gp) {                                                                \
                 case 16: CALL(16, kPairThreads, FS, false, false, false); break;             \
@@ -1036,21 +1036,24 @@ static int pair_setup(Ctx *c, PairArgs<R> &a, size_t &lds, PairVariant &v, int l
             }                                                                                \
         }                                                                                    \
     } while (0)
-#define DLPX_PAIR_VARIANTS(v, CALL)                                                          \
+#define DLPX_PAIR_FORMS(v, CALL, FS)                                                         \
     do {                                                                                     \
         if ((v).gt) {                                                                        \
-            if ((v).pp) { if ((v).fs) CALL(8, kPairThreads, true, false, true, true); else CALL(8, kPairThreads, false, false, true, true); } \
-            else { if ((v).fs) CALL(8, kPairThreads, true, false, false, true); else CALL(8, kPairThreads, false, false, false, true); }      \
+            if ((v).pp) CALL(8, kPairThreads, FS, false, true, true);                        \
+            else CALL(8, kPairThreads, FS, false, false, true);                              \
         } else if ((v).pp) {                                                                 \
-            if ((v).direct) { if ((v).fs) CALL(8, kPairThreads, true, true, true, false); else CALL(8, kPairThreads, false, true, true, false); } \
-            else { if ((v).fs) DLPX_PAIR_SHAPES(v, CALL, true, true); else DLPX_PAIR_SHAPES(v, CALL, false, true); } \
+            if ((v).direct) DLPX_PAIR_SHAPES(v, CALL, FS, true, true);                       \
+            else DLPX_PAIR_SHAPES(v, CALL, FS, false, true);                                 \
         } else if ((v).direct) {                                                             \
-            if ((v).fs) CALL(8, kPairThreads, true, true, false, false); else CALL(8, kPairThreads, false, true, false, false); \
-        } else if ((v).fs) {                                                                 \
-            DLPX_PAIR_SHAPES(v, CALL, true, false);                                                 \
+            DLPX_PAIR_SHAPES(v, CALL, FS, true, false);                                      \
         } else {                                                                             \
-            DLPX_PAIR_SHAPES(v, CALL, false, false);                                                \
+            DLPX_PAIR_SHAPES(v, CALL, FS, false, false);                                     \
         }                                                                                    \
+    } while (0)
+#define DLPX_PAIR_VARIANTS(v, CALL)                                                          \
+    do {                                                                                     \
+        if ((v).fs) DLPX_PAIR_FORMS(v, CALL, true);                                          \
+        else DLPX_PAIR_FORMS(v, CALL, false);                                                \
     } while (0)
 // Calls CALL(GP, REL, NT) for the combined-table kernel's shapes.
 #define DLPX_COMB_VARIANTS(v, CALL)                                                          \

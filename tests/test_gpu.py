@@ -1021,3 +1021,37 @@ def test_pair_launch_shapes_agree(kind, size, monkeypatch):
             print("case", kind, size, precision, lanes, rms_rel(r["frc"], ref["frc"]), flush=True)
             assert rms_rel(r["frc"], ref["frc"]) <= tol
             assert abs(r["engsrp"] - ref["engsrp"]) <= etol * abs(ref["engsrp"])
+
+
+@pytest.mark.parametrize("size", [(8, 8, 8), (8, 8, 16), (8, 8, 17)])
+@pytest.mark.parametrize("direct", [False, True])
+def test_per_particle_and_direct_launch_shapes_agree(size, direct):
+    """Per-particle output and analytic vdW forms on both sides of the line
+    between 32 and 8 lanes to an atom (8,192 atoms): per-particle evaluations
+    give the plain ones' forces (another kernel with the same arithmetic, 1e-12),
+    analytic forms the tables' (the tables' interpolation error, below 1e-5),
+    and each atom's energies and stresses add up the same with the atoms taken
+    in reverse order (1e-12 of the largest)."""
+    s = systems.nacl(ncells=size, kvec=(32, 32, 32), seed=15)
+    rev = systems.nacl(ncells=size, kvec=(32, 32, 32), seed=15)
+    for k in ("pos", "vel", "types"):
+        setattr(rev, k, getattr(s, k)[::-1].copy())
+    got = {}
+    for name, sys_, pp in (("plain", s, False), ("pp", s, True), ("rev", rev, True)):
+        sys_.vdw_direct = direct
+        ctx = lib.Context(sys_, precision=lib.FP64)
+        ctx.link_cell_pairs(sys_.pos)
+        got[name] = ctx.two_body_forces(sys_.pos, per_particle=pp)
+        ctx.close()
+    s.vdw_direct = False
+    ctx = lib.Context(s, precision=lib.FP64)
+    ctx.link_cell_pairs(s.pos)
+    tables = ctx.two_body_forces(s.pos)
+    ctx.close()
+    a, b = got["pp"], got["rev"]
+    print("case", size, direct, rms_rel(a["frc"], got["plain"]["frc"]), flush=True)
+    assert rms_rel(a["frc"], got["plain"]["frc"]) <= 1e-12
+    assert rms_rel(a["frc"], tables["frc"]) <= 1e-5
+    assert rms_rel(b["frc"][::-1], a["frc"]) <= 1e-12
+    st = np.abs(a["pp_stress"]).max()
+    assert np.abs(b["pp_stress"][::-1] - a["pp_stress"]).max() <= 1e-12 * st
