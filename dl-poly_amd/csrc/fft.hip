@@ -629,7 +629,7 @@ template <typename T>
 static int run_y(Ctx *c, int sign)
 {
     if (use_lines(c, c->K[1])) {
-        const int lpb = lines_lpb<T>();
+        const int lpb = lines_lpb<T>(0, c->K[1]);
         const C2CArgs<T> a = y_args<T>(c, sign, lpb);
         return lines_c2c<T>(c, c->sp, a, ceil_div(a.lm.nl, lpb));
     }
@@ -655,7 +655,7 @@ static int run_z_conv(Ctx *c, const InflParams &ip)
     int r;
     if (ip.mode == 0 && (r = theta_update(c, ip, c->sp))) return r;
     if (ip.mode == 0 && use_lines(c, c->K[2])) {
-        const int ll = lines_lpb<T>();
+        const int ll = lines_lpb<T>(1, c->K[2]);
         const ZConvArgs<T> a = z_args<T>(c, ip, ll);
         const int nb = ceil_div(a.lm.nl, ll);
         for (int k = R_RS11; k <= R_RS33; k++) c->red_rows[k] = nb;
@@ -680,7 +680,7 @@ static int run_x(Ctx *c, bool forward, void *grid, bool clear = false)
 {
     const int n = c->K[0];
     if (use_lines(c, n)) {
-        const int ll = lines_lpb<T>(), nb = x_blocks(c, ll);
+        const int ll = lines_lpb<T>(2, n), nb = x_blocks(c, ll);
         if (forward) {
             const R2CArgs<T> a = r2c_args<T>(c, grid, clear);
             return lines_x<T>(c, c->sp, &a, nullptr, nb);
@@ -814,7 +814,7 @@ static int fft_prepare_t(const std::vector<Ctx *> &cs, const std::vector<InflPar
             if (std::find(distinct.begin(), distinct.end(), keys[k]) == distinct.end()) distinct.push_back(keys[k]);
         }
         for (int key : distinct) {
-            const int lpb = key > 0 ? lines_lpb<T>() : lg[d];
+            const int lpb = key > 0 ? lines_lpb<T>(d == 0 ? 2 : d == 1 ? 0 : 1, key) : lg[d];
             int r = 0;
             if (key > kPlaneKey) {
                 const int n = key - kPlaneKey;
@@ -916,7 +916,7 @@ int fft_launch(Ctx *c, hipStream_t s, const FftBatch &fb)
 int conv_blocks(const Ctx *c)
 {
     if (use_lines(c, c->K[2])) {
-        const int ll = c->prm.precision == DLPX_MIXED ? lines_lpb<float>() : lines_lpb<double>();
+        const int ll = c->prm.precision == DLPX_MIXED ? lines_lpb<float>(1, c->K[2]) : lines_lpb<double>(1, c->K[2]);
         return ceil_div((long)z_lines(c, ll).nl, ll);
     }
     const int lpb = c->prm.precision == DLPX_MIXED ? z_lpb<float>(c) : z_lpb<double>(c);

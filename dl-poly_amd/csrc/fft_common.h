@@ -222,7 +222,7 @@ bool lines_supported(int n);
 template <typename T> size_t plane_lds(int n);
 template <typename T> int plane_run(Ctx *c, hipStream_t s, bool inverse, int n, const PlaneArgs<T> &a);
 template <typename T> int plane_batch(Ctx *c, hipStream_t s, bool inverse, int n, const BatchLaunch &bl);
-template <typename T> int lines_lpb();
+template <typename T> int lines_lpb(int kind, int n);
 template <typename T> size_t lines_lds(int kind, int n);
 template <typename T> int lines_c2c(Ctx *c, hipStream_t s, const C2CArgs<T> &a, int nb);
 template <typename T> int lines_zconv(Ctx *c, hipStream_t s, const ZConvArgs<T> &a, int nb);

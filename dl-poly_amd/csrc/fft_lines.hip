@@ -14,6 +14,11 @@
 // radix 2, 3, 4 and 5 butterflies with constant twiddles.  The z pass runs
 // forward, influence function and inverse (the inverse in the transposed
 // order, starting from the registers stage B left) with two exchanges.
+//
+// Bound by HBM at large meshes: 360^3 in FP32 (188 MB of half spectrum) the y
+// passes take 80 and 72 us (4.7-5.2 TB/s), the x passes 91 and 82, the z pass
+// 181 (565 MB with theta, 3.1 TB/s); the Stockham kernels 126 each, 140, 125
+// and 360.
 #include <algorithm>
 
 #include "fft_reg.h"
@@ -38,6 +43,14 @@ __device__ __forceinline__ void load_line(const typename C2T<T>::type *__restric
 #pragma unroll
         for (int n1 = 0; n1 < N1; n1++) x[n1] = zero2<T2>();
 }
+
+// Lines beyond 128 points exchange in one LDS buffer, with a barrier between a
+// buffer's last read and its next write, where shorter ones alternate between
+// two: the second buffer cost occupancy (95 KB of LDS a workgroup at 360
+// points).  Against two buffers a step of 8,000 ions on a mesh of 240^3 takes
+// 226 us instead of 252 mixed and 400 instead of 440 in FP64, of 360^3 1,119
+// instead of 1,387 in FP64.
+constexpr bool one_exchange(int n1, int n2) { return n1 <= n2 && n1 * n2 > 128; }
 
 // ---- y axis: complex lines of the half spectrum, in place --------------------
 template <typename T, int N1, int N2, int LPB, int SGN>
@@ -82,7 +95,8 @@ __device__ __forceinline__ void lines_zconv_body(const ZConvArgs<T> &a, int bid)
     using D2 = RegDft<T, T2, N2, 1>;
     extern __shared__ __align__(16) unsigned char smem[];
     double *lred = (double *)smem;
-    T2 *ex0 = (T2 *)(smem + kConvRedBytes), *ex1 = ex0 + LPB * EXS, *stw = ex1 + LPB * EXS;
+    constexpr bool ONE = one_exchange(N1, N2);
+    T2 *ex0 = (T2 *)(smem + kConvRedBytes), *ex1 = ONE ? ex0 : ex0 + LPB * EXS, *stw = ex1 + LPB * EXS;
     const LineMap &lm = a.lm;
     const InflParams &ip = a.ip;
     const int ll = threadIdx.x % LPB, t = threadIdx.x / LPB;
@@ -111,6 +125,7 @@ __device__ __forceinline__ void lines_zconv_body(const ZConvArgs<T> &a, int bid)
     if (t < N2) stage_a<T, N1, N2, 1>(x, t, ex0 + ll * EXS, stw);
     __syncthreads();
     double acc[6] = {0, 0, 0, 0, 0, 0};
+    T2 one[ONE ? N2 : 1];  // ONE: the inverse's values until the exchange has been read
     if (t < N2) {
         // Reciprocal stress (ewald_spole.F90:1362-1378) of an orthorhombic
         // cell: m = (j r0, ky r4, kz r8) along the line, so with the per
@@ -146,6 +161,11 @@ __device__ __forceinline__ void lines_zconv_body(const ZConvArgs<T> &a, int bid)
                 // inverse over m2: u[q] = V[m1][n2 = perm(q)], then the
                 // twiddle exp(-2 pi i n2 m1 / N) and the exchange
                 RegDft<T, T2, N2, -1>::template run<0, 1>(u);
+                if constexpr (ONE) {
+#pragma unroll
+                    for (int q = 0; q < N2; q++) one[q] = u[q];
+                    continue;
+                }
 #pragma unroll
                 for (int q = 0; q < N2; q++) {
                     const int n2 = RegDft<T, T2, N2, -1>::perm(q);
@@ -172,6 +192,22 @@ __device__ __forceinline__ void lines_zconv_body(const ZConvArgs<T> &a, int bid)
             acc[3] = cp * my * my * W;
             acc[4] = my * r8 * Wz + (partner ? myp * r8 * Wzp : 0.0);
             acc[5] = cp * r8 * r8 * Wzz;
+        }
+    }
+    if constexpr (ONE) {
+        __syncthreads();
+        if (t < N1) {
+#pragma unroll
+            for (int q = 0; q < N2; q++) {
+                const int n2 = RegDft<T, T2, N2, -1>::perm(q);
+                T2 v = one[q];
+                if (n2 != 0) {
+                    T2 w = stw[n2 * t];
+                    w.y = -w.y;
+                    v = cmul(v, w);
+                }
+                ex1[ll * EXS + t * N2 + n2] = v;
+            }
         }
     }
     __syncthreads();
@@ -206,7 +242,8 @@ __device__ __forceinline__ void lines_r2c_body(const R2CArgs<T> &a, int bid)
     constexpr int N = N1 * N2, EXS = N + 1, RB = (N1 + N2 - 1) / N2, K1h = N / 2 + 1;
     constexpr int NT = (LPB * N2 + 63) / 64 * 64, UN = x_per_thread<LPB, N, NT>();
     extern __shared__ __align__(16) unsigned char smem[];
-    T2 *ex0 = (T2 *)smem, *ex1 = ex0 + LPB * EXS, *stw = ex1 + LPB * EXS;
+    constexpr bool ONE = one_exchange(N1, N2);
+    T2 *ex0 = (T2 *)smem, *ex1 = ONE ? ex0 : ex0 + LPB * EXS, *stw = ex1 + LPB * EXS;
     T *__restrict__ Q = a.Q;
     const int nreal = a.nreal_lines, npairs = (nreal + 1) / 2;
     const int P0 = bid * LPB, np = min(LPB, npairs - P0);
@@ -242,24 +279,24 @@ __device__ __forceinline__ void lines_r2c_body(const R2CArgs<T> &a, int bid)
     __syncthreads();
     const int ll = threadIdx.x % LPB, t = threadIdx.x / LPB;
     const bool on = t < N2 && ll < np;
-    if (on) {
+    {
         T2 x[N1];
+        if (on)
 #pragma unroll
-        for (int n1 = 0; n1 < N1; n1++) x[n1] = ex0[ll * EXS + t + N2 * n1];
-        stage_a<T, N1, N2, 1>(x, t, ex1 + ll * EXS, stw);
+            for (int n1 = 0; n1 < N1; n1++) x[n1] = ex0[ll * EXS + t + N2 * n1];
+        if (ONE) __syncthreads();
+        if (on) stage_a<T, N1, N2, 1>(x, t, ex1 + ll * EXS, stw);
     }
     __syncthreads();
-    if (on) {
 #pragma unroll
-        for (int r = 0; r < RB; r++) {
-            const int m1 = t + N2 * r;
-            if (m1 < N1) {
-                T2 y[N2];
-                stage_b<T, N1, N2, 1>(m1, ex1 + ll * EXS, y);
+    for (int r = 0; r < RB; r++) {
+        const int m1 = t + N2 * r;
+        T2 y[N2];
+        if (on && m1 < N1) stage_b<T, N1, N2, 1>(m1, ex1 + ll * EXS, y);
+        if (ONE) __syncthreads();
+        if (on && m1 < N1)
 #pragma unroll
-                for (int p = 0; p < N2; p++) ex0[ll * EXS + m1 + N1 * RegDft<T, T2, N2, 1>::perm(p)] = y[p];
-            }
-        }
+            for (int p = 0; p < N2; p++) ex0[ll * EXS + m1 + N1 * RegDft<T, T2, N2, 1>::perm(p)] = y[p];
     }
     __syncthreads();
     T2 *__restrict__ H = a.H;
@@ -295,8 +332,10 @@ __device__ __forceinline__ void lines_c2r_body(const C2RArgs<T> &a, int bid)
                   UN = x_per_thread<LPB, N, NT>();
     extern __shared__ __align__(16) unsigned char smem[];
     // hb: the two half spectra of each pair (2 K1h), later the output lines
-    T2 *ex = (T2 *)smem, *stw = ex + LPB * EXS, *hb = stw + N;
+    constexpr bool ONE = one_exchange(N1, N2);
     constexpr int HBS = 2 * K1h > N ? 2 * K1h : N;
+    static_assert(!ONE || HBS >= EXS, "the exchange lies in the half spectra's rows");
+    T2 *ex = (T2 *)smem, *stw = ex + LPB * (ONE ? HBS : EXS), *hb = ONE ? ex : stw + N;
     const T2 *__restrict__ H = a.H;
     T *__restrict__ Q = a.Q;
     const int nreal = a.nreal_lines, npairs = (nreal + 1) / 2, hs = a.hs;
@@ -322,38 +361,38 @@ __device__ __forceinline__ void lines_c2r_body(const C2RArgs<T> &a, int bid)
     __syncthreads();
     const int ll = threadIdx.x % LPB, t = threadIdx.x / LPB;
     const bool on = t < N2 && ll < np;
-    if (on) {
+    {
         T2 x[N1];
         const T2 *hl = hb + ll * HBS;
+        if (on)
 #pragma unroll
-        for (int n1 = 0; n1 < N1; n1++) {
-            const int k = t + N2 * n1;
-            const int kh = k < K1h ? k : N - k;
-            const T2 A = hl[kh], B = hl[K1h + kh];
-            T2 z;
-            if (k < K1h) {
-                z.x = A.x - B.y;
-                z.y = A.y + B.x;
-            } else {
-                z.x = A.x + B.y;
-                z.y = -A.y + B.x;
+            for (int n1 = 0; n1 < N1; n1++) {
+                const int k = t + N2 * n1;
+                const int kh = k < K1h ? k : N - k;
+                const T2 A = hl[kh], B = hl[K1h + kh];
+                T2 z;
+                if (k < K1h) {
+                    z.x = A.x - B.y;
+                    z.y = A.y + B.x;
+                } else {
+                    z.x = A.x + B.y;
+                    z.y = -A.y + B.x;
+                }
+                x[n1] = z;
             }
-            x[n1] = z;
-        }
-        stage_a<T, N1, N2, -1>(x, t, ex + ll * EXS, stw);
+        if (ONE) __syncthreads();
+        if (on) stage_a<T, N1, N2, -1>(x, t, ex + ll * EXS, stw);
     }
     __syncthreads();
-    if (on) {
 #pragma unroll
-        for (int r = 0; r < RB; r++) {
-            const int m1 = t + N2 * r;
-            if (m1 < N1) {
-                T2 y[N2];
-                stage_b<T, N1, N2, -1>(m1, ex + ll * EXS, y);
+    for (int r = 0; r < RB; r++) {
+        const int m1 = t + N2 * r;
+        T2 y[N2];
+        if (on && m1 < N1) stage_b<T, N1, N2, -1>(m1, ex + ll * EXS, y);
+        if (ONE) __syncthreads();
+        if (on && m1 < N1)
 #pragma unroll
-                for (int p = 0; p < N2; p++) hb[ll * HBS + m1 + N1 * RegDft<T, T2, N2, -1>::perm(p)] = y[p];
-            }
-        }
+            for (int p = 0; p < N2; p++) hb[ll * HBS + m1 + N1 * RegDft<T, T2, N2, -1>::perm(p)] = y[p];
     }
     __syncthreads();
 #pragma unroll
@@ -408,6 +447,7 @@ bool lines_supported(int n)
     switch (n) {
 #define DLPX_CASE(N, A, B) case N:
         DLPX_LINE_LENGTHS(DLPX_CASE)
+        DLPX_LONG_LINE_LENGTHS(DLPX_CASE)
 #undef DLPX_CASE
         return true;
         default: return false;
@@ -419,31 +459,50 @@ static int line_split2(int n)
     switch (n) {
 #define DLPX_CASE(N, A, B) case N: return B;
         DLPX_LINE_LENGTHS(DLPX_CASE)
+        DLPX_LONG_LINE_LENGTHS(DLPX_CASE)
 #undef DLPX_CASE
         default: return 0;
     }
 }
 
+// Lines per workgroup.  The strided y and z lines in 128-byte runs: 16
+// columns of FP32 complex, 8 of FP64.  The x and z passes of lines split over
+// more than 16 threads take 8 in FP32 too: with 16 their workgroups of five
+// wavefronts, at 130-170 registers a lane, fit a CU badly and not at all
+// beside one of the pair kernel.  At 360^3, 16 lines against 8: z pass 240 and
+// 181 us, forward x pass 141 and 91; at 240^3 (16 threads a line) a step of
+// 8,000 ions takes 226 us with 16 and 254 with 8.
 template <typename T>
-int lines_lpb()
+constexpr int line_lpb(int kind, int n2)
 {
-    // 128-byte runs of the strided y and z lines: 16 columns of FP32
-    // complex, 8 of FP64
-    return sizeof(T) == 4 ? 16 : 8;
+    return sizeof(T) == 4 && !(n2 > 16 && kind != 0) ? 16 : 8;
 }
-template int lines_lpb<float>();
-template int lines_lpb<double>();
+template <typename T>
+int lines_lpb(int kind, int n)
+{
+    return line_lpb<T>(kind, line_split2(n));
+}
+template int lines_lpb<float>(int, int);
+template int lines_lpb<double>(int, int);
 
 template <typename T>
-static int threads_for(int n)
+static int threads_for(int kind, int n)
 {
-    return (lines_lpb<T>() * line_split2(n) + 63) / 64 * 64;
+    return (lines_lpb<T>(kind, n) * line_split2(n) + 63) / 64 * 64;
 }
 
 template <typename T>
 size_t lines_lds(int kind, int n)
 {
-    const size_t e = sizeof(typename C2T<T>::type), lpb = lines_lpb<T>(), rows = lpb * (n + 1);
+    const size_t e = sizeof(typename C2T<T>::type), lpb = lines_lpb<T>(kind, n), rows = lpb * (n + 1);
+    const int n2 = line_split2(n);
+    if (one_exchange(n / n2, n2)) {
+        switch (kind) {
+            case 1: return kConvRedBytes + e * (rows + n);
+            case 3: return e * (lpb * std::max(2 * (n / 2 + 1), n) + n);
+            default: return e * (rows + n);
+        }
+    }
     switch (kind) {
         case 0: return e * (rows + n);                      // c2c
         case 1: return kConvRedBytes + e * (2 * rows + n);  // z pass
@@ -457,21 +516,21 @@ template size_t lines_lds<double>(int, int);
 template <typename T>
 int lines_c2c(Ctx *c, hipStream_t s, const C2CArgs<T> &a, int nb)
 {
-    constexpr int LPB = sizeof(T) == 4 ? 16 : 8;
-    const int n = a.pl.n, nt = threads_for<T>(n);
+    const int n = a.pl.n, nt = threads_for<T>(0, n);
     const size_t lds = lines_lds<T>(0, n);
     switch (n) {
 #define DLPX_CASE(N, A, B)                                                                                        \
     case N:                                                                                                       \
         if (a.sign > 0) {                                                                                         \
-            DLPX_LDS_MAX(c, (k_lines_c2c<T, A, B, LPB, 1>));                                                      \
-            hipLaunchKernelGGL((k_lines_c2c<T, A, B, LPB, 1>), dim3(nb), dim3(nt), lds, s, a);                    \
+            DLPX_LDS_MAX(c, (k_lines_c2c<T, A, B, line_lpb<T>(0, B), 1>));                                                      \
+            hipLaunchKernelGGL((k_lines_c2c<T, A, B, line_lpb<T>(0, B), 1>), dim3(nb), dim3(nt), lds, s, a);                    \
         } else {                                                                                                  \
-            DLPX_LDS_MAX(c, (k_lines_c2c<T, A, B, LPB, -1>));                                                     \
-            hipLaunchKernelGGL((k_lines_c2c<T, A, B, LPB, -1>), dim3(nb), dim3(nt), lds, s, a);                   \
+            DLPX_LDS_MAX(c, (k_lines_c2c<T, A, B, line_lpb<T>(0, B), -1>));                                                     \
+            hipLaunchKernelGGL((k_lines_c2c<T, A, B, line_lpb<T>(0, B), -1>), dim3(nb), dim3(nt), lds, s, a);                   \
         }                                                                                                         \
         break;
         DLPX_LINE_LENGTHS(DLPX_CASE)
+        DLPX_LONG_LINE_LENGTHS(DLPX_CASE)
 #undef DLPX_CASE
         default: return fail(c, DLPX_ERR_STATE, "no line kernel for this FFT length");
     }
@@ -482,16 +541,16 @@ int lines_c2c(Ctx *c, hipStream_t s, const C2CArgs<T> &a, int nb)
 template <typename T>
 int lines_zconv(Ctx *c, hipStream_t s, const ZConvArgs<T> &a, int nb)
 {
-    constexpr int LPB = sizeof(T) == 4 ? 16 : 8;
-    const int n = a.pl.n, nt = threads_for<T>(n);
+    const int n = a.pl.n, nt = threads_for<T>(1, n);
     const size_t lds = lines_lds<T>(1, n);
     switch (n) {
 #define DLPX_CASE(N, A, B)                                                                                        \
     case N:                                                                                                       \
-        DLPX_LDS_MAX(c, (k_lines_zconv<T, A, B, LPB>));                                                           \
-        hipLaunchKernelGGL((k_lines_zconv<T, A, B, LPB>), dim3(nb), dim3(nt), lds, s, a);                         \
+        DLPX_LDS_MAX(c, (k_lines_zconv<T, A, B, line_lpb<T>(1, B)>));                                                           \
+        hipLaunchKernelGGL((k_lines_zconv<T, A, B, line_lpb<T>(1, B)>), dim3(nb), dim3(nt), lds, s, a);                         \
         break;
         DLPX_LINE_LENGTHS(DLPX_CASE)
+        DLPX_LONG_LINE_LENGTHS(DLPX_CASE)
 #undef DLPX_CASE
         default: return fail(c, DLPX_ERR_STATE, "no line kernel for this FFT length");
     }
@@ -502,21 +561,21 @@ int lines_zconv(Ctx *c, hipStream_t s, const ZConvArgs<T> &a, int nb)
 template <typename T>
 int lines_x(Ctx *c, hipStream_t s, const R2CArgs<T> *fwd, const C2RArgs<T> *inv, int nb)
 {
-    constexpr int LPB = sizeof(T) == 4 ? 16 : 8;
-    const int n = fwd ? fwd->pl.n : inv->pl.n, nt = threads_for<T>(n);
+    const int n = fwd ? fwd->pl.n : inv->pl.n, nt = threads_for<T>(2, n);
     const size_t lds = lines_lds<T>(fwd ? 2 : 3, n);
     switch (n) {
 #define DLPX_CASE(N, A, B)                                                                                        \
     case N:                                                                                                       \
         if (fwd) {                                                                                                \
-            DLPX_LDS_MAX(c, (k_lines_r2c<T, A, B, LPB>));                                                         \
-            hipLaunchKernelGGL((k_lines_r2c<T, A, B, LPB>), dim3(nb), dim3(nt), lds, s, *fwd);                    \
+            DLPX_LDS_MAX(c, (k_lines_r2c<T, A, B, line_lpb<T>(2, B)>));                                                         \
+            hipLaunchKernelGGL((k_lines_r2c<T, A, B, line_lpb<T>(2, B)>), dim3(nb), dim3(nt), lds, s, *fwd);                    \
         } else {                                                                                                  \
-            DLPX_LDS_MAX(c, (k_lines_c2r<T, A, B, LPB>));                                                         \
-            hipLaunchKernelGGL((k_lines_c2r<T, A, B, LPB>), dim3(nb), dim3(nt), lds, s, *inv);                    \
+            DLPX_LDS_MAX(c, (k_lines_c2r<T, A, B, line_lpb<T>(2, B)>));                                                         \
+            hipLaunchKernelGGL((k_lines_c2r<T, A, B, line_lpb<T>(2, B)>), dim3(nb), dim3(nt), lds, s, *inv);                    \
         }                                                                                                         \
         break;
         DLPX_LINE_LENGTHS(DLPX_CASE)
+        DLPX_LONG_LINE_LENGTHS(DLPX_CASE)
 #undef DLPX_CASE
         default: return fail(c, DLPX_ERR_STATE, "no line kernel for this FFT length");
     }
@@ -527,9 +586,7 @@ int lines_x(Ctx *c, hipStream_t s, const R2CArgs<T> *fwd, const C2RArgs<T> *inv,
 template <typename T>
 int lines_batch(Ctx *c, hipStream_t s, int kind, int n, const BatchLaunch &bl)
 {
-    constexpr int LPB = sizeof(T) == 4 ? 16 : 8;
-    const int nt = threads_for<T>(n);
-    const dim3 g(bl.total), b(nt);
+    const dim3 g(bl.total), b(threads_for<T>(kind == 2 ? 1 : kind == 1 || kind == 3 ? 0 : 2, n));
 #define DLPX_BL(KERNEL, ARGS, ...)                                                                                \
     do {                                                                                                          \
         DLPX_LDS_MAX(c, (KERNEL<__VA_ARGS__>));                                                                   \
@@ -539,14 +596,15 @@ int lines_batch(Ctx *c, hipStream_t s, int kind, int n, const BatchLaunch &bl)
 #define DLPX_CASE(N, A, B)                                                                                        \
     case N:                                                                                                       \
         switch (kind) {                                                                                           \
-            case 0: DLPX_BL(k_lines_r2c_batch, R2CArgs, T, A, B, LPB); break;                                     \
-            case 1: DLPX_BL(k_lines_c2c_batch, C2CArgs, T, A, B, LPB, 1); break;                                  \
-            case 2: DLPX_BL(k_lines_zconv_batch, ZConvArgs, T, A, B, LPB); break;                                 \
-            case 3: DLPX_BL(k_lines_c2c_batch, C2CArgs, T, A, B, LPB, -1); break;                                 \
-            default: DLPX_BL(k_lines_c2r_batch, C2RArgs, T, A, B, LPB); break;                                    \
+            case 0: DLPX_BL(k_lines_r2c_batch, R2CArgs, T, A, B, line_lpb<T>(2, B)); break;                                     \
+            case 1: DLPX_BL(k_lines_c2c_batch, C2CArgs, T, A, B, line_lpb<T>(0, B), 1); break;                                  \
+            case 2: DLPX_BL(k_lines_zconv_batch, ZConvArgs, T, A, B, line_lpb<T>(1, B)); break;                                 \
+            case 3: DLPX_BL(k_lines_c2c_batch, C2CArgs, T, A, B, line_lpb<T>(0, B), -1); break;                                 \
+            default: DLPX_BL(k_lines_c2r_batch, C2RArgs, T, A, B, line_lpb<T>(2, B)); break;                                    \
         }                                                                                                         \
         break;
         DLPX_LINE_LENGTHS(DLPX_CASE)
+        DLPX_LONG_LINE_LENGTHS(DLPX_CASE)
 #undef DLPX_CASE
         default: return fail(c, DLPX_ERR_STATE, "no line kernel for this FFT length");
     }

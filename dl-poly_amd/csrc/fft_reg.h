@@ -215,5 +215,30 @@ __device__ __forceinline__ void stage_b(int m1, const typename C2T<T>::type *ex,
     X(100, 10, 10)           \
     X(120, 12, 10)           \
     X(128, 16, 8)
+// Longer lines (no plane kernels), N1 <= N2 (see one_exchange).  Steps of 8,000
+// ions on an N^3 mesh, Stockham kernels against these: N = 135 155 and 133 us
+// mixed, 212 and 168 in FP64; 200 239 and 182, 416 and 276; 256 388 and 261,
+// 692 and 432; 360 988 and 650, 1,988 and 1,120 (1.17 to 1.55 times mixed and 1.27
+// to 1.92 times in FP64 over all of them).  Longer ones stay with the Stockham
+// kernels: a factor above 20 no longer fits the registers in FP64.
+#define DLPX_LONG_LINE_LENGTHS(X) \
+    X(135, 9, 15)     \
+    X(144, 12, 12)    \
+    X(150, 10, 15)    \
+    X(160, 10, 16)    \
+    X(162, 9, 18)     \
+    X(180, 12, 15)    \
+    X(192, 12, 16)    \
+    X(200, 10, 20)    \
+    X(216, 12, 18)    \
+    X(225, 15, 15)    \
+    X(240, 15, 16)    \
+    X(256, 16, 16)    \
+    X(270, 15, 18)    \
+    X(288, 16, 18)    \
+    X(300, 15, 20)    \
+    X(320, 16, 20)    \
+    X(324, 18, 18)    \
+    X(360, 18, 20)
 
 }  // namespace dlpx

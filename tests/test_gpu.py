@@ -1055,3 +1055,32 @@ def test_per_particle_and_direct_launch_shapes_agree(size, direct):
     assert rms_rel(b["frc"][::-1], a["frc"]) <= 1e-12
     st = np.abs(a["pp_stress"]).max()
     assert np.abs(b["pp_stress"][::-1] - a["pp_stress"]).max() <= 1e-12 * st
+
+
+@pytest.mark.parametrize("n", [135, 144, 150, 160, 162, 180, 192, 200, 216, 225, 240, 256, 270, 288, 300, 320, 324, 360])
+def test_long_line_transforms_agree(n, monkeypatch):
+    """Meshes with an axis beyond 128 points: the line kernels and the generic
+    ones (DLPX_FFT_LINES=0) along x, y and z, the other axes shorter and of odd
+    line counts.  The same transform in another order of factors: FP64 forces,
+    energy and stress to 1e-12, mixed ones to the mode's bar (forces 1e-5 RMS,
+    energies 1e-6) against FP64's.  One call on host arrays and two resident steps
+    (the batched kernels)."""
+    for kvec in ((n, 27, 25), (25, n, 27), (30, 25, n)):
+        s = systems.nacl(ncells=5, kvec=kvec, seed=17)
+        ref = None
+        for precision, tol, etol in ((lib.FP64, 1e-12, 1e-12), (lib.MIXED, 1e-5, 1e-6)):
+            for lines in ("0", "1"):
+                monkeypatch.setenv("DLPX_FFT_LINES", lines)
+                ctx = lib.Context(s, precision=precision)
+                ctx.link_cell_pairs(s.pos)
+                r = ctx.two_body_forces(s.pos)
+                ctx.md_load(s.pos, s.vel)
+                ctx.md_run(3, s.timestep)
+                md = ctx.md_store()[2]
+                ctx.close()
+                ref = ref or (r, md)
+                print("case", kvec, precision, lines, rms_rel(r["frc"], ref[0]["frc"]), flush=True)
+                assert rms_rel(r["frc"], ref[0]["frc"]) <= tol
+                assert rms_rel(md, ref[1]) <= 10.0 * tol
+                assert abs(r["engcpe"] - ref[0]["engcpe"]) <= etol * abs(ref[0]["engcpe"])
+                assert np.abs(r["stress"] - ref[0]["stress"]).max() <= max(tol, etol) * np.abs(ref[0]["stress"]).max()
