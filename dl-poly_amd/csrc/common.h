@@ -4,6 +4,7 @@
 
 #include <atomic>
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -352,7 +353,7 @@ struct BatchLaunch {
 // the batched kernels of one list build (neighbours.hip)
 struct ListBatch {
     BatchLaunch wrap, scat, sort, bsub, blink, excl;
-    int32_t *gate = nullptr;  // one system: its F_UPD word, else null (per-system gates only)
+    std::shared_ptr<const void> one;  // one system: its kernels' arguments (a ListChain)
     // several systems: the compacted chain's plan (k_list_plan), its inputs
     // and the fixed grid of each kernel
     int32_t *plan = nullptr, *plan_nb = nullptr;

@@ -838,29 +838,19 @@ __device__ __forceinline__ void list_exclude_body(const ExclListArgs &a, int bid
 // of only the systems whose rebuild is due, from the plan k_list_plan wrote
 // (their indices act[], count at [nsys], and per kernel `row` the prefix sums
 // of their block counts), so the systems without a rebuild cost no dispatch.
-#define DLPX_LIST_KERNELS(NAME, ARGS, BOUNDS, CALL_SINGLE, CALL_BATCH, XCD)                                      \
-    __global__ void __launch_bounds__ BOUNDS NAME(ARGS a)                                                    \
+#define DLPX_LIST_KERNELS(NAME, ARGS, BOUNDS, CALL_SINGLE, CALL_BATCH, LOOP)                               \
+    __global__ void __launch_bounds__ BOUNDS NAME(ARGS a, int nb)                                            \
     {                                                                                                     \
         if (skip_build(a.upd)) return;                                                                    \
-        CALL_SINGLE;                                                                                      \
-    }                                                                                                     \
-    __global__ void __launch_bounds__ BOUNDS NAME##_batch(const ARGS *__restrict__ av,                       \
-                                                       const int32_t *__restrict__ boff, int nsys,        \
-                                                       const int32_t *__restrict__ gate)                  \
-    {                                                                                                     \
-        if (skip_build(gate)) return;                                                                     \
-        BatchPos bp;                                                                                      \
-        if (XCD) {                                                                                        \
-            if (!batch_pos(boff, nsys, bp)) return;                                                       \
+        int b = blockIdx.x;                                                                               \
+        if constexpr (LOOP) {                                                                             \
+            for (; b < nb; b += gridDim.x) {                                                              \
+                CALL_SINGLE;                                                                              \
+                __syncthreads(); /* the next block's use of LDS */                                       \
+            }                                                                                             \
         } else {                                                                                          \
-            if ((int)blockIdx.x >= boff[nsys]) return;                                                    \
-            bp.s = batch_find(boff, nsys, blockIdx.x);                                                    \
-            bp.b = blockIdx.x - boff[bp.s];                                                               \
-            bp.nb = boff[bp.s + 1] - boff[bp.s];                                                          \
+            CALL_SINGLE;                                                                                  \
         }                                                                                                 \
-        const ARGS &a = av[bp.s];                                                                          \
-        if (skip_build(a.upd)) return;                                                                    \
-        CALL_BATCH;                                                                                       \
     }                                                                                                     \
     __global__ void __launch_bounds__ BOUNDS NAME##_cbatch(const ARGS *__restrict__ av,                      \
                                                         const int32_t *__restrict__ plan, int nsys, int row) \
@@ -883,18 +873,14 @@ __device__ __forceinline__ void list_exclude_body(const ExclListArgs &a, int bid
             __syncthreads(); /* the next block's use of LDS */                                           \
         }                                                                                                 \
     }
-DLPX_LIST_KERNELS(k_wrap_scan, WrapArgs, (kWrapThreads), wrap_scan_body(a, blockIdx.x, gridDim.x),
-                  wrap_scan_body(a, bp.b, bp.nb), false)
-DLPX_LIST_KERNELS(k_scatter_copy, ScatterArgs, (256), scatter_copy_body(a, blockIdx.x), scatter_copy_body(a, bp.b), false)
-DLPX_LIST_KERNELS(k_sort_permute, SortArgs, (256), sort_permute_body(a, blockIdx.x), sort_permute_body(a, bp.b), false)
-DLPX_LIST_KERNELS(k_list_exclude, ExclListArgs, (kExclThreads), list_exclude_body(a, blockIdx.x), list_exclude_body(a, bp.b),
-                  false)
-DLPX_LIST_KERNELS(k_build_list, BuildArgs, (kListThreads),
-                  build_list_body<kLanesPerAtom>(a, xcd_block(blockIdx.x, gridDim.x)),
-                  build_list_body<kLanesPerAtom>(a, bp.b), true)
+DLPX_LIST_KERNELS(k_wrap_scan, WrapArgs, (kWrapThreads), wrap_scan_body(a, b, nb), wrap_scan_body(a, bp.b, bp.nb), true)
+DLPX_LIST_KERNELS(k_scatter_copy, ScatterArgs, (256), scatter_copy_body(a, b), scatter_copy_body(a, bp.b), true)
+DLPX_LIST_KERNELS(k_sort_permute, SortArgs, (256), sort_permute_body(a, b), sort_permute_body(a, bp.b), true)
+DLPX_LIST_KERNELS(k_list_exclude, ExclListArgs, (kExclThreads), list_exclude_body(a, b), list_exclude_body(a, bp.b), true)
+DLPX_LIST_KERNELS(k_build_list, BuildArgs, (kListThreads), build_list_body<kLanesPerAtom>(a, xcd_block(b, nb)),
+                  build_list_body<kLanesPerAtom>(a, bp.b), false)
 DLPX_LIST_KERNELS(k_build_list_sub, BuildArgs, (kListThreads, 6),
-                  build_list_sub_body<kLanesPerAtom>(a, xcd_block(blockIdx.x, gridDim.x)),
-                  build_list_sub_body<kLanesPerAtom>(a, bp.b), true)
+                  build_list_sub_body<kLanesPerAtom>(a, xcd_block(b, nb)), build_list_sub_body<kLanesPerAtom>(a, bp.b), false)
 #undef DLPX_LIST_KERNELS
 
 // The plan of a compacted list chain: the systems whose F_UPD asks for a
@@ -1056,22 +1042,30 @@ static int list_chain(Ctx *c, const int32_t *upd, ListChain &lc, int nsys = 1)
 }
 
 // Bin, sort and permute the atoms of a list chain (everything before the
-// list kernel itself).
+// list kernel itself).  The workgroups loop over the blocks of a launch beyond
+// kListGrid: in a resident run most steps' launches find no rebuild due and
+// return at once, and at 1,728,000 ions handing out the 216,000 workgroups of
+// the sort took 41 us of each step.  The list kernels have a workgroup per block
+// all the same (51 us there): a loop's hoisted arguments no longer fit the
+// scalar registers, and a rebuild of 4,000 atoms took 25 us instead of 20.
+constexpr int kListGrid = 4096;
 static void launch_sort(const ListChain &lc, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_wrap_scan, dim3(ceil_div(lc.n, kWrapThreads)), dim3(kWrapThreads), 0, s, lc.wrap);
-    hipLaunchKernelGGL(k_scatter_copy, dim3(ceil_div(lc.n, 256)), dim3(256), 0, s, lc.scat);
-    hipLaunchKernelGGL(k_sort_permute, dim3(lc.nkey), dim3(lc.sub ? 64 : 256), 0, s, lc.sort);
+    const int nw = ceil_div(lc.n, kWrapThreads), na = ceil_div(lc.n, 256);
+    hipLaunchKernelGGL(k_wrap_scan, dim3(std::min(nw, kListGrid)), dim3(kWrapThreads), 0, s, lc.wrap, nw);
+    hipLaunchKernelGGL(k_scatter_copy, dim3(std::min(na, kListGrid)), dim3(256), 0, s, lc.scat, na);
+    hipLaunchKernelGGL(k_sort_permute, dim3(std::min(lc.nkey, kListGrid)), dim3(lc.sub ? 64 : 256), 0, s, lc.sort, lc.nkey);
 }
 
 static void launch_build(const ListChain &lc, hipStream_t s)
 {
+    const int nb = xcd_grid(lc.nbuild), ne = ceil_div(lc.n, kExclAtoms);
     if (lc.sub)
-        hipLaunchKernelGGL(k_build_list_sub, dim3(xcd_grid(lc.nbuild)), dim3(kListThreads), 0, s, lc.build);
+        hipLaunchKernelGGL(k_build_list_sub, dim3(nb), dim3(kListThreads), 0, s, lc.build, nb);
     else
-        hipLaunchKernelGGL(k_build_list, dim3(xcd_grid(lc.nbuild)), dim3(kListThreads), 0, s, lc.build);
+        hipLaunchKernelGGL(k_build_list, dim3(nb), dim3(kListThreads), 0, s, lc.build, nb);
     if (lc.excl_on)
-        hipLaunchKernelGGL(k_list_exclude, dim3(ceil_div(lc.n, kExclAtoms)), dim3(kExclThreads), 0, s, lc.excl);
+        hipLaunchKernelGGL(k_list_exclude, dim3(std::min(ne, kListGrid)), dim3(kExclThreads), 0, s, lc.excl, ne);
 }
 
 // Bin, sort, permute and build the list from c->pos (current order); the
@@ -1152,6 +1146,13 @@ int list_prepare(const std::vector<Ctx *> &cs, ListBatch &lb)
         ListChain lc;
         if ((r = list_chain(c, c->flags + F_UPD, lc, (int)std::min<size_t>(cs.size(), 512)))) return r;
         if (c->cap_lane == 0 || !c->nbr) return fail(c, DLPX_ERR_STATE, "no list to rebuild on the device");
+        // a lone system: the kernels of a host-decided build, each gated on its
+        // decision word; several run the compacted chain
+        if (cs.size() == 1) {
+            list_batch_free(lb);
+            lb.one = std::make_shared<ListChain>(lc);
+            return 0;
+        }
         wrap.push_back(lc.wrap);
         scat.push_back(lc.scat);
         sort.push_back(lc.sort);
@@ -1173,34 +1174,29 @@ int list_prepare(const std::vector<Ctx *> &cs, ListBatch &lb)
         (r = batch_upload(c0, lb.blink, blink.data(), sizeof(BuildArgs), nb_link, true)) ||
         (r = batch_upload(c0, lb.excl, excl.data(), sizeof(ExclListArgs), nb_excl, false)))
         return r;
-    // a batch of one system gates every kernel on its own decision word, read
-    // first thing by each workgroup; several systems run the compacted chain
-    lb.gate = cs.size() == 1 ? c0->flags + F_UPD : nullptr;
-    if (cs.size() > 1) {
-        const int nsys = (int)cs.size();
-        const std::vector<int> *nbs[kListKernels] = {&nb_wrap, &nb_atoms, &nb_keys, &nb_sub, &nb_link, &nb_excl};
-        std::vector<int32_t> nb((size_t)kListKernels * nsys);
-        for (int q = 0; q < kListKernels; q++)
-            for (int k = 0; k < nsys; k++) nb[(size_t)q * nsys + k] = (*nbs[q])[k];
-        std::vector<int32_t *> gates(nsys);
-        for (int k = 0; k < nsys; k++) gates[k] = cs[k]->flags + F_UPD;
-        const size_t plan_words = (size_t)nsys + 1 + (size_t)kListKernels * (nsys + 1);
-        DLPX_HIP(c0, hipMalloc((void **)&lb.plan, sizeof(int32_t) * plan_words));
-        DLPX_HIP(c0, hipMalloc((void **)&lb.plan_nb, sizeof(int32_t) * nb.size()));
-        DLPX_HIP(c0, hipMalloc((void **)&lb.plan_gates, sizeof(int32_t *) * nsys));
-        DLPX_HIP(c0, dev_upload(c0->stream, lb.plan_nb, nb.data(), sizeof(int32_t) * nb.size()));
-        DLPX_HIP(c0, dev_upload(c0->stream, lb.plan_gates, gates.data(), sizeof(int32_t *) * nsys));
-        // fixed grids of the compacted kernels: enough workgroups to fill the
-        // GPU a few times over (the subcell and link-cell builds hold 52 KB of
-        // LDS each, three to a CU)
-        const int cap[kListKernels] = {2048, 2048, 8192, 1024, 1024, 2048};
-        for (int q = 0; q < kListKernels; q++) {
-            long tot = 0;
-            for (int k = 0; k < nsys; k++) tot += (*nbs[q])[k];
-            lb.plan_grid[q] = (int)std::min<long>(tot, cap[q]);
-        }
-        lb.nsys = nsys;
+    const int nsys = (int)cs.size();
+    const std::vector<int> *nbs[kListKernels] = {&nb_wrap, &nb_atoms, &nb_keys, &nb_sub, &nb_link, &nb_excl};
+    std::vector<int32_t> nb((size_t)kListKernels * nsys);
+    for (int q = 0; q < kListKernels; q++)
+        for (int k = 0; k < nsys; k++) nb[(size_t)q * nsys + k] = (*nbs[q])[k];
+    std::vector<int32_t *> gates(nsys);
+    for (int k = 0; k < nsys; k++) gates[k] = cs[k]->flags + F_UPD;
+    const size_t plan_words = (size_t)nsys + 1 + (size_t)kListKernels * (nsys + 1);
+    DLPX_HIP(c0, hipMalloc((void **)&lb.plan, sizeof(int32_t) * plan_words));
+    DLPX_HIP(c0, hipMalloc((void **)&lb.plan_nb, sizeof(int32_t) * nb.size()));
+    DLPX_HIP(c0, hipMalloc((void **)&lb.plan_gates, sizeof(int32_t *) * nsys));
+    DLPX_HIP(c0, dev_upload(c0->stream, lb.plan_nb, nb.data(), sizeof(int32_t) * nb.size()));
+    DLPX_HIP(c0, dev_upload(c0->stream, lb.plan_gates, gates.data(), sizeof(int32_t *) * nsys));
+    // fixed grids of the compacted kernels: enough workgroups to fill the
+    // GPU a few times over (the subcell and link-cell builds hold 52 KB of
+    // LDS each, three to a CU)
+    const int cap[kListKernels] = {2048, 2048, 8192, 1024, 1024, 2048};
+    for (int q = 0; q < kListKernels; q++) {
+        long tot = 0;
+        for (int k = 0; k < nsys; k++) tot += (*nbs[q])[k];
+        lb.plan_grid[q] = (int)std::min<long>(tot, cap[q]);
     }
+    lb.nsys = nsys;
     return 0;
 }
 
@@ -1231,21 +1227,11 @@ int list_launch(Ctx *c, hipStream_t s, const ListBatch &lb, int part)
         DLPX_HIP(c, hipGetLastError());
         return 0;
     }
-#define DLPX_LB(K, BL, ARGS, NT)                                                                          \
-    if ((BL).total > 0)                                                                                  \
-        hipLaunchKernelGGL(K, dim3((BL).total), dim3(NT), 0, s, (const ARGS *)(BL).args, (BL).boff, (BL).nsys, \
-                           (const int32_t *)lb.gate)
-    if (p0) {
-        DLPX_LB(k_wrap_scan_batch, lb.wrap, WrapArgs, kWrapThreads);
-        DLPX_LB(k_scatter_copy_batch, lb.scat, ScatterArgs, 256);
-        DLPX_LB(k_sort_permute_batch, lb.sort, SortArgs, 256);
+    if (lb.one) {
+        const ListChain &lc = *static_cast<const ListChain *>(lb.one.get());
+        if (p0) launch_sort(lc, s);
+        if (p1) launch_build(lc, s);
     }
-    if (p1) {
-        DLPX_LB(k_build_list_sub_batch, lb.bsub, BuildArgs, kListThreads);
-        DLPX_LB(k_build_list_batch, lb.blink, BuildArgs, kListThreads);
-        DLPX_LB(k_list_exclude_batch, lb.excl, ExclListArgs, kExclThreads);
-    }
-#undef DLPX_LB
     DLPX_HIP(c, hipGetLastError());
     return 0;
 }
@@ -1257,7 +1243,7 @@ void list_batch_free(ListBatch &lb)
         if (p) (void)hipFree(p);
     lb.plan = lb.plan_nb = nullptr;
     lb.plan_gates = nullptr;
-    lb.gate = nullptr;
+    lb.one.reset();
 }
 
 int count_pairs_dev(Ctx *c, double r, int64_t *npairs)
