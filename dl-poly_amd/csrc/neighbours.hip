@@ -60,46 +60,89 @@ __device__ __forceinline__ bool skip_build(const int32_t *upd) { return upd && *
 // hundreds of thousands of keys at a million atoms).  The counts are zeroed
 // once read, ready for the next build.  With subcells (cell_start not null)
 // the link-cell starts are the starts of every 8th key.
+//
+// Bound by latency, one workgroup on one CU: a pass is a scan inside each
+// wavefront, one barrier and the wavefronts' totals, with the next pass's
+// counts already being read; a thread's run moves in 8- and 16-byte pieces (a
+// word at a time its 32 accesses, 32 bytes from lane to lane, took 14 us a pass).
+// The whole kernel at a rebuild: 1,728,000 ions in 216,000 subcells 404 -> 118 us,
+// 64,000 ions 18 -> 12, a 4,000-atom mixture 9.4 -> 6.6.
 constexpr int kScanRun = 8;
 constexpr int kWrapThreads = 1024;
 __device__ __forceinline__ void scan_keys(int32_t *count, int32_t *start, int32_t *fill, int n, int32_t *cell_start)
 {
-    __shared__ int32_t part[kWrapThreads];
-    __shared__ int32_t carry;
-    if (threadIdx.x == 0) carry = 0;
-    __syncthreads();
-    for (int base = 0; base < n; base += kWrapThreads * kScanRun) {
-        const int i0 = base + threadIdx.x * kScanRun;
-        int v[kScanRun], sum = 0;
+    constexpr int NW = kWrapThreads / 64, STEP = kWrapThreads * kScanRun;
+    __shared__ int32_t wsum[2][NW];  // alternating, so that one barrier a pass is enough
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int32_t v[kScanRun];
+    static_assert(kScanRun == 8, "runs of two 16-byte stores, and the link-cell starts");
+    auto read = [&](const int i0) {
+        if (i0 + kScanRun <= n) {
 #pragma unroll
-        for (int k = 0; k < kScanRun; k++) {
-            v[k] = i0 + k < n ? load_coherent(&count[i0 + k]) : 0;
-            sum += v[k];
-        }
-#pragma unroll
-        for (int k = 0; k < kScanRun; k++)
-            if (i0 + k < n) count[i0 + k] = 0;
-        part[threadIdx.x] = sum;
-        __syncthreads();
-        for (int o = 1; o < kWrapThreads; o <<= 1) {
-            int t = threadIdx.x >= o ? part[threadIdx.x - o] : 0;
-            __syncthreads();
-            part[threadIdx.x] += t;
-            __syncthreads();
-        }
-        int run = carry + part[threadIdx.x] - sum;
-#pragma unroll
-        for (int k = 0; k < kScanRun; k++) {
-            if (i0 + k < n) {
-                start[i0 + k] = run;
-                fill[i0 + k] = run;
-                if (cell_start && ((i0 + k) & 7) == 0) cell_start[(i0 + k) >> 3] = run;
+            for (int k = 0; k < kScanRun; k += 2) {
+                const uint64_t t = load_coherent((const uint64_t *)&count[i0 + k]);
+                v[k] = (int32_t)t;
+                v[k + 1] = (int32_t)(t >> 32);
             }
-            run += v[k];
+        } else {
+#pragma unroll
+            for (int k = 0; k < kScanRun; k++) v[k] = i0 + k < n ? load_coherent(&count[i0 + k]) : 0;
         }
+    };
+    int carry = 0, turn = 0;
+    read(threadIdx.x * kScanRun);
+    for (int base = 0; base < n; base += STEP, turn ^= 1) {
+        const int i0 = base + threadIdx.x * kScanRun;
+        int32_t u[kScanRun], sum = 0;
+#pragma unroll
+        for (int k = 0; k < kScanRun; k++) {
+            u[k] = v[k];
+            sum += u[k];
+        }
+        read(i0 + STEP);
+        int incl = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += t;
+        }
+        if (lane == 63) wsum[turn][w] = incl;
         __syncthreads();
-        if (threadIdx.x == kWrapThreads - 1) carry += part[kWrapThreads - 1];
-        __syncthreads();
+        int run = carry + incl - sum;
+#pragma unroll
+        for (int q = 0; q < NW; q++) {
+            const int t = wsum[turn][q];
+            if (q < w) run += t;
+            carry += t;
+        }
+        if (cell_start && i0 < n) cell_start[i0 >> 3] = run;
+        if (i0 + kScanRun <= n) {
+            int4 o[2];
+            o[0].x = run;
+            o[0].y = o[0].x + u[0];
+            o[0].z = o[0].y + u[1];
+            o[0].w = o[0].z + u[2];
+            o[1].x = o[0].w + u[3];
+            o[1].y = o[1].x + u[4];
+            o[1].z = o[1].y + u[5];
+            o[1].w = o[1].z + u[6];
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                ((int4 *)(start + i0))[h] = o[h];
+                ((int4 *)(fill + i0))[h] = o[h];
+                ((int4 *)(count + i0))[h] = make_int4(0, 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < kScanRun; k++) {
+                if (i0 + k < n) {
+                    start[i0 + k] = run;
+                    fill[i0 + k] = run;
+                    count[i0 + k] = 0;
+                }
+                run += u[k];
+            }
+        }
     }
     if (threadIdx.x == 0) {
         start[n] = carry;
