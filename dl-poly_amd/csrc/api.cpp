@@ -6,6 +6,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "common.h"
@@ -584,16 +585,24 @@ int dlpx_create(const dlpx_params *p, dlpx_ctx **out)
     if (dev_zero(c->stream, c->flags, sizeof(int32_t) * F_WORDS) != hipSuccess) return bail(DLPX_ERR_HIP);
     c->serial = next_serial();
     // host words the GPU writes directly (the displacement maximum of each step)
-    // the second half of h_flags: a copy of the device words
-    auto pinned = [](auto **host, auto **dev, size_t bytes) {
-        return hipHostMalloc((void **)host, bytes, hipHostMallocMapped) == hipSuccess &&
-               hipHostGetDevicePointer((void **)dev, *host, 0) == hipSuccess;
-    };
-    if (!pinned(&c->h_flags, &c->h_flags_dev, sizeof(int32_t) * 2 * F_WORDS) ||
-        !pinned(&c->h_red, &c->h_red_dev, sizeof(double) * kReduceSlots) ||
-        !pinned(&c->h_st, &c->h_st_dev, sizeof(double) * 9 * n) || !pinned(&c->h_t, &c->h_t_dev, sizeof(int32_t) * n) ||
-        !pinned(&c->h_disp, &c->h_disp_dev, sizeof(double) * (n / 64 + 1)))
-        return bail(DLPX_ERR_HIP);
+    // one pinned block (an allocation each would add its 50-100 us to every
+    // context): atom rows, displacements, sums, flags (their second half a copy
+    // of the device words), types
+    {
+        const size_t st = sizeof(double) * 9 * ((n + 3) / 4 * 4), disp = sizeof(double) * (n / 64 + 1),
+                     red = sizeof(double) * kReduceSlots, flags = sizeof(int32_t) * 2 * F_WORDS;
+        if (hipHostMalloc((void **)&c->h_st, st + disp + red + flags + sizeof(int32_t) * n, hipHostMallocMapped) != hipSuccess ||
+            hipHostGetDevicePointer((void **)&c->h_st_dev, c->h_st, 0) != hipSuccess)
+            return bail(DLPX_ERR_HIP);
+        auto part = [&](auto **host, auto **dev, size_t at) {
+            *host = (std::remove_reference_t<decltype(*host)>)((char *)c->h_st + at);
+            *dev = (std::remove_reference_t<decltype(*dev)>)((char *)c->h_st_dev + at);
+        };
+        part(&c->h_disp, &c->h_disp_dev, st);
+        part(&c->h_red, &c->h_red_dev, st + disp);
+        part(&c->h_flags, &c->h_flags_dev, st + disp + red);
+        part(&c->h_t, &c->h_t_dev, st + disp + red + flags);
+    }
     if (p->electrostatics && (r = spme_setup(c))) return bail(r);
     if ((r = scratch_address(c))) return bail(r);
     *out = reinterpret_cast<dlpx_ctx *>(c);
@@ -617,10 +626,6 @@ int dlpx_destroy(dlpx_ctx *ctx)
     for (void *p : dev)
         if (p) (void)hipFree(p);
     if (c->h_st) (void)hipHostFree(c->h_st);
-    if (c->h_t) (void)hipHostFree(c->h_t);
-    if (c->h_disp) (void)hipHostFree(c->h_disp);
-    if (c->h_flags) (void)hipHostFree(c->h_flags);
-    if (c->h_red) (void)hipHostFree(c->h_red);
     for (int k = 0; k < 8; k++)
         if (c->ev[k]) (void)hipEventDestroy(c->ev[k]);
     if (c->fork_ev) (void)hipEventDestroy(c->fork_ev);
