@@ -39,7 +39,7 @@ VALU_PEAK = {lib.FP64: 78.6e12, lib.MIXED: 157.3e12}  # FLOP/s, vector FP64 / FP
 # kernels of each stage (mixed precision, spline order 8, 128^3 mesh), as the
 # stage-timed pass launches them (single-system kernels; resident runs launch
 # the _batch forms of the same bodies)
-KERNELS = {"pair": "k_pair_comb<8, 1024, true>", "spread": "k_spread_cells<float, 8>",
+KERNELS = {"pair": "k_pair_comb<8, 1024, true>", "spread": "k_spread_tiles<float, 8>",
            "fft": "k_plane/k_lines_zconv/k_plane<float, 16, 8>",
            "gather": "k_gather<float, 8>"}
 # the FFT stage's kernels and their launches per stage: x and y passes fused

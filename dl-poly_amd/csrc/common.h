@@ -171,7 +171,7 @@ struct Ctx {
     // resident runs replay one captured step graph (batch.cpp) unless
     // DLPX_GRAPHS=0 or stage timing asks for eager steps
     bool use_graphs = true;
-    bool finish_in_vv2 = false;      // the last evaluation left the reciprocal finish to stage 2
+    bool finish_in_vv2 = false;      // the last evaluation left the reciprocal finish to stage 2 (or the force store)
     bool vdw_force_shift = false;    // vdws%l_force_shift
     bool vdw_direct = false;         // vdws%l_direct: analytic forms per pair
     bool list_subcells = true;       // list build over half-edge subcells (needs >= 3 link cells per axis)
@@ -257,8 +257,8 @@ struct Ctx {
     int32_t *cnt = nullptr;          // cap*G per-lane counts
     int32_t *flags = nullptr;        // [0] overflow lane max, [1] ibig, [3] pairs, [4..5] displacement
                                      // maximum (double bits), [6] workgroups done
-    int32_t *h_flags = nullptr;      // pinned, mapped host words: [0..3] list flags, [4..5] vnl_check,
-                                     // [8..9] displacement maximum of the last md step
+    int32_t *h_flags = nullptr;      // pinned, mapped host words: [0..3] list flags, [8..9] displacement
+                                     // maximum of the last md step; from F_WORDS a copy of the device words
     int32_t *h_flags_dev = nullptr;  // device address of h_flags
 
     // tables on device
