@@ -998,7 +998,10 @@ int dlpx_two_body_forces(dlpx_ctx *ctx, const double cell[9], const dlpx_atoms *
     }
     r = evaluate(c, !c->timing, true);
     c->pp_now = false;
-    if (r) return r;
+    if (r) {
+        (void)hipStreamSynchronize(c->stream);  // the load still reads the pinned rows
+        return r;
+    }
     c->pp_valid = c->per_particle;
     if ((r = store_forces(c, atoms))) return r;
     assemble(c, c->h_red, out);

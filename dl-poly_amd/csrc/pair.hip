@@ -944,6 +944,7 @@ static PairVariant pair_variant(const Ctx *c, int lanes, long natms, size_t &lds
         const bool rel = c->list_coded && c->rel_pairs;
         int threads = comb_threads(c);
         if (threads == kCombThreads) wide_shape(natms, lanes, threads);
+        else lanes = 8;  // the one shape of 512-thread workgroups
         lds = (rel ? sizeof(float4) * 256 : 0) + sizeof(float4) * (size_t)(nt * (nt + 1) / 2) * (c->max_grid + 1) + ktab +
               sizeof(double) * 10 * (kCombThreads / 64);
         PairVariant v{lanes, false, false, false, false, true, rel};

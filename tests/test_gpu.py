@@ -1084,3 +1084,20 @@ def test_long_line_transforms_agree(n, monkeypatch):
                 assert rms_rel(md, ref[1]) <= 10.0 * tol
                 assert abs(r["engcpe"] - ref[0]["engcpe"]) <= etol * abs(ref[0]["engcpe"])
                 assert np.abs(r["stress"] - ref[0]["stress"]).max() <= max(tol, etol) * np.abs(ref[0]["stress"]).max()
+
+
+@pytest.mark.parametrize("lanes", ["4", "16", None])
+def test_pair_workgroups_of_512_threads(lanes, monkeypatch):
+    """DLPX_COMB_THREADS=512 has one shape, 8 lanes to an atom, whatever the
+    lanes asked for: every atom is served (mixed against FP64, 1e-5 RMS)."""
+    s = systems.nacl(ncells=6, kvec=(32, 32, 32), seed=18)
+    monkeypatch.setenv("DLPX_COMB_THREADS", "512")
+    if lanes:
+        monkeypatch.setenv("DLPX_PAIR_LANES", lanes)
+    frc = []
+    for precision in (lib.FP64, lib.MIXED):
+        ctx = lib.Context(s, precision=precision)
+        ctx.link_cell_pairs(s.pos)
+        frc.append(ctx.two_body_forces(s.pos)["frc"])
+        ctx.close()
+    assert rms_rel(frc[1], frc[0]) <= 1e-5
