@@ -325,11 +325,13 @@ constexpr int kCombThreads = 1024;
 constexpr int kWideLanes = 32, kWideMin = 256, kWideMax = 512;  // launches of few atoms, see wide_shape
 
 // A table from global memory into LDS by the whole workgroup, eight loads of
-// a thread in flight at a time.
+// a thread in flight at a time.  A system without vdW interactions has no
+// table rows (n = 0), and then nothing may be read.
 template <typename T>
 __device__ __forceinline__ void table_to_lds(T *__restrict__ dst, const T *__restrict__ src, const int n)
 {
     constexpr int U = 8;
+    if (n <= 0) return;  // uniform
     const int nt = blockDim.x;
     int k = threadIdx.x;
     for (; k + (U - 1) * nt < n; k += U * nt) {

@@ -1101,3 +1101,33 @@ def test_pair_workgroups_of_512_threads(lanes, monkeypatch):
         frc.append(ctx.two_body_forces(s.pos)["frc"])
         ctx.close()
     assert rms_rel(frc[1], frc[0]) <= 1e-5
+
+
+@pytest.mark.parametrize("size", [(5, 5, 5), (8, 8, 17)])
+def test_coulomb_only_system_matches_oracle(size):
+    """Ions without any vdW interaction: no vdW table rows, so the pair kernel
+    has none to load, in both of its launch shapes (32 and 8 lanes to an atom),
+    with and without per-particle output and force-shifting (which keeps mixed
+    precision off the combined tables).  FP64 to 1e-10 of the oracle, mixed to
+    1e-5."""
+    s = systems.nacl(ncells=size, kvec=(32, 32, 32), seed=21)
+    s.vdw = []
+    o = oracle.two_body(s, per_particle=True)
+    for precision, tol, etol in ((lib.FP64, 1e-10, 1e-11), (lib.MIXED, 1e-5, 1e-6)):
+        for pp, shift in ((False, False), (True, False), (False, True)):
+            print("case coulomb only", s.natms, precision, pp, shift, flush=True)
+            s.vdw_force_shift = shift
+            ctx = lib.Context(s, precision=precision)
+            ctx.link_cell_pairs(s.pos)
+            r = ctx.two_body_forces(s.pos, per_particle=pp)
+            ctx.close()
+            assert rms_rel(r["frc"], o["frc"]) <= tol
+            assert r["engsrp"] == 0.0
+            # per-particle output takes the Coulomb virial from the atoms' stresses
+            keys = ("engcpe",) if pp else ("engcpe", "vircpe")
+            sc = energy_scales(o, precision == lib.MIXED)
+            for k in keys:
+                assert abs(r[k] - o[k]) <= etol * max(abs(o[k]), sc[k]), k
+            if pp:
+                assert rms_rel(r["pp_energy"], o["pp_energy"]) <= tol
+                assert rms_rel(r["pp_stress"], o["pp_stress"]) <= tol
