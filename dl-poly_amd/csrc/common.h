@@ -115,8 +115,8 @@ enum Flag : int {
     F_NREB = 8,     // rebuilds decided on the device since the run began
     F_STEP = 9,     // per-step energy records written since the run began
     F_ERR = 10,     // sticky: a list-build kernel met an index outside the atoms (internal error)
-    F_STRAY = 11,   // the last position upload (its number) with an atom further than half the padding
-                    // from its bin of the last list build
+    F_STRAY = 11,   // the last position upload (its number) with an atom further from its place at the list
+                    // build than the tiles' lists allow for
     F_WDONE = 12,   // workgroups of the list binning finished (zero between launches)
     F_WORDS = 16
 };
@@ -472,6 +472,7 @@ int spme_forces(Ctx *c);                     // adds into c->frc and reduction s
 int spme_setup(Ctx *c);
 bool spread_by_tiles(const Ctx *c);          // the context's charges are spread by mesh tiles
 int tile_room(Ctx *c);                       // after a list build: that choice, and the tiles' room
+double tile_reach(const Ctx *c, int d);      // how far an atom may move before the tiles' lists miss it (fraction of the cell)
 int ensure_red_rows(Ctx *c, int rows);
 int reduce_partials(Ctx *c, double *rec = nullptr);  // red -> red_out (device), and rec
 int pair_blocks(const Ctx *c);

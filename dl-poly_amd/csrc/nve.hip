@@ -157,15 +157,15 @@ int freeze_atoms(Ctx *c)
     return 0;
 }
 
-// The test of an upload onto an existing list: whether each atom is still
-// within half the padding of its bin (of the last list build, in fractions of
-// the cell edge), where the tiled spreading looks for it.
+// The test of an upload onto an existing list: whether each atom is still as
+// near its place at the list build as the tiles' lists of the spreading allow
+// for (tile_drift, spme.hip), per axis in fractions of the cell, so that a
+// change of the cell counts too.
 struct StrayArgs {
     const double4 *xref;
-    double L0[3], invL0[3];   // the cell of the list build
-    double invL[3], reach[3]; // the present cell; half the padding as a fraction of its edge
-    int bins[3];
-    int32_t *flag;
+    double invL0[3], invL[3]; // the cell of the list build; the present one
+    double reach[3];
+    int32_t *flag;            // null: no list to hold them to
     int32_t no;
 };
 __device__ __forceinline__ bool strayed(const StrayArgs &a, const double (&x)[3], const double (&x0)[3])
@@ -173,10 +173,9 @@ __device__ __forceinline__ bool strayed(const StrayArgs &a, const double (&x)[3]
     bool out = false;
 #pragma unroll
     for (int d = 0; d < 3; d++) {
-        const double lo = (double)cell_coord(x0[d], a.L0[d], a.invL0[d], a.bins[d]) / (double)a.bins[d];
-        double f = x[d] * a.invL[d] + 0.5 - (lo - a.reach[d]);  // from the reach's lower end
-        f -= floor(f);
-        out = out || f > 1.0 / (double)a.bins[d] + 2.0 * a.reach[d];
+        double f = x[d] * a.invL[d] - x0[d] * a.invL0[d];
+        f -= rint(f);
+        out = out || !(fabs(f) <= a.reach[d]);  // a coordinate that is no number strays
     }
     return out;
 }
@@ -221,7 +220,7 @@ __global__ void __launch_bounds__(kLoadThreads) k_load(LoadArgs a)
         if (a.slot) {
             const double4 q = a.stray.xref[s];
             const double x[3] = {p.x, p.y, p.z}, x0[3] = {q.x, q.y, q.z};
-            if (strayed(a.stray, x, x0)) *a.stray.flag = a.stray.no;
+            if (a.stray.flag && strayed(a.stray, x, x0)) *a.stray.flag = a.stray.no;
             const double dx = min_image_1(p.x, q.x, a.b.L[0], a.b.invL[0]);
             const double dy = min_image_1(p.y, q.y, a.b.L[1], a.b.invL[1]);
             const double dz = min_image_1(p.z, q.z, a.b.L[2], a.b.invL[2]);
@@ -661,14 +660,14 @@ int load_atoms(Ctx *c, bool identity, bool with_vel, bool disp)
     if (!identity) {
         StrayArgs &sa = a.stray;
         sa.xref = c->xref;
-        for (int d = 0; d < 3; d++) {
-            sa.L0[d] = c->list_L[d];
-            sa.invL0[d] = 1.0 / c->list_L[d];
-            sa.invL[d] = c->invL[d];
-            sa.reach[d] = 0.5 * c->prm.padding * c->invL[d] * (1.0 + 1.0e-9) + 1.0e-12;
-            sa.bins[d] = (c->list_coded ? 2 : 1) * c->nc[d];
+        if (c->tile_cap > 0) {
+            for (int d = 0; d < 3; d++) {
+                sa.invL0[d] = 1.0 / c->list_L[d];
+                sa.invL[d] = c->invL[d];
+                sa.reach[d] = tile_reach(c, d);
+            }
+            sa.flag = c->flags + F_STRAY;
         }
-        sa.flag = c->flags + F_STRAY;
         c->upload_no = c->upload_no == INT32_MAX ? 1 : c->upload_no + 1;
         sa.no = c->upload_no;
     }

@@ -453,8 +453,9 @@ __global__ void __launch_bounds__(256) k_splines_batch(const SplineArgs<R> *__re
 // The atoms come from the tile's own list, made when the Verlet list is: every
 // atom of the bins in reach that comes within half the Verlet padding of the
 // tile's reach (its points and S - 1 below them); no atom moves further
-// without a rebuild.  A host that evaluates such positions all the same is
-// noticed at the upload (F_STRAY), and then every atom is tested.  The splines
+// without a rebuild.  A host that evaluates such positions all the same, or in
+// another cell, is noticed at the upload, which holds every atom's displacement
+// against the same bound (F_STRAY), and then every atom is tested.  The splines
 // of a chunk of kTileChunk atoms are laid out in LDS over the tile's points
 // with zeros outside, while the next chunk's are being loaded; each chunk of
 // the list is in y order, so that a wavefront only meets the groups of four
@@ -1227,11 +1228,15 @@ static SpreadArgs<R> spread_args(const Ctx *c)
 {
     return SpreadArgs<R>{c->pos, c->cell_start, c->ncell, spme_params(c), (R *)c->Q};
 }
-// Grid points an atom moves along axis d at most between list builds.
+// How far along axis d an atom of a tile's list may be from its place at the
+// list build, in grid points: half the padding, and 1e-4 points of which the
+// upload's test leaves half to the rounding of either side.
 static double tile_drift(const Ctx *c, int d)
 {
     return 0.5 * c->prm.padding * c->K[d] / c->list_L[d] * (1.0 + 1.0e-6) + 1.0e-4;
 }
+// The largest displacement since then that passes that test, as a fraction of the cell.
+double tile_reach(const Ctx *c, int d) { return (tile_drift(c, d) - 0.5e-4) / c->K[d]; }
 static int tile_slack(const Ctx *c, int d) { return (int)std::ceil(tile_drift(c, d)) + 1; }
 static int tile_blocks(const Ctx *c)
 {

@@ -1131,3 +1131,43 @@ def test_coulomb_only_system_matches_oracle(size):
             if pp:
                 assert rms_rel(r["pp_energy"], o["pp_energy"]) <= tol
                 assert rms_rel(r["pp_stress"], o["pp_stress"]) <= tol
+
+
+@pytest.mark.parametrize("precision,tol", [(lib.FP64, 1e-12), (lib.MIXED, 1e-6)])
+@pytest.mark.parametrize("ncells,kvec", [((5, 5, 5), (32, 32, 32)), ((7, 8, 9), (45, 50, 54))])
+def test_one_atom_moved_within_its_bin(ncells, kvec, precision, tol, monkeypatch):
+    """A trial move without a rebuild: one atom 1, 2 and 3 A along an axis, every
+    other at its place in the list, so that the atom stays in the bin of the
+    list build (it starts in the lowest quarter of a subcell, and one of two
+    link cells is longer still) but reaches mesh tiles that did not list it.
+    The reciprocal energy and forces of a list's second and later evaluations,
+    which spread by tiles, are those by link cells: to 1e-12 in FP64, to the
+    FP32 grid's rounding mixed."""
+    s = systems.nacl(ncells=ncells, kvec=kvec, seed=23)
+    s.vdw = []  # an ion moved onto another adds no vdW force that hides the mesh's
+    L = np.diag(s.cell.reshape(3, 3))
+    nc = np.floor(L / (s.cutoff + s.padding + 1e-6))
+    frac = ((s.pos / L + 0.5) * 2 * nc) % 1.0
+    movers = np.flatnonzero((frac < 0.25).all(1))[:12]
+    assert len(movers) >= 6
+    got = {}
+    for tiles in ("0", "1"):
+        monkeypatch.setenv("DLPX_SPREAD_TILES", tiles)
+        ctx = lib.Context(s, precision=precision)
+        ctx.link_cell_pairs(s.pos)
+        ctx.two_body_forces(s.pos)
+        got[tiles] = []
+        for i in movers:
+            for d in range(3):
+                for step in (1.0, 2.0, 3.0):
+                    p = s.pos.copy()
+                    p[i, d] += step
+                    r = ctx.two_body_forces(p)
+                    got[tiles].append((r["buffer"][9], r["frc"]))
+        got[tiles].append((ctx.two_body_forces(s.pos)["buffer"][9], None))  # and back
+        ctx.close()
+    for k, (a, b) in enumerate(zip(got["1"], got["0"])):
+        print("case moved", ncells, precision, k, a[0] / b[0] - 1.0, flush=True)
+        assert abs(a[0] - b[0]) <= tol * abs(b[0])
+        if a[1] is not None:
+            assert rms_rel(a[1], b[1]) <= tol
