@@ -426,6 +426,25 @@ static int md_begin(Ctx *c, int nsteps, double tstep)
     return nsteps > 0 ? nve_first(c, tstep) : 0;
 }
 
+// Forces at the loaded or restored configuration, from a list of its own:
+// dlpx_md_load's, for a run whose start needs them again.
+static int restart(Ctx *c)
+{
+    int r;
+    if ((r = build_list(c))) return r;
+    if ((r = evaluate(c))) return r;
+    return freeze_atoms(c);
+}
+
+// A run's list belongs to the run's cell: where a force call has changed the
+// cell since the list build, the list is built anew before the first step.
+// Device-decided rebuilds bin in the present cell, so what the host knows of
+// the list (list_L, the link cells of its entries' codes) stays right.
+static int run_list(Ctx *c)
+{
+    return c->list_L[0] == c->L[0] && c->list_L[1] == c->L[1] && c->list_L[2] == c->L[2] ? 0 : restart(c);
+}
+
 // Step s of a host-decided resident run (nve.F90:127-215 with
 // refresh_mappings/vnl_check and the force call, drivers.F90:2105-2199): wait
 // for this context's stage 1, rebuild the list if an atom moved by padding/2,
@@ -463,9 +482,7 @@ static int md_step(Ctx *c, int s, int nsteps, double tstep, bool energies, int &
 int md_fallback(Ctx *c, int nsteps, double tstep, bool energies, int &rebuilds)
 {
     int r;
-    if ((r = build_list(c))) return r;
-    if ((r = evaluate(c))) return r;
-    if ((r = freeze_atoms(c))) return r;
+    if ((r = restart(c))) return r;
     rebuilds = 0;
     if ((r = md_begin(c, nsteps, tstep))) return r;
     for (int s = 0; s < nsteps; s++)
@@ -1121,6 +1138,7 @@ int dlpx_md_run(dlpx_ctx *ctx, int32_t nsteps, double tstep, double *energies, i
     int r, rebuilds = 0;
     if (energies && (r = energies_room(c, nsteps))) return r;
     c->run_dt = tstep;
+    if (nsteps > 0 && (r = run_list(c))) return r;
     if (c->use_graphs && !c->timing) {
         // device-decided rebuilds and captured steps: a batch of one
         std::vector<Ctx *> cs{c};
@@ -1170,6 +1188,7 @@ int dlpx_md_run_ensemble_energies(dlpx_ctx *const *ctxs, int32_t nctx, int32_t n
     bool batched = true;
     for (int k = 0; k < nctx; k++) {
         cs[k]->run_dt = tsteps[k];
+        if (nsteps > 0 && (r = run_list(cs[k]))) return r;
         if (energies && (r = energies_room(cs[k], nsteps))) return r;
         // stage timing on the first context times the batched steps eagerly
         batched = batched && cs[k]->use_graphs && (k == 0 || !cs[k]->timing) &&

@@ -497,7 +497,6 @@ struct TileArgs {
     int fresh;              // so it is
     const int32_t *flags;
     int32_t no;             // upload whose strays matter (F_STRAY), 0: none
-    int all;                // test every atom
     SpmeParams sp;
     R *Q;
 };
@@ -663,7 +662,7 @@ __device__ __forceinline__ void spread_tile_body(const TileArgs<R> &a, int b)
         __syncthreads();
     };
 
-    const bool all = a.all != 0 || (a.no != 0 && a.flags[F_STRAY] == a.no);
+    const bool all = a.no != 0 && a.flags[F_STRAY] == a.no;
     const bool fresh = a.fresh != 0 || (a.upd && *a.upd != 0);
     const int have = fresh || all ? -1 : a.count[b];
     if (have >= 0) {
@@ -1330,8 +1329,6 @@ static TileArgs<R> tile_args(const Ctx *c, int32_t no, const int32_t *upd)
         a.invL0[d] = 1.0 / c->list_L[d];
         a.drift_k[d] = tile_drift(c, d);
         a.slack[d] = tile_slack(c, d);
-        // the lists of another cell than the present one, positions not compared with them
-        if (no == 0 && c->list_L[d] != c->L[d]) a.all = 1;
     }
     a.sp = spme_params(c);
     a.Q = (R *)c->Q;

@@ -1171,3 +1171,45 @@ def test_one_atom_moved_within_its_bin(ncells, kvec, precision, tol, monkeypatch
         assert abs(a[0] - b[0]) <= tol * abs(b[0])
         if a[1] is not None:
             assert rms_rel(a[1], b[1]) <= tol
+
+
+@pytest.mark.parametrize("precision,tol", [(lib.FP64, 1e-9), (lib.MIXED, 1e-5)])
+@pytest.mark.parametrize("graphs,scale", [("0", 1.03), ("1", 1.03), ("1", 1.007)])
+def test_run_in_another_cell_than_the_list(graphs, scale, precision, tol, monkeypatch):
+    """dlpx_md_load, a force call in a cell 0.7 or 3 % longer (the latter five
+    link cells to an axis instead of four) and a run there: the run and its
+    per-step energies are those of the configuration loaded in that cell, and
+    force calls after it, on positions with one atom moved, spread by tiles as
+    by link cells."""
+    monkeypatch.setenv("DLPX_GRAPHS", graphs)
+    s = systems.nacl(ncells=10, kvec=(64, 64, 64), seed=24)
+    pos = s.pos * scale
+    steps, got = 12, {}
+    for name, tiles in (("there", "0"), ("there", "1"), ("loaded", "0")):
+        monkeypatch.setenv("DLPX_SPREAD_TILES", tiles)
+        ctx = lib.Context(s, precision=precision)
+        if name == "there":
+            ctx.md_load(s.pos, s.vel)
+            ctx.cell = ctx.cell * scale
+            ctx.two_body_forces(pos)
+        else:
+            ctx.cell = ctx.cell * scale
+            ctx.md_load(pos, s.vel)
+        e, reb = ctx.md_run(steps, s.timestep)
+        assert reb > 0
+        x, _, f = ctx.md_store()
+        after = []
+        for i in range(0, s.natms, 401):
+            for d in range(3):
+                p = x.copy()
+                p[i, d] += 2.0
+                after.append(ctx.two_body_forces(p)["buffer"][9])
+        ctx.close()
+        got[name, tiles] = (f, e, np.array(after))
+    ref = got["loaded", "0"]
+    for k in (("there", "0"), ("there", "1")):
+        f, e, after = got[k]
+        print("case cell", graphs, scale, precision, k, rms_rel(f, ref[0]), flush=True)
+        assert rms_rel(f, ref[0]) <= tol
+        assert np.abs(e - ref[1]).max() <= tol * np.abs(ref[1]).max()
+        assert np.abs(after - ref[2]).max() <= tol * np.abs(ref[2]).max()
