@@ -285,7 +285,7 @@ struct Ctx {
                                      // between evaluations (the forward x pass clears each line it has read)
     void *spl_z = nullptr, *spl_wq = nullptr;  // the atoms' splines of one evaluation (spme.hip, k_splines)
     ushort4 *spl_base = nullptr;
-    int32_t *tile_list = nullptr;    // atoms of each mesh tile, tile_cap each, then their numbers (spme.hip)
+    int32_t *tile_list = nullptr;    // atoms of each mesh tile, tile_cap each, then two words a tile (spme.hip)
     size_t tile_words = 0;
     int tile_cap = 0;                // 0: the charges are spread by link cells
     int list_evals = 0;              // reciprocal sums since the last host-driven list build
@@ -472,6 +472,8 @@ int spme_forces(Ctx *c);                     // adds into c->frc and reduction s
 int spme_setup(Ctx *c);
 bool spread_by_tiles(const Ctx *c);          // the context's charges are spread by mesh tiles
 int tile_room(Ctx *c);                       // after a list build: that choice, and the tiles' room
+int tile_blocks(const Ctx *c);               // mesh tiles
+int32_t *tile_found(const Ctx *c);           // a word per tile, zero before an evaluation on uploaded positions
 double tile_reach(const Ctx *c, int d);      // how far an atom may move before the tiles' lists miss it (fraction of the cell)
 int ensure_red_rows(Ctx *c, int rows);
 int reduce_partials(Ctx *c, double *rec = nullptr);  // red -> red_out (device), and rec

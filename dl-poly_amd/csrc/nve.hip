@@ -202,6 +202,8 @@ struct LoadArgs {
     unsigned long long *disp;
     Box b;
     StrayArgs stray;
+    int32_t *clear;  // words zeroed for the spreading (k_splines); null: none
+    int nclear;
 };
 constexpr int kLoadThreads = 256;
 __global__ void __launch_bounds__(kLoadThreads) k_load(LoadArgs a)
@@ -209,6 +211,7 @@ __global__ void __launch_bounds__(kLoadThreads) k_load(LoadArgs a)
     __shared__ double wmax[kLoadThreads / 64];
     const int h = blockIdx.x * kLoadThreads + threadIdx.x;
     double r2 = 0.0;
+    for (int k = h; k < a.nclear; k += gridDim.x * kLoadThreads) a.clear[k] = 0;
     if (h < a.n) {
         const int s = a.slot ? a.slot[h] : h;
         const double4 *r = (const double4 *)(a.st + (size_t)a.row * h);
@@ -667,6 +670,8 @@ int load_atoms(Ctx *c, bool identity, bool with_vel, bool disp)
                 sa.reach[d] = tile_reach(c, d);
             }
             sa.flag = c->flags + F_STRAY;
+            a.clear = tile_found(c);
+            a.nclear = tile_blocks(c);
         }
         c->upload_no = c->upload_no == INT32_MAX ? 1 : c->upload_no + 1;
         sa.no = c->upload_no;

@@ -397,6 +397,14 @@ __global__ void __launch_bounds__(spread_threads<R>()) k_spread_cells_batch(cons
 //   D[t] = z[t] - z[t+1]   (z[S] = 0),
 // in [atom][axis][S]; {w_x, w_y, w_z, charge}; and the folded grid points
 // {floor(u_x), floor(u_y), floor(u_z), whether the atom has a charge}.
+//
+// When an atom has moved further than the tiles' lists allow for (F_STRAY), the
+// lists are not used.  Up to kStrayTest atoms every tile then tests every atom;
+// with more, each charged atom is put here on the lists of the tiles that it
+// reaches, by an atomic count per tile (which the upload has cleared), in any
+// order.  A force call on such positions, tested and listed: 4,096 ions, mixed,
+// 127 and 167 us (the counts' atomics, and lists without y order), 21,952 272 and
+// 286, 27,000 286 and 281, 46,656 478 and 375; 1,728,000 ions 116 and 11.1 ms.
 template <typename R> struct R4T;
 template <> struct R4T<double> { using type = double4; };
 template <> struct R4T<float> { using type = float4; };
@@ -407,8 +415,13 @@ struct SplineArgs {
     SpmeParams sp;
     R *z, *wq;
     ushort4 *base;
+    const int32_t *flags;
+    int32_t no;                 // upload whose strays matter (F_STRAY), 0: none
+    int32_t *list, *found;      // the tiles' lists and, for strays, the atoms found for each
+    int cap, tiles[3];
 };
-template <typename R, int S>
+constexpr int kTileX = 16, kTileY = 8, kTileZ = 16;
+template <typename R, int S, bool STRAYS>
 __device__ __forceinline__ void splines_body(const SplineArgs<R> &a, int bid)
 {
     const int k = bid * 256 + threadIdx.x, i = k / 3, d = k - 3 * i;
@@ -428,10 +441,37 @@ __device__ __forceinline__ void splines_body(const SplineArgs<R> &a, int bid)
     if (d == 0) {
         a.wq[4 * (size_t)i + 3] = (R)p.w;
         b[3] = fabs(p.w) > kZeroPlus ? 1 : 0;
+        if (STRAYS && a.no != 0 && a.flags[F_STRAY] == a.no && b[3]) {
+            // the tiles of the atom's S points from floor(u) - S + 1 on, per axis
+            constexpr int T[3] = {kTileX, kTileY, kTileZ}, MT = 2 + (S + 6) / 8;
+            int tl[3][MT], nt[3];
+#pragma unroll
+            for (int x = 0; x < 3; x++) {
+                int g = idx;
+                if (x > 0) grid_coord(a.sp, x, p.x, p.y, p.z, g, w);
+                g -= S - 1;
+                if (g < 0) g += a.sp.K[x];
+                nt[x] = 0;
+                for (int left = S; left > 0 && nt[x] < MT;) {
+                    const int tile = g / T[x], step = min((tile + 1) * T[x], a.sp.K[x]) - g;
+                    tl[x][nt[x]++] = tile;
+                    left -= step;
+                    g += step;
+                    if (g >= a.sp.K[x]) g = 0;
+                }
+            }
+            for (int q2 = 0; q2 < nt[2]; q2++)
+                for (int q1 = 0; q1 < nt[1]; q1++)
+                    for (int q0 = 0; q0 < nt[0]; q0++) {
+                        const int tile = (tl[2][q2] * a.tiles[1] + tl[1][q1]) * a.tiles[0] + tl[0][q0];
+                        const int slot = atomicAdd(&a.found[tile], 1);
+                        if (slot < a.cap) a.list[(size_t)tile * a.cap + slot] = i;
+                    }
+        }
     }
 }
 template <typename R, int S>
-__global__ void __launch_bounds__(256) k_splines(SplineArgs<R> a) { splines_body<R, S>(a, blockIdx.x); }
+__global__ void __launch_bounds__(256) k_splines(SplineArgs<R> a) { splines_body<R, S, true>(a, blockIdx.x); }
 template <typename R, int S>
 __global__ void __launch_bounds__(256) k_splines_batch(const SplineArgs<R> *__restrict__ av,
                                                        const int32_t *__restrict__ boff, int nsys)
@@ -439,7 +479,7 @@ __global__ void __launch_bounds__(256) k_splines_batch(const SplineArgs<R> *__re
     const int lb = blockIdx.x;
     if (lb >= boff[nsys]) return;
     const int s = batch_find(boff, nsys, lb);
-    splines_body<R, S>(av[s], lb - boff[s]);
+    splines_body<R, S, false>(av[s], lb - boff[s]);  // a resident run's atoms never stray
 }
 // Charge spreading by mesh tiles: one workgroup per tile of kTileX x kTileY x
 // kTileZ grid points sums every atom that reaches into it and stores each
@@ -455,8 +495,8 @@ __global__ void __launch_bounds__(256) k_splines_batch(const SplineArgs<R> *__re
 // tile's reach (its points and S - 1 below them); no atom moves further
 // without a rebuild.  A host that evaluates such positions all the same, or in
 // another cell, is noticed at the upload, which holds every atom's displacement
-// against the same bound (F_STRAY), and then every atom is tested.  The splines
-// of a chunk of kTileChunk atoms are laid out in LDS over the tile's points
+// against the same bound (F_STRAY), and then the lists are not used (k_splines).
+// The splines of a chunk of kTileChunk atoms are laid out in LDS over the tile's points
 // with zeros outside, while the next chunk's are being loaded; each chunk of
 // the list is in y order, so that a wavefront only meets the groups of four
 // that reach its planes.
@@ -474,11 +514,11 @@ __global__ void __launch_bounds__(256) k_splines_batch(const SplineArgs<R> *__re
 // (190 registers); 16 planes to a tile: 40 against 34; a wavefront's bounds of
 // 5 per SIMD keep the list making's registers off the rest (1,728,000 ions
 // 593 -> 546).
-constexpr int kTileX = 16, kTileY = 8, kTileZ = 16;
 constexpr int kTileThreads = 256, kTileChunk = 64;
 constexpr int kTilePlanes = kTileY / (kTileThreads / 64);
 constexpr int kTileScan = 2;     // candidates a thread tests per round of a list's making
 constexpr int kTileBins = 1024;  // most bins within a tile's reach
+constexpr int kStrayTest = 24576; // most atoms that every tile tests when some have strayed (k_splines)
 template <typename R>
 struct TileArgs {
     const R *z, *wq;        // the atoms' splines and grid points (k_splines)
@@ -488,6 +528,7 @@ struct TileArgs {
     CellGrid g;             // sub: 1 bins are link cells, 2 subcells
     int bins[3], tiles[3];
     int32_t *list, *count;  // cap atoms per tile; their number, -1 none
+    const int32_t *found;   // of strays, the atoms k_splines found for each tile; null: it looked for none
     int cap;
     const double4 *xref;    // the positions of the list build, in a cell of
     double invL0[3];        // these reciprocal edges
@@ -511,7 +552,7 @@ __device__ __forceinline__ int lanes_before(unsigned long long mask)
 {
     return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
 }
-template <typename R, int S>
+template <typename R, int S, bool STRAYS>
 __device__ __forceinline__ void spread_tile_body(const TileArgs<R> &a, int b)
 {
     typedef double double4v __attribute__((ext_vector_type(4)));
@@ -662,10 +703,13 @@ __device__ __forceinline__ void spread_tile_body(const TileArgs<R> &a, int b)
         __syncthreads();
     };
 
-    const bool all = a.no != 0 && a.flags[F_STRAY] == a.no;
+    // strays: the lists k_splines made, and every atom tested for a tile whose
+    // list they outgrew
+    const bool all = STRAYS && a.no != 0 && a.flags[F_STRAY] == a.no;
     const bool fresh = a.fresh != 0 || (a.upd && *a.upd != 0);
-    const int have = fresh || all ? -1 : a.count[b];
-    if (have >= 0) {
+    const int have = all ? (a.found ? a.found[b] : -1) : fresh ? -1 : a.count[b];
+    if (have >= 0 && (!STRAYS || have <= a.cap)) {
+        if (all && t == 0) a.count[b] = -1;
         sum(have);
     } else {
         // the list made anew, from the bins within reach
@@ -811,7 +855,7 @@ template <typename R, int S>
 __global__ void __launch_bounds__(kTileThreads, 5) k_spread_tiles(TileArgs<R> a)
 {
     const int b = xcd_block(blockIdx.x, gridDim.x);
-    if (b < a.tiles[0] * a.tiles[1] * a.tiles[2]) spread_tile_body<R, S>(a, b);
+    if (b < a.tiles[0] * a.tiles[1] * a.tiles[2]) spread_tile_body<R, S, true>(a, b);
 }
 template <typename R, int S>
 __global__ void __launch_bounds__(kTileThreads, 5) k_spread_tiles_batch(const TileArgs<R> *__restrict__ av,
@@ -819,7 +863,7 @@ __global__ void __launch_bounds__(kTileThreads, 5) k_spread_tiles_batch(const Ti
 {
     BatchPos bp;
     if (!batch_pos(boff, nsys, bp)) return;
-    spread_tile_body<R, S>(av[bp.s], bp.b);
+    spread_tile_body<R, S, false>(av[bp.s], bp.b);
 }
 
 // Lanes per atom in the gather: the next power of two >= S, lane tx < S
@@ -1237,10 +1281,13 @@ static double tile_drift(const Ctx *c, int d)
 // The largest displacement since then that passes that test, as a fraction of the cell.
 double tile_reach(const Ctx *c, int d) { return (tile_drift(c, d) - 0.5e-4) / c->K[d]; }
 static int tile_slack(const Ctx *c, int d) { return (int)std::ceil(tile_drift(c, d)) + 1; }
-static int tile_blocks(const Ctx *c)
+int tile_blocks(const Ctx *c)
 {
     return ceil_div(c->K[0], kTileX) * ceil_div(c->K[1], kTileY) * ceil_div(c->K[2], kTileZ);
 }
+// After the tiles' lists: the number of atoms of each, and of those found for each among strays.
+static int32_t *tile_count(const Ctx *c) { return c->tile_list + (size_t)tile_blocks(c) * c->tile_cap; }
+int32_t *tile_found(const Ctx *c) { return tile_count(c) + tile_blocks(c); }
 // Mesh tiles need a mesh that holds a tile and an atom's reach without
 // meeting itself (an atom then has one image in reach of a tile), and bins
 // not much finer than a tile (kTileBins of them in reach).
@@ -1286,7 +1333,7 @@ int tile_room(Ctx *c)
         0.27 * c->natms / std::min(cells, 256.0) + 5.0)
         return 0;
     const int cap = kTileScan * kTileThreads + (int)(1.3 * mean / 64.0 + 1.0) * 64;
-    const size_t words = (size_t)tile_blocks(c) * (cap + 1);
+    const size_t words = (size_t)tile_blocks(c) * (cap + 2);
     if (words > c->tile_words) {
         if (c->tile_list) (void)hipFree(c->tile_list);
         c->tile_list = nullptr;
@@ -1298,9 +1345,17 @@ int tile_room(Ctx *c)
     return 0;
 }
 template <typename R>
-static SplineArgs<R> spline_args(const Ctx *c)
+static SplineArgs<R> spline_args(const Ctx *c, int32_t no)
 {
-    return SplineArgs<R>{c->pos, c->natms, spme_params(c), (R *)c->spl_z, (R *)c->spl_wq, c->spl_base};
+    SplineArgs<R> a{c->pos, c->natms, spme_params(c), (R *)c->spl_z, (R *)c->spl_wq, c->spl_base};
+    a.flags = c->flags;
+    a.no = c->natms > kStrayTest ? no : 0;
+    a.list = c->tile_list;
+    a.found = tile_found(c);
+    a.cap = c->tile_cap;
+    const int T[3] = {kTileX, kTileY, kTileZ};
+    for (int d = 0; d < 3; d++) a.tiles[d] = ceil_div(c->K[d], T[d]);
+    return a;
 }
 static int spline_blocks(const Ctx *c) { return ceil_div(3L * c->natms, 256); }
 template <typename R>
@@ -1316,7 +1371,8 @@ static TileArgs<R> tile_args(const Ctx *c, int32_t no, const int32_t *upd)
     a.start = c->list_coded ? c->key_start : c->cell_start;
     a.list = c->tile_list;
     a.cap = c->tile_cap;
-    a.count = c->tile_list + (size_t)tile_blocks(c) * c->tile_cap;
+    a.count = tile_count(c);
+    a.found = c->natms > kStrayTest ? tile_found(c) : nullptr;
     a.xref = c->xref;
     a.upd = upd;
     a.fresh = c->tile_lists ? 0 : 1;
@@ -1381,7 +1437,7 @@ static int spme_run(Ctx *c)
     const bool tiles = spread_by_tiles(c);
     c->list_evals++;
     if (tiles) {
-        const SplineArgs<R> sa = spline_args<R>(c);
+        const SplineArgs<R> sa = spline_args<R>(c, c->stray_no);
 #define DLPX_SPLINES(SS) hipLaunchKernelGGL((k_splines<R, SS>), dim3(spline_blocks(c)), dim3(256), 0, s, sa)
         DLPX_S_SWITCH(sp.S, DLPX_SPLINES)
 #undef DLPX_SPLINES
@@ -1463,7 +1519,7 @@ static int spme_prepare_t(const std::vector<Ctx *> &cs, SpmeBatch &sb)
             if ((r = grid_zero<R>(c, c->stream))) return r;
             DLPX_HIP(c, hipStreamSynchronize(c->stream));
         }
-        sa.push_back(tiles ? spline_args<R>(c) : SplineArgs<R>{});
+        sa.push_back(tiles ? spline_args<R>(c, 0) : SplineArgs<R>{});
         nbp.push_back(tiles ? spline_blocks(c) : 0);
         spa.push_back(on && !tiles ? spread_args<R>(c) : SpreadArgs<R>{});
         ta.push_back(tiles ? tile_args<R>(c, 0, c->flags + F_UPD) : TileArgs<R>{});

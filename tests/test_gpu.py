@@ -1213,3 +1213,34 @@ def test_run_in_another_cell_than_the_list(graphs, scale, precision, tol, monkey
         assert rms_rel(f, ref[0]) <= tol
         assert np.abs(e - ref[1]).max() <= tol * np.abs(ref[1]).max()
         assert np.abs(after - ref[2]).max() <= tol * np.abs(ref[2]).max()
+
+
+@pytest.mark.parametrize("ncells,order,kvec", [(10, 4, (64, 64, 64)), (10, 8, (50, 45, 54)), (10, 16, (64, 45, 54)),
+                                               (15, 4, (50, 45, 54)), (15, 8, (96, 90, 100)), (15, 16, (64, 45, 54))])
+def test_moved_atoms_beyond_a_tiles_room(ncells, order, kvec, monkeypatch):
+    """Positions further from the list's than the tiles' lists allow for, with
+    8,000 ions (every tile tests every atom) and 27,000 (lists from where the
+    atoms are), at meshes of whole and partial tiles.  A droplet, whose tiles hold more atoms than
+    their room, and the same ions over the whole box, most of them charged and
+    one in seven not.  FP64 against the spreading by link cells, to rounding."""
+    s = systems.nacl(ncells=ncells, kvec=kvec, nsplines=order, seed=25)
+    s.cutoff = s.vdw_cutoff = 6.0
+    s.vdw = []
+    rng = np.random.default_rng(26)
+    wide = s.pos + rng.uniform(-2.0, 2.0, s.pos.shape)
+    drop = s.pos * 0.4 - 0.25 * s.cell[0]
+    far = drop + rng.uniform(-2.0, 2.0, s.pos.shape)
+    got = {}
+    for tiles in ("1", "0"):
+        monkeypatch.setenv("DLPX_SPREAD_TILES", tiles)
+        ctx = lib.Context(s, precision=lib.FP64)
+        ctx.q = np.where(np.arange(s.natms) % 7 == 0, 0.0, ctx.q)
+        got[tiles] = []
+        for at, to in ((s.pos, wide), (drop, far)):
+            ctx.link_cell_pairs(at)
+            got[tiles] += [ctx.two_body_forces(p) for p in (at, to, at, to)]
+        ctx.close()
+    for k, (a, b) in enumerate(zip(got["1"], got["0"])):
+        print("case strays", ncells, order, kvec, k, a["buffer"][9] / b["buffer"][9] - 1.0, flush=True)
+        assert rms_rel(a["frc"], b["frc"]) <= 1e-12
+        assert abs(a["buffer"][9] - b["buffer"][9]) <= 1e-12 * abs(b["buffer"][9])
