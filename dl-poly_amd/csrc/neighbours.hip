@@ -329,7 +329,7 @@ __device__ __forceinline__ void sort_permute_body(const SortArgs &a, int c)
 // image shift is -L, 0 or +L per axis.  The separation is x_i - (x_j + s L)
 // and the criterion r^2 <= (cutoff+padding)^2 (neighbours.F90:991-992).  A
 // single-precision distance settles every pair that is clearly inside or
-// outside; pairs within a relative 2e-5 of the cutoff are decided in double
+// outside; pairs within its error of the cutoff (filter_band) are decided in double
 // precision without fused multiply-add from the FP64 positions, with the
 // arithmetic of the host, so the accepted set is reproducible bit for bit.
 // With fewer than 3 cells on an axis the stencil shift need not be the
@@ -361,6 +361,7 @@ struct BuildArgs {
     CellGrid g;
     const int32_t *start;  // link-cell starts (k_build_list) or subcell-key starts (k_build_list_sub)
     double rc2;
+    float rc2_lo, rc2_hi;  // between them the FP32 distance does not decide (filter_band)
     int cap_lane;
     int32_t *nbr, *cnt, *flags;
     const int32_t *upd;
@@ -418,7 +419,7 @@ __device__ __forceinline__ void build_list_body(const BuildArgs &a, int b)
     __syncthreads();
     const int ncand = s_off[27];
     const int hs = start[c], nat = start[c + 1] - hs;
-    const float rc2_lo = (float)(rc2 * (1.0 - 2.0e-5)), rc2_hi = (float)(rc2 * (1.0 + 2.0e-5));
+    const float rc2_lo = a.rc2_lo, rc2_hi = a.rc2_hi;
     const float Lf[3] = {(float)g.L[0], (float)g.L[1], (float)g.L[2]};
     const float iLf[3] = {(float)g.invL[0], (float)g.invL[1], (float)g.invL[2]};
     for (int a0 = 0; a0 < nat; a0 += kListAtomChunk) {
@@ -526,7 +527,7 @@ __device__ __forceinline__ void build_list_body(const BuildArgs &a, int b)
 // entries, so the loops and the list counter are wavefront-uniform.  Entry e
 // of atom i sits at list_slot(i, e / G, e % G), the layout of the link-cell
 // build, and list lane g then holds entries e = g, g + G, ...  The accept
-// test (FP32 filter, FP64 decision within 2e-5 of the cutoff) is the link-cell
+// test (FP32 filter, FP64 decision within its error) is the link-cell
 // build's, so both give the same set.
 //
 // Bound by instruction issue, and the scalar unit, which the four SIMDs of a
@@ -614,7 +615,7 @@ __device__ __forceinline__ void build_list_sub_body(const BuildArgs &a, int lb)
     const int ncand = s_off[kSubStencil];
     const int hs = s_lo[0], nat = s_lo[8] - hs;
     const int cap_tot = cap_lane * G;
-    const float rc2_lo = (float)(rc2 * (1.0 - 2.0e-5)), rc2_hi = (float)(rc2 * (1.0 + 2.0e-5));
+    const float rc2_lo = a.rc2_lo, rc2_hi = a.rc2_hi;
     for (int a0 = 0; a0 < nat; a0 += kListAtomChunk) {
         const int a1 = min(nat, a0 + kListAtomChunk);
         for (int r0 = 0; r0 < ncand; r0 += kListStage) {
@@ -1014,6 +1015,25 @@ struct ListChain {
     int n, ncell, nkey, nbuild;
 };
 
+// The relative error of a squared FP32 distance near the cutoff, with a margin:
+// at least 2e-5, and more in long cells.  A separation's error on axis d is at
+// most 2^-24 of the numbers rounded on the way to it: two coordinates, each up
+// to L/2 and the candidate's a stencil (two cells) beyond, and their difference,
+// up to three cells; with fewer than three cells on an axis the difference, up
+// to L, its image's, up to L/2, and the cell edge.  Twice the separation error
+// over the cutoff is that of the square, and a few roundings of its own.  (2e-5
+// covers cubic cells to about 90 cutoffs, for instance 1,100 A.)
+static double filter_band(const Ctx *c, double rc)
+{
+    const bool small = c->nc[0] < 3 || c->nc[1] < 3 || c->nc[2] < 3;
+    double a2 = 0.0;
+    for (int d = 0; d < 3; d++) {
+        const double a = small ? 3.5 * c->L[d] : c->L[d] * (1.0 + 5.0 / c->nc[d]);
+        a2 += a * a;
+    }
+    return std::max(2.0e-5, 0x1p-23 * std::sqrt(a2) / rc + 0x1p-21);
+}
+
 static int list_chain(Ctx *c, const int32_t *upd, ListChain &lc, int nsys = 1)
 {
     const int n = c->natms;
@@ -1067,13 +1087,15 @@ static int list_chain(Ctx *c, const int32_t *upd, ListChain &lc, int nsys = 1)
     lc.sort = SortArgs{c->perm,    kstart, nkey,   n,      upd,     c->flags,
                        c->pos_alt, c->pos, c->typ_alt, c->typ, c->gid_alt, c->gid,
                        res ? c->vel_alt : nullptr, res ? c->vel : nullptr, c->slot, c->xref};
+    const double rc2 = rc_ext * rc_ext, band = filter_band(c, rc_ext);
     // several workgroups per link cell, each staging the cell's surroundings for
     // some of its atoms, where the cells are too few to fill the GPU (with the
     // other systems of a batch), down to an atom per wavefront; at 512 of them
     // every CU has two.  One and several: 2,592 atoms in 27 cells 66 and 24 us,
     // 10,296 in 120 cells 87 and 40, 4,000 in 216 cells 25 and 20.
     const int parts = std::max(1, std::min(512 / (ncell * nsys), ceil_div(n, 8 * ncell)));
-    lc.build = BuildArgs{c->pos, g, sub ? c->key_start : c->cell_start, rc_ext * rc_ext, c->cap_lane,
+    lc.build = BuildArgs{c->pos, g, sub ? c->key_start : c->cell_start, rc2, (float)(rc2 * (1.0 - band)),
+                         (float)(rc2 * (1.0 + band)), c->cap_lane,
                          c->nbr, c->cnt, c->flags, upd, c->sub_of, parts};
     lc.nbuild = ncell * parts;
     c->list_coded = sub;

@@ -1244,3 +1244,34 @@ def test_moved_atoms_beyond_a_tiles_room(ncells, order, kvec, monkeypatch):
         print("case strays", ncells, order, kvec, k, a["buffer"][9] / b["buffer"][9] - 1.0, flush=True)
         assert rms_rel(a["frc"], b["frc"]) <= 1e-12
         assert abs(a["buffer"][9] - b["buffer"][9]) <= 1e-12 * abs(b["buffer"][9])
+
+
+@pytest.mark.parametrize("edge,subcells", [(26.0, "1"), (40.0, "1"), (40.0, "0")])
+def test_pair_set_in_a_long_cell(edge, subcells, monkeypatch):
+    """A cell of edge x edge x 6,000 A (two and four link cells on the short
+    axes, 631 on the long one), where FP32 coordinates are 2e-4 A apart: atoms
+    in pairs whose distances lie within 1.2e-4 of the cutoff with padding,
+    relative, in any direction and across every face.  The pair set is the one
+    of FP64 distances."""
+    monkeypatch.setenv("DLPX_LIST_SUBCELLS", subcells)
+    rng = np.random.default_rng(27)
+    L = np.array([edge, edge, 6000.0])
+    n, rc = 3000, 9.5
+    base = rng.uniform(-0.5, 0.5, (n, 3)) * L
+    base[: n // 3, 2] = np.sign(base[: n // 3, 2]) * (3000.0 - rng.uniform(0.0, 6.0, n // 3))  # at the long axis's faces
+    u = rng.normal(size=(n, 3)) * (0.3, 0.3, 1.0)
+    u /= np.linalg.norm(u, axis=1)[:, None]
+    other = base + u * (rc * (1.0 + rng.uniform(-1.2e-4, 1.2e-4, n)))[:, None]
+    s = systems.argon(ncells=10)
+    s.pos = np.stack([base, other], 1).reshape(-1, 3)
+    s.pos = s.pos - L * np.floor(s.pos / L + 0.5)
+    s.vel, s.types = np.zeros_like(s.pos), np.zeros(2 * n, np.int32)
+    s.cell = np.diag(L).reshape(9)
+    s.cutoff = s.vdw_cutoff = rc - s.padding
+    ctx = lib.Context(s, precision=lib.FP64)
+    ctx.link_cell_pairs(s.pos)
+    got = {tuple(p[:2]) for p in ctx.get_pairs()}
+    ctx.close()
+    want = {tuple(p[:2]) for p in oracle.pairs(s.cell, s.pos, rc, "brute")}
+    print("case long cell", edge, subcells, len(got), len(want), len(got ^ want), flush=True)
+    assert not got ^ want
