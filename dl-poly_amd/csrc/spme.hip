@@ -1308,8 +1308,21 @@ static bool tiles_fit(const Ctx *c)
 // evaluation spreads by link cells, the next by tiles (4,000 atoms of three
 // species on 36^3: 14 us by cells, 32 by tiles with the making of the lists).
 bool spread_by_tiles(const Ctx *c) { return c->tile_cap > 0 && (c->resident || c->tile_lists || c->list_evals > 0); }
+// How much denser than the mean the atoms are where they are densest, from the
+// largest neighbour count of the list build: 1 for fluids and solids that fill
+// the cell, more for slabs and droplets.
+static double crowding(const Ctx *c)
+{
+    const double rc = c->prm.cutoff + c->prm.padding, mean = c->natms / (c->L[0] * c->L[1] * c->L[2]);
+    const double r = (c->h_flags[F_IBIG] + 1) / (4.0 / 3.0 * kPi * rc * rc * rc * mean);
+    return r <= 1.3 ? 1.0 : r;
+}
 // After a list build: whether the charges are spread by tiles, and room for
-// the tiles' lists (1.3 times the mean, and one round of their making).
+// the tiles' lists: 1.3 times the mean where the atoms are densest (a list that
+// outgrows its room is made anew at every evaluation: 7,200 ions in an eighth of
+// their cell, 72 x 60 x 72, S = 8 FP64, 70 us instead of 46), in steps of sqrt(2)
+// so that the configurations of one system get the same room and captured
+// graphs, and one round of their making.
 // Where the mesh allows, the faster of the two by their measured times: a
 // tile's workgroup takes 1.35 us for each chunk of its atoms, one by link
 // cells 0.27 us for each atom of its cell, the busiest CU sets the time, and
@@ -1332,7 +1345,8 @@ int tile_room(Ctx *c)
         1.35 * chunks * std::max(1.0, tile_blocks(c) / 256.0) + 3.5 >
         0.27 * c->natms / std::min(cells, 256.0) + 5.0)
         return 0;
-    const int cap = kTileScan * kTileThreads + (int)(1.3 * mean / 64.0 + 1.0) * 64;
+    const double crowd = crowding(c), steps = crowd > 1.0 ? std::exp2(0.5 * std::ceil(2.0 * std::log2(crowd))) : 1.0;
+    const int cap = kTileScan * kTileThreads + (int)(1.3 * std::min<double>(c->natms, mean * steps) / 64.0 + 1.0) * 64;
     const size_t words = (size_t)tile_blocks(c) * (cap + 2);
     if (words > c->tile_words) {
         if (c->tile_list) (void)hipFree(c->tile_list);
