@@ -1317,19 +1317,57 @@ static double crowding(const Ctx *c)
     const double r = (c->h_flags[F_IBIG] + 1) / (4.0 / 3.0 * kPi * rc * rc * rc * mean);
     return r <= 1.3 ? 1.0 : r;
 }
+// Estimated times (us) of the spreading by mesh tiles (atoms: in the densest
+// tile's reach) and by link cells: a start; what the busiest workgroup takes
+// (a tile for each chunk of its atoms; a cell for each of its atoms, over the
+// 64-lane passes of an atom's S x S columns and again for each further slab of its
+// window, and for its window's points); and the whole's throughput.  Fitted to
+// 4,447 measured pairs of systems of 400 to 150,000 ions at every spline order, on
+// meshes of 0.35 to 1.8 points to the A, cutoffs of 8 to 12 A, filling the cell or
+// as slabs and droplets: nine of ten within 0.75 to 1.17 of the time measured by
+// tiles and 0.64 to 1.27 of that by cells.  A tile's chunk is then charged 0.4 +
+// 0.006 S^2 us more, for its share of the lists' making (1.5 us a chunk at each
+// rebuild) and of the CUs beside the pair kernel.
+static double tiles_us(const Ctx *c, double atoms)
+{
+    const bool mixed = c->prm.precision == DLPX_MIXED;
+    const double S = c->prm.nsplines, chunks = std::ceil(atoms / kTileChunk), perCU = tile_blocks(c) / 256.0;
+    return mixed ? 11.0 + 1.31e-5 * S * std::sqrt(S) * c->natms + (0.43 + 0.032 * S) * perCU +
+                       (1.44 + 0.0089 * S * S) * chunks
+                 : 11.0 + 1.58e-5 * S * std::sqrt(S) * c->natms + (0.51 + 0.056 * S) * perCU +
+                       (1.27 + 0.0125 * S * S) * chunks;
+}
+static double cells_us(const Ctx *c, double crowd)
+{
+    const bool mixed = c->prm.precision == DLPX_MIXED;
+    const double S = c->prm.nsplines, passes = std::ceil(S * S / 64.0);
+    double ext[3];
+    for (int d = 0; d < 3; d++) ext[d] = (double)c->K[d] / c->nc[d] + S;
+    const double window = ext[0] * ext[1] * ext[2];
+    const double planes = std::max(1.0, std::floor(kSlabBytes / sizeof(double) / (ext[0] * ext[1])));
+    const double slabs = std::ceil(ext[2] / std::min(planes, ext[2]));
+    const double atoms = (double)c->natms / c->ncell * crowd, perCU = c->ncell / 256.0;
+    const double points = perCU / crowd * window, each = S * passes * c->natms / 256.0;
+    return mixed ? 5.75 + 0.0175 * S * passes * atoms + 0.308e-3 * window + 0.0051 * S * atoms * (slabs - 1.0) +
+                       0.0085 * each + 0.464e-3 * points + passes * perCU * (0.503 + 0.75 / crowd)
+                 : 6.8 + 0.0250 * S * passes * atoms + 0.410e-3 * window + 0.0109 * S * atoms * (slabs - 1.0) +
+                       0.0083 * each + 0.571e-3 * points + passes * perCU * (0.55 + 1.63 / crowd);
+}
 // After a list build: whether the charges are spread by tiles, and room for
 // the tiles' lists: 1.3 times the mean where the atoms are densest (a list that
 // outgrows its room is made anew at every evaluation: 7,200 ions in an eighth of
 // their cell, 72 x 60 x 72, S = 8 FP64, 70 us instead of 46), in steps of sqrt(2)
 // so that the configurations of one system get the same room and captured
 // graphs, and one round of their making.
-// Where the mesh allows, the faster of the two by their measured times: a
-// tile's workgroup takes 1.35 us for each chunk of its atoms, one by link
-// cells 0.27 us for each atom of its cell, the busiest CU sets the time, and
-// they start from 3.5 us (the splines' kernel) and 5.  Many tiles or none on
-// a CU, tiles win by their lower rate; few atoms in many link cells and many
-// in few tiles (a coarse mesh) are the other case: 4,000 atoms on 36^3, 216
-// cells and 45 tiles, 14 us by cells and 21 by tiles.
+// Where the mesh allows, the faster of the two by their estimates: over the
+// resident steps of 1,877 such systems with either, 0.4 % of the time is lost to
+// the faster choice, and 9 steps are more than 3 % (11 % at most) slower by tiles
+// than by cells.  (Without the order, the precision and the crowding in it: 2 %,
+// and 160.)  Few atoms to a tile (fine meshes) are the tiles': 64,000 ions on 128^3
+// at order 4, 8 and 16, mixed, 33, 52 and 474 us by cells and 22, 34 and 81 by
+// tiles.  Many, or a part of the cell crowded, are the cells': the same on 64^3 20,
+// 35 and 292 and 35, 75 and 226; 8,000 ions on 36^3 at order 8 in FP64 32 and 56;
+// the 7,200 ions above 31 and 46.
 int tile_room(Ctx *c)
 {
     c->tile_cap = 0;
@@ -1340,12 +1378,9 @@ int tile_room(Ctx *c)
     double mean = c->natms;
     for (int d = 0; d < 3; d++)
         mean *= std::min(1.0, (T[d] + c->prm.nsplines - 1 + 2.0 * tile_drift(c, d)) / c->K[d]);
-    const double chunks = mean / kTileChunk, cells = std::max(1, c->ncell);
-    if (c->spread_tiles < 0 &&
-        1.35 * chunks * std::max(1.0, tile_blocks(c) / 256.0) + 3.5 >
-        0.27 * c->natms / std::min(cells, 256.0) + 5.0)
-        return 0;
-    const double crowd = crowding(c), steps = crowd > 1.0 ? std::exp2(0.5 * std::ceil(2.0 * std::log2(crowd))) : 1.0;
+    const double crowd = crowding(c), most = std::min<double>(c->natms, mean * crowd);
+    if (c->spread_tiles < 0 && tiles_us(c, most) > cells_us(c, crowd)) return 0;
+    const double steps = crowd > 1.0 ? std::exp2(0.5 * std::ceil(2.0 * std::log2(crowd))) : 1.0;
     const int cap = kTileScan * kTileThreads + (int)(1.3 * std::min<double>(c->natms, mean * steps) / 64.0 + 1.0) * 64;
     const size_t words = (size_t)tile_blocks(c) * (cap + 2);
     if (words > c->tile_words) {
