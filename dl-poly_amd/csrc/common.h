@@ -471,7 +471,7 @@ int excl_blocks(const Ctx *c);
 int spme_forces(Ctx *c);                     // adds into c->frc and reduction slots
 int spme_setup(Ctx *c);
 bool spread_by_tiles(const Ctx *c);          // the context's charges are spread by mesh tiles
-int tile_room(Ctx *c);                       // after a list build: that choice, and the tiles' room
+void tile_room(Ctx *c);                      // after a list build: that choice, and the tiles' room
 int tile_blocks(const Ctx *c);               // mesh tiles
 int32_t *tile_found(const Ctx *c);           // a word per tile, zero before an evaluation on uploaded positions
 double tile_reach(const Ctx *c, int d);      // how far an atom may move before the tiles' lists miss it (fraction of the cell)

@@ -1191,7 +1191,8 @@ int build_list(Ctx *c)
     c->have_list = true;
     for (int d = 0; d < 3; d++) c->list_L[d] = c->L[d];
     c->stray_no = 0;
-    return tile_room(c);
+    tile_room(c);
+    return 0;
 }
 
 // Batched list builds of an ensemble, each gated by its context's device

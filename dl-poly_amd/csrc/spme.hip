@@ -1217,9 +1217,6 @@ int spme_setup(Ctx *c)
     DLPX_HIP(c, hipMalloc(&c->theta, 2 * rs * c->nhalf));
     DLPX_HIP(c, dev_zero(c->stream, c->theta, 2 * rs * c->nhalf));  // the row padding stays zero
     c->theta_valid = false;
-    DLPX_HIP(c, hipMalloc(&c->spl_z, rs * 3 * S * (size_t)c->cap));
-    DLPX_HIP(c, hipMalloc(&c->spl_wq, rs * 4 * (size_t)c->cap));
-    DLPX_HIP(c, hipMalloc((void **)&c->spl_base, sizeof(ushort4) * (size_t)c->cap));
     const int ksum = c->K[0] + c->K[1] + c->K[2];
     std::vector<double> n2(ksum);
     bspline_norm2(c->K[0], S, n2.data());
@@ -1368,18 +1365,27 @@ static double cells_us(const Ctx *c, double crowd)
 // tiles.  Many, or a part of the cell crowded, are the cells': the same on 64^3 20,
 // 35 and 292 and 35, 75 and 226; 8,000 ions on 36^3 at order 8 in FP64 32 and 56;
 // the 7,200 ions above 31 and 46.
-int tile_room(Ctx *c)
+// The room, and that of the splines, is taken when the tiles first need it (332 MB
+// at 1,728,000 ions in FP64 at order 8); without memory for it the cells are there.
+void tile_room(Ctx *c)
 {
+    auto room = [](auto **p, size_t bytes) {
+        if (!*p && hipMalloc((void **)p, bytes) != hipSuccess) {
+            *p = nullptr;
+            (void)hipGetLastError();
+        }
+        return *p != nullptr;
+    };
     c->tile_cap = 0;
     c->tile_lists = false;
     c->list_evals = 0;
-    if (!tiles_fit(c)) return 0;
+    if (!tiles_fit(c)) return;
     const int T[3] = {kTileX, kTileY, kTileZ};
     double mean = c->natms;
     for (int d = 0; d < 3; d++)
         mean *= std::min(1.0, (T[d] + c->prm.nsplines - 1 + 2.0 * tile_drift(c, d)) / c->K[d]);
     const double crowd = crowding(c), most = std::min<double>(c->natms, mean * crowd);
-    if (c->spread_tiles < 0 && tiles_us(c, most) > cells_us(c, crowd)) return 0;
+    if (c->spread_tiles < 0 && tiles_us(c, most) > cells_us(c, crowd)) return;
     const double steps = crowd > 1.0 ? std::exp2(0.5 * std::ceil(2.0 * std::log2(crowd))) : 1.0;
     const int cap = kTileScan * kTileThreads + (int)(1.3 * std::min<double>(c->natms, mean * steps) / 64.0 + 1.0) * 64;
     const size_t words = (size_t)tile_blocks(c) * (cap + 2);
@@ -1387,11 +1393,13 @@ int tile_room(Ctx *c)
         if (c->tile_list) (void)hipFree(c->tile_list);
         c->tile_list = nullptr;
         c->tile_words = 0;
-        DLPX_HIP(c, hipMalloc((void **)&c->tile_list, sizeof(int32_t) * words));
+        if (!room(&c->tile_list, sizeof(int32_t) * words)) return;
         c->tile_words = words;
     }
-    c->tile_cap = cap;
-    return 0;
+    const size_t rs = c->prm.precision == DLPX_MIXED ? sizeof(float) : sizeof(double), n = c->cap;
+    if (room(&c->spl_z, rs * 3 * c->prm.nsplines * n) && room(&c->spl_wq, rs * 4 * n) &&
+        room(&c->spl_base, sizeof(ushort4) * n))
+        c->tile_cap = cap;
 }
 template <typename R>
 static SplineArgs<R> spline_args(const Ctx *c, int32_t no)

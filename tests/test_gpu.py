@@ -1275,3 +1275,31 @@ def test_pair_set_in_a_long_cell(edge, subcells, monkeypatch):
     want = {tuple(p[:2]) for p in oracle.pairs(s.cell, s.pos, rc, "brute")}
     print("case long cell", edge, subcells, len(got), len(want), len(got ^ want), flush=True)
     assert not got ^ want
+
+
+def test_memory_of_the_splines_only_for_tiles(monkeypatch):
+    """A context that spreads by link cells holds no splines of its atoms (3 S
+    + 4 reals and 8 bytes an atom): device memory in use after a list build,
+    by tiles and by cells."""
+    import ctypes
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0
+        return f.value
+
+    s = systems.nacl(ncells=30, kvec=(128, 128, 128), seed=28)
+    used = {}
+    for tiles in ("0", "1", "0", "1"):  # the first two load the kernels
+        monkeypatch.setenv("DLPX_SPREAD_TILES", tiles)
+        before = free()
+        ctx = lib.Context(s, precision=lib.FP64)
+        ctx.link_cell_pairs(s.pos)
+        for _ in range(3):
+            ctx.two_body_forces(s.pos)
+        used[tiles] = before - free()
+        ctx.close()
+    splines = s.natms * (8 * (3 * 8 + 4) + 8)
+    print("case memory", s.natms, used, splines, flush=True)
+    assert used["1"] - used["0"] >= splines
