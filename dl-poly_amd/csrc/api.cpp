@@ -163,6 +163,14 @@ int upload_tables(Ctx *c)
     return c->noalloc_now ? 0 : upload_comb(c);
 }
 
+// Wait for the stream; the pinned rows are the host's again.
+static int settle(Ctx *c)
+{
+    DLPX_HIP(c, hipStreamSynchronize(c->stream));
+    c->rows_busy = false;
+    return 0;
+}
+
 // host arrays (strided) -> pinned staging -> cell order.  With disp the
 // displacements since the list build go to h_disp.
 static int upload(Ctx *c, const dlpx_atoms *a, bool identity, const double *vx, const double *vy, const double *vz,
@@ -175,6 +183,8 @@ static int upload(Ctx *c, const dlpx_atoms *a, bool identity, const double *vx, 
     auto at = [st](const double *p, int i) { return *(const double *)((const char *)p + (size_t)st * i); };
     auto atv = [vst](const double *p, int i) { return *(const double *)((const char *)p + (size_t)vst * i); };
     const int row = vx ? 8 : 4;
+    int r;
+    if (c->rows_busy && (r = settle(c))) return r;  // a call that failed has not waited for its load
     // charge per atom type, for the pair kernel's combined-table path
     std::vector<double> tq(c->prm.ntypes, 0.0);
     std::vector<char> seen(c->prm.ntypes, 0);
@@ -368,7 +378,8 @@ static void assemble(Ctx *c, const double *red, dlpx_two_body_out *o)
 // Wait for an evaluation with fetch: h_red holds its sums.
 static int fetch_red(Ctx *c)
 {
-    DLPX_HIP(c, hipStreamSynchronize(c->stream));
+    int r;
+    if ((r = settle(c))) return r;
     return collect_timing(c);
 }
 
@@ -883,8 +894,7 @@ int dlpx_add_per_particle(dlpx_ctx *ctx, double *energy, double *stress)
                                                : 0.0;
     const double share = (c->prm.electrostatics ? c->self_energy : 0.0) / n + c->elrc / n;
     int r;
-    if ((r = store_per_particle(c, scale))) return r;
-    DLPX_HIP(c, hipStreamSynchronize(c->stream));
+    if ((r = store_per_particle(c, scale)) || (r = settle(c))) return r;
     const int sym[9] = {0, 1, 2, 1, 3, 4, 2, 4, 5};  // 3x3 element -> (xx, xy, xz, yy, yz, zz)
     for (int h = 0; h < n; h++) {
         const double *p = c->h_st + (size_t)7 * h;
@@ -976,8 +986,7 @@ int dlpx_vnl_check(dlpx_ctx *ctx, const dlpx_atoms *atoms, int32_t *update)
         return 0;
     }
     int r;
-    if ((r = upload(c, atoms, false, nullptr, nullptr, nullptr, nullptr, 0, true))) return r;
-    DLPX_HIP(c, hipStreamSynchronize(c->stream));
+    if ((r = upload(c, atoms, false, nullptr, nullptr, nullptr, nullptr, 0, true)) || (r = settle(c))) return r;
     // the largest of the workgroups' maxima, as bit patterns
     uint64_t b = 0;
     for (int k = 0; k < load_blocks(c); k++) b = std::max(b, bits(c->h_disp[k]));
@@ -1015,10 +1024,7 @@ int dlpx_two_body_forces(dlpx_ctx *ctx, const double cell[9], const dlpx_atoms *
     }
     r = evaluate(c, !c->timing, true);
     c->pp_now = false;
-    if (r) {
-        (void)hipStreamSynchronize(c->stream);  // the load still reads the pinned rows
-        return r;
-    }
+    if (r) return r;
     c->pp_valid = c->per_particle;
     if ((r = store_forces(c, atoms))) return r;
     assemble(c, c->h_red, out);
@@ -1229,9 +1235,8 @@ int dlpx_md_store(dlpx_ctx *ctx, double *x, double *y, double *z, double *vx, do
     if (!c || stride < 0 || vstride < 0) return DLPX_ERR_BAD_ARG;
     if (!c->resident) return fail(c, DLPX_ERR_STATE, "call dlpx_md_load first");
     int r;
-    if ((r = store_atoms(c, true, false))) return r;
+    if ((r = store_atoms(c, true, false)) || (r = settle(c))) return r;
     const int n = c->natms;
-    DLPX_HIP(c, hipStreamSynchronize(c->stream));
     double *dst[9] = {x, y, z, vx, vy, vz, fx, fy, fz};
     for (int k = 0; k < 9; k++) {
         if (!dst[k]) continue;

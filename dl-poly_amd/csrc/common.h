@@ -234,6 +234,7 @@ struct Ctx {
     double *h_st = nullptr, *h_st_dev = nullptr;
     int32_t *h_t = nullptr, *h_t_dev = nullptr;
     double *h_disp = nullptr, *h_disp_dev = nullptr;
+    bool rows_busy = false;          // a kernel that reads or writes them may still run
     int32_t *cell_of = nullptr, *perm = nullptr;
 
     // link cells

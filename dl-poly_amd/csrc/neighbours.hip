@@ -1163,6 +1163,7 @@ int build_list(Ctx *c)
         int32_t *const all = c->h_flags + F_WORDS;  // every word in one copy
         DLPX_HIP(c, hipMemcpyAsync(all, c->flags, sizeof(int32_t) * F_WORDS, hipMemcpyDeviceToHost, s));
         DLPX_HIP(c, hipStreamSynchronize(s));
+        c->rows_busy = false;
         std::memcpy(c->h_flags, all, sizeof(int32_t) * 4);
         if (all[F_ERR] != 0) {
             c->have_list = false;

@@ -691,6 +691,7 @@ int load_atoms(Ctx *c, bool identity, bool with_vel, bool disp)
         a.b.L[d] = c->L[d];
         a.b.invL[d] = c->invL[d];
     }
+    c->rows_busy = true;
     hipLaunchKernelGGL(k_load, dim3(load_blocks(c)), dim3(kLoadThreads), 0, c->stream, a);
     DLPX_HIP(c, hipGetLastError());
     return 0;
@@ -710,6 +711,7 @@ int store_atoms(Ctx *c, bool with_state, bool finish)
     a.two_scale = finish ? 2.0 * recip_scale(c) : 0.0;
     a.inv_n = 1.0 / (double)c->natms;
     const dim3 grid(ceil_div(c->natms, kStoreThreads));
+    c->rows_busy = true;
     if (with_state) hipLaunchKernelGGL(k_store<9>, grid, dim3(kStoreThreads), 0, c->stream, a);
     else hipLaunchKernelGGL(k_store<3>, grid, dim3(kStoreThreads), 0, c->stream, a);
     DLPX_HIP(c, hipGetLastError());
@@ -718,6 +720,7 @@ int store_atoms(Ctx *c, bool with_state, bool finish)
 
 int store_per_particle(Ctx *c, double scale)
 {
+    c->rows_busy = true;
     hipLaunchKernelGGL(k_store_pp, dim3(ceil_div(c->natms, kStoreThreads)), dim3(kStoreThreads), 0, c->stream,
                        c->h_st_dev, c->natms, c->slot, c->pp, c->prm.electrostatics ? c->frc_recip : nullptr, scale);
     DLPX_HIP(c, hipGetLastError());

@@ -1303,3 +1303,29 @@ def test_memory_of_the_splines_only_for_tiles(monkeypatch):
     splines = s.natms * (8 * (3 * 8 + 4) + 8)
     print("case memory", s.natms, used, splines, flush=True)
     assert used["1"] - used["0"] >= splines
+
+
+def test_calls_after_a_failed_one_match_fresh_ones():
+    """List builds and loads that fail after they have queued their upload (a
+    cell too small for the cutoff), each at once followed by a good one with
+    other positions: the pinned rows are not written while the load still reads
+    them, and forces are a fresh context's."""
+    s = systems.nacl(ncells=20, kvec=(64, 64, 64), seed=29)
+    rng = np.random.default_rng(30)
+    ctx, fresh = lib.Context(s), lib.Context(s)
+    cell = ctx.cell.copy()
+    for k in range(4):
+        p = s.pos + rng.uniform(-0.1, 0.1, s.pos.shape)
+        for load in (False, True):
+            ctx.cell = cell * 0.1
+            with pytest.raises(lib.DlpxError) as e:
+                ctx.md_load(s.pos, s.vel) if load else ctx.link_cell_pairs(s.pos)
+            assert e.value.code == 95
+            ctx.cell = cell.copy()
+            ctx.link_cell_pairs(p)
+            fresh.link_cell_pairs(p)
+            a, b = ctx.two_body_forces(p), fresh.two_body_forces(p)
+            assert rms_rel(a["frc"], b["frc"]) <= 1e-13
+            assert a["engcpe"] == pytest.approx(b["engcpe"], rel=1e-13)
+    ctx.close()
+    fresh.close()
