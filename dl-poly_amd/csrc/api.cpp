@@ -472,6 +472,8 @@ static int md_step(Ctx *c, int s, int nsteps, double tstep, bool energies, int &
     if (update) {
         if ((r = build_list(c))) return r;
         rebuilds++;
+    } else {
+        c->stray_no = 0;  // no atom is beyond the lists' reach, whatever a force call before the run found
     }
     const bool last = s == nsteps - 1;
     if ((r = evaluate(c, true))) return r;

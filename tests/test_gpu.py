@@ -1329,3 +1329,29 @@ def test_calls_after_a_failed_one_match_fresh_ones():
             assert a["engcpe"] == pytest.approx(b["engcpe"], rel=1e-13)
     ctx.close()
     fresh.close()
+
+
+@pytest.mark.parametrize("graphs", ["0", "1"])
+def test_run_from_a_force_call_on_moved_positions(graphs, monkeypatch):
+    """A force call with one atom just beyond half the padding, then a run whose
+    first drift brings it back, so that nothing is rebuilt: the tiles' lists, not
+    those of the force call, with 27,000 ions (whose force call puts atoms on
+    lists where they are).  Against link cells, FP64 to rounding."""
+    monkeypatch.setenv("DLPX_GRAPHS", graphs)
+    s = systems.nacl(ncells=15, kvec=(96, 96, 96), seed=31, temperature=1.0)
+    p, v = s.pos.copy(), s.vel.copy()
+    p[11, 0] += 0.5 * s.padding + 0.01
+    v[11] = (-20.0, 0.0, 0.0)
+    got = {}
+    for tiles in ("0", "1"):
+        monkeypatch.setenv("DLPX_SPREAD_TILES", tiles)
+        ctx = lib.Context(s, precision=lib.FP64)
+        ctx.md_load(s.pos, v)
+        ctx.two_body_forces(p)
+        e, reb = ctx.md_run(3, s.timestep)
+        got[tiles] = (e, reb, ctx.md_store()[2])
+        ctx.close()
+    (e1, r1, f1), (e0, r0, f0) = got["1"], got["0"]
+    assert r1 == r0 == 0
+    assert np.abs(e1 - e0).max() <= 1e-11 * np.abs(e0).max()
+    assert rms_rel(f1, f0) <= 1e-10
