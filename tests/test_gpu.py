@@ -1355,3 +1355,27 @@ def test_run_from_a_force_call_on_moved_positions(graphs, monkeypatch):
     assert r1 == r0 == 0
     assert np.abs(e1 - e0).max() <= 1e-11 * np.abs(e0).max()
     assert rms_rel(f1, f0) <= 1e-10
+
+
+@pytest.mark.parametrize("size", [(8, 8, 8), (8, 8, 17)])
+def test_per_particle_energies_in_host_order(size):
+    """Each atom's energy and stress on both sides of the line between 32 and 8
+    lanes to an atom, with the atoms given forwards and in reverse (which moves
+    the vdW energy of pairs across the cell's faces to their other atom), against
+    the oracle: FP64 to 1e-10 of the largest, mixed to 1e-5 RMS."""
+    for order in (1, -1):
+        s = systems.nacl(ncells=size, kvec=(32, 32, 32), seed=32)
+        for k in ("pos", "vel", "types"):
+            setattr(s, k, getattr(s, k)[::order].copy())
+        o = oracle.two_body(s, per_particle=True)
+        for precision in (lib.FP64, lib.MIXED):
+            ctx = lib.Context(s, precision=precision)
+            ctx.link_cell_pairs(s.pos)
+            r = ctx.two_body_forces(s.pos, per_particle=True)
+            ctx.close()
+            for k in ("pp_energy", "pp_stress"):
+                print("case per particle", s.natms, order, precision, k, rms_rel(r[k], o[k]), flush=True)
+                if precision == lib.FP64:
+                    assert np.abs(r[k] - o[k]).max() <= 1e-10 * np.abs(o[k]).max()
+                else:
+                    assert rms_rel(r[k], o[k]) <= 1e-5
