@@ -1323,16 +1323,16 @@ static double crowding(const Ctx *c)
 // meshes of 0.35 to 1.8 points to the A, cutoffs of 8 to 12 A, filling the cell or
 // as slabs and droplets: nine of ten within 0.75 to 1.17 of the time measured by
 // tiles and 0.64 to 1.27 of that by cells.  A tile's chunk is then charged 0.4 +
-// 0.006 S^2 us more, for its share of the lists' making (1.5 us a chunk at each
-// rebuild) and of the CUs beside the pair kernel.
+// 0.012 S^2 us more (mixed 0.4 + 0.008 S^2), for its share of the lists' making (1.5 us a
+// chunk at each rebuild) and of the CUs beside the pair kernel.
 static double tiles_us(const Ctx *c, double atoms)
 {
     const bool mixed = c->prm.precision == DLPX_MIXED;
     const double S = c->prm.nsplines, chunks = std::ceil(atoms / kTileChunk), perCU = tile_blocks(c) / 256.0;
     return mixed ? 11.0 + 1.31e-5 * S * std::sqrt(S) * c->natms + (0.43 + 0.032 * S) * perCU +
-                       (1.44 + 0.0089 * S * S) * chunks
+                       (1.44 + 0.0109 * S * S) * chunks
                  : 11.0 + 1.58e-5 * S * std::sqrt(S) * c->natms + (0.51 + 0.056 * S) * perCU +
-                       (1.27 + 0.0125 * S * S) * chunks;
+                       (1.27 + 0.0178 * S * S) * chunks;
 }
 static double cells_us(const Ctx *c, double crowd)
 {
@@ -1356,15 +1356,16 @@ static double cells_us(const Ctx *c, double crowd)
 // their cell, 72 x 60 x 72, S = 8 FP64, 70 us instead of 46), in steps of sqrt(2)
 // so that the configurations of one system get the same room and captured
 // graphs, and one round of their making.
-// Where the mesh allows, the faster of the two by their estimates: over the
-// resident steps of 1,877 such systems with either, 0.4 % of the time is lost to
-// the faster choice, and 9 steps are more than 3 % (11 % at most) slower by tiles
-// than by cells.  (Without the order, the precision and the crowding in it: 2 %,
-// and 160.)  Few atoms to a tile (fine meshes) are the tiles': 64,000 ions on 128^3
-// at order 4, 8 and 16, mixed, 33, 52 and 474 us by cells and 22, 34 and 81 by
-// tiles.  Many, or a part of the cell crowded, are the cells': the same on 64^3 20,
-// 35 and 292 and 35, 75 and 226; 8,000 ions on 36^3 at order 8 in FP64 32 and 56;
-// the 7,200 ions above 31 and 46.
+// Where the mesh allows, by tiles unless cells are a fifth faster by these
+// estimates (beside the other systems of a batch, which fill the GPU, tiles are the
+// better choice a little longer): over the resident steps of 1,877 such systems
+// with either, 0.25 % of the time is lost to the faster choice, and 20 steps are more
+// than 3 % (11 % at most) slower by tiles than by cells.  (Without the order, the
+// precision and the crowding in it: 2 %, and 230.)  Few atoms to a tile (fine
+// meshes) are the tiles': 64,000 ions on 128^3 at order 4, 8 and 16, mixed, 33, 52
+// and 474 us by cells and 22, 34 and 81 by tiles.  Many, or a part of the cell
+// crowded, are the cells': the same on 64^3 20, 35 and 292 and 35, 75 and 226; 8,000
+// ions on 36^3 at order 8 in FP64 32 and 56; the 7,200 ions above 31 and 46.
 // The room, and that of the splines, is taken when the tiles first need it (332 MB
 // at 1,728,000 ions in FP64 at order 8); without memory for it the cells are there.
 void tile_room(Ctx *c)
@@ -1385,7 +1386,7 @@ void tile_room(Ctx *c)
     for (int d = 0; d < 3; d++)
         mean *= std::min(1.0, (T[d] + c->prm.nsplines - 1 + 2.0 * tile_drift(c, d)) / c->K[d]);
     const double crowd = crowding(c), most = std::min<double>(c->natms, mean * crowd);
-    if (c->spread_tiles < 0 && tiles_us(c, most) > cells_us(c, crowd)) return;
+    if (c->spread_tiles < 0 && tiles_us(c, most) > 1.2 * cells_us(c, crowd)) return;
     const double steps = crowd > 1.0 ? std::exp2(0.5 * std::ceil(2.0 * std::log2(crowd))) : 1.0;
     const int cap = kTileScan * kTileThreads + (int)(1.3 * std::min<double>(c->natms, mean * steps) / 64.0 + 1.0) * 64;
     const size_t words = (size_t)tile_blocks(c) * (cap + 2);
