@@ -356,11 +356,11 @@ int ensemble_run(const std::vector<Ctx *> &cs, Ensemble *&E, int nsteps, bool en
         if (c != c0) DLPX_HIP(c, hipStreamSynchronize(c->stream));
     for (Ctx *c : cs) {
         if ((r = snapshot(c, false))) return r;
-        // counters of the run: sticky overflow, rebuild count, record index;
-        // F_DMAX and F_DONE of stage 1 are zero between launches
+        // counters of the run: sticky overflow, rebuild count, record index,
+        // and the step kernel's finished workgroups (zero between launches)
         DLPX_HIP(c, hipMemsetAsync(c->flags + F_OVF_ANY, 0, sizeof(int32_t), c0->stream));
         DLPX_HIP(c, hipMemsetAsync(c->flags + F_NREB, 0, sizeof(int32_t) * 2, c0->stream));
-        DLPX_HIP(c, hipMemsetAsync(c->flags + F_DMAX, 0, sizeof(int32_t) * 3, c0->stream));
+        DLPX_HIP(c, hipMemsetAsync(c->flags + F_DONE, 0, sizeof(int32_t), c0->stream));
         // the totals that the gather accumulates atomically
         DLPX_HIP(c, hipMemsetAsync(c->acc, 0, sizeof(double) * 4 * kAccSlots, c0->stream));
     }

@@ -109,8 +109,8 @@ enum Flag : int {
     F_IBIG = 1,     // largest per-atom count of the last build
     F_OVF_ANY = 2,  // sticky overflow of any device-decided build in a resident run
     F_PAIRS = 3,    // stored entries of the last build
-    F_DMAX = 4,     // [4..5] displacement maximum (double bits), stage 1
-    F_DONE = 6,     // workgroups of stage 1 finished
+    F_DMAX = 4,     // [4..5] displacement maximum (double bits), k_vv1 (md_begin clears it)
+    F_DONE = 6,     // workgroups of k_vv1 or the step kernel finished
     F_UPD = 7,      // 1: the list is rebuilt before the coming force evaluation
     F_NREB = 8,     // rebuilds decided on the device since the run began
     F_STEP = 9,     // per-step energy records written since the run began

@@ -390,7 +390,7 @@ __global__ void __launch_bounds__(spread_threads<R>()) k_spread_cells_batch(cons
 }
 
 // The spline data of every atom, once per evaluation, for the spreading by
-// tiles (where an atom is met in about four tiles) and the gather: per axis
+// tiles (where an atom is met in about four tiles): per axis
 // the order S-1 values z[0..S-1] that the last step of the recursion
 // (bspline) turns into the values and first derivatives of order S,
 //   M[t] = (pt z[t] + (S - pt) z[t+1]) / (S - 1), pt = w + S - 1 - t,
