@@ -1322,9 +1322,9 @@ static double crowding(const Ctx *c)
 // 4,447 measured pairs of systems of 400 to 150,000 ions at every spline order, on
 // meshes of 0.35 to 1.8 points to the A, cutoffs of 8 to 12 A, filling the cell or
 // as slabs and droplets: nine of ten within 0.75 to 1.17 of the time measured by
-// tiles and 0.64 to 1.27 of that by cells.  A tile's chunk is then charged 0.4 +
-// 0.012 S^2 us more (mixed 0.4 + 0.008 S^2), for its share of the lists' making (1.5 us a
-// chunk at each rebuild) and of the CUs beside the pair kernel.
+// tiles and 0.64 to 1.27 of that by cells.  A tile's chunk is then charged 0.015 S^2
+// us more (mixed 0.4 + 0.008 S^2), for its share of the lists' making (1.5 us a chunk
+// at each rebuild) and of the CUs beside the pair kernel.
 static double tiles_us(const Ctx *c, double atoms)
 {
     const bool mixed = c->prm.precision == DLPX_MIXED;
@@ -1332,7 +1332,7 @@ static double tiles_us(const Ctx *c, double atoms)
     return mixed ? 11.0 + 1.31e-5 * S * std::sqrt(S) * c->natms + (0.43 + 0.032 * S) * perCU +
                        (1.44 + 0.0109 * S * S) * chunks
                  : 11.0 + 1.58e-5 * S * std::sqrt(S) * c->natms + (0.51 + 0.056 * S) * perCU +
-                       (1.27 + 0.0178 * S * S) * chunks;
+                       (0.87 + 0.0208 * S * S) * chunks;
 }
 static double cells_us(const Ctx *c, double crowd)
 {
@@ -1358,10 +1358,10 @@ static double cells_us(const Ctx *c, double crowd)
 // graphs, and one round of their making.
 // Where the mesh allows, by tiles unless cells are a fifth faster by these
 // estimates (beside the other systems of a batch, which fill the GPU, tiles are the
-// better choice a little longer): over the resident steps of 1,877 such systems
-// with either, 0.25 % of the time is lost to the faster choice, and 20 steps are more
-// than 3 % (11 % at most) slower by tiles than by cells.  (Without the order, the
-// precision and the crowding in it: 2 %, and 230.)  Few atoms to a tile (fine
+// better choice a little longer): over the resident steps of 667 more such systems
+// with either, 0.26 % of the time is lost to the faster choice (1.9 % without the
+// order, the precision and the crowding in it), and 12 steps instead of 77 are more
+// than 3 % (9 % at most, 40 %) slower by tiles than by cells.  Few atoms to a tile (fine
 // meshes) are the tiles': 64,000 ions on 128^3 at order 4, 8 and 16, mixed, 33, 52
 // and 474 us by cells and 22, 34 and 81 by tiles.  Many, or a part of the cell
 // crowded, are the cells': the same on 64^3 20, 35 and 292 and 35, 75 and 226; 8,000
