@@ -184,7 +184,11 @@ static int upload(Ctx *c, const dlpx_atoms *a, bool identity, const double *vx, 
     auto atv = [vst](const double *p, int i) { return *(const double *)((const char *)p + (size_t)vst * i); };
     const int row = vx ? 8 : 4;
     int r;
-    if (c->rows_busy && (r = settle(c))) return r;  // a call that failed has not waited for its load
+    if (c->rows_busy) {
+        // a call that failed has not waited for its load, nor joined the reciprocal sum it may have begun
+        DLPX_HIP(c, hipStreamSynchronize(c->recip_stream));
+        if ((r = settle(c))) return r;
+    }
     // charge per atom type, for the pair kernel's combined-table path
     std::vector<double> tq(c->prm.ntypes, 0.0);
     std::vector<char> seen(c->prm.ntypes, 0);
